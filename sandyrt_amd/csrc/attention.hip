@@ -40,7 +40,7 @@
 //     call.
 // The probabilities enter the PV product as two bf16 operands (hi + lo), so
 // P keeps about 17 bits and the normaliser is the float sum of the same p.
-#include "common.h"
+#include "attention_prefill.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -1212,6 +1212,39 @@ __global__ __launch_bounds__(256) void attention_decode_f32_kernel(GenArgs a) {
 
 using namespace sandy_hip;
 
+// The MFMA prefill kernel's arguments from a general call (dense K/V strides,
+// or page tables), where it takes the shape.
+static bool prefill_args(const GenArgs& g, int64_t B, PrefillArgs* p) {
+    if (g.qs[3] != 1 || g.os[3] != 1 || (!g.paged && (g.ks[3] != 1 || g.vs[3] != 1)) || g.tk > (1LL << 30)) return false;
+    *p = PrefillArgs{};
+    p->q = g.q;
+    p->out = g.out;
+    p->k = g.k;
+    p->v = g.v;
+    for (int i = 0; i < 3; i++) {
+        p->qs[i] = g.qs[i];
+        p->os[i] = g.os[i];
+        p->ks[i] = g.ks[i];
+        p->vs[i] = g.vs[i];
+    }
+    p->k_pages = g.k_pages;
+    p->v_pages = g.v_pages;
+    p->kv_rows_b = g.kv_rows_b;
+    while (g.paged && (int64_t{1} << p->log2_page) < g.page_size && p->log2_page < 30) p->log2_page++;
+    p->pos = g.pos;
+    p->pos_dt = g.pos_dt;
+    p->batch = static_cast<int32_t>(B);
+    p->hq = g.hq;
+    p->hkv = g.hkv;
+    p->group = g.hq / g.hkv;
+    p->tq = g.tq;
+    p->tk = static_cast<int32_t>(g.tk);
+    p->window = g.window;
+    p->scale_log2 = g.scale * kLog2e;
+    p->errw = g.errw;
+    return prefill_takes(*p, g.dt, g.d);
+}
+
 extern "C" int sandy_hip_attention(const SandyTensor* q, const SandyTensor* k, const SandyTensor* v,
                                    const SandyTensor* position_offsets, int64_t window, double scale,
                                    const SandyTensor* out, void* stream_, char* err, size_t err_cap) {
@@ -1271,10 +1304,12 @@ extern "C" int sandy_hip_attention(const SandyTensor* q, const SandyTensor* k, c
     a.d = D;
     a.window = window;
     a.scale = scale <= 0.0 ? 1.0f / sqrtf(static_cast<float>(D)) : static_cast<float>(scale);
+    a.errw = errw;
+    PrefillArgs pre;
+    if (prefill_args(a, B, &pre)) return launch_prefill(pre, D, stream, e);
     const size_t sbytes = static_cast<size_t>(B * hq * tq * std::max<int64_t>(tk, 1)) * sizeof(float);
     a.scores = static_cast<float*>(device_workspace(1, sbytes, stream, e, &status));
     if (status) return status;
-    a.errw = errw;
     dim3 grid(static_cast<unsigned>(tq), static_cast<unsigned>(hq), static_cast<unsigned>(B));
     if (a.tk <= kGenStage && env_int("SANDY_ATTN_UNSTAGED", 0) == 0) {
         if (q->dtype == SANDY_BF16) hipLaunchKernelGGL(attention_staged_kernel<BF16>, grid, dim3(256), 0, stream, a);
@@ -1648,10 +1683,12 @@ extern "C" int sandy_hip_attention_paged_view(const SandyTensor* q, const SandyP
     a.d = D;
     a.window = window;
     a.scale = sc;
+    a.errw = errw;
+    PrefillArgs pre;
+    if (prefill_args(a, B, &pre)) return launch_prefill(pre, D, stream, e);
     const size_t sbytes = static_cast<size_t>(B * hq * tq * std::max<int64_t>(tk, 1)) * sizeof(float);
     a.scores = static_cast<float*>(device_workspace(1, sbytes, stream, e, &status));
     if (status) return status;
-    a.errw = errw;
     dim3 grid(static_cast<unsigned>(tq), static_cast<unsigned>(hq), static_cast<unsigned>(B));
     if (a.tk <= kGenStage && env_int("SANDY_ATTN_UNSTAGED", 0) == 0) {
         if (q->dtype == SANDY_BF16) hipLaunchKernelGGL(attention_staged_kernel<BF16>, grid, dim3(256), 0, stream, a);

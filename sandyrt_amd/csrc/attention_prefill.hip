@@ -1,0 +1,497 @@
+// attention_prefill.hip -- causal attention of prompts and prompt chunks
+// (AttentionKernelOp with Tq > 1, src/core/TensorCalc.cpp:1167-1314), bf16,
+// over dense K/V or the reference's paged K/V.
+//
+// The general kernel (attention.hip) runs one workgroup per (query, head)
+// and walks the keys in the reference's order; every query re-reads its K and
+// V rows and all products are scalar: 14.4 ms for 2048 queries of 32 heads.
+// Here the products run on v_mfma_f32_32x32x16_bf16 with an online softmax:
+//   - the rows of one kv head are its (query, head of the group) pairs, query
+//     major, so a workgroup's rows are a few neighbouring queries of the whole
+//     GQA group: every staged key serves all heads of the group and the
+//     causal frontier stays narrow;
+//   - S^T = K Q^T (keys are MFMA rows, queries columns), so a lane holds the
+//     scores of one query and the softmax needs one cross-lane exchange;
+//   - P^T leaves the product in the B-operand layout of O^T += V^T P^T, with
+//     V^T read by ds_read_b64_tr_b16 in the same key order;
+//   - P enters as two bf16 operands (hi + lo), about 17 bits of each
+//     probability; the row sums are kept in float64.
+// Four score waves a workgroup: RW of them own 32 rows each and KW = 4 / RW
+// share the keys of a chunk (merged at the end), so short prompts still fill
+// the chip; at D 256 a second wave per score tile owns half of the head dims.
+// Chunks of K and V go global -> registers -> LDS, double buffered where they
+// fit, one barrier each.
+// Bound: softmax VALU work (49% of the cycles at D 64, MFMA 22%).  Measured,
+// us a call (general kernel -> here): 2048 queries, 32 / 4 heads, D 64
+// 14357 -> 44; 777 queries after 1500 keys, window 1024, 8 / 2 heads, D 256,
+// pages of 16: 4896 -> 46; 1500 after 300, 16 / 2 heads, D 128: 54.
+#include "attention_prefill.h"
+
+#include <algorithm>
+
+namespace sandy_hip {
+namespace {
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef short short4_t __attribute__((ext_vector_type(4)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+
+constexpr int kMaxKeys = 1 << 30;
+constexpr int kTablePages = 512;  // page addresses of K and V held in LDS
+
+// Geometry of a variant.  LDS rows are padded so that MFMA-layout reads touch
+// every bank once: 16 lanes x 16 bytes down a K column (pitch 16 bytes past a
+// multiple of 128), 4 rows x 64 bytes of V per transposing read (pitch 64
+// bytes past a multiple of 256 or 128).
+template <int D, int RW>
+struct Geo {
+    // D 256: two waves share a score tile and own half of the head dims each,
+    // so that two waves fit a SIMD (one wave with all of O^T in its registers
+    // had nothing to run behind its waits)
+    static constexpr int DS = D == 256 ? 2 : 1;
+    static constexpr int THREADS = 256 * DS;
+    static constexpr int DT = D / 32 / DS;    // 32-dim tiles of O^T a wave owns
+    static constexpr int KW = 4 / RW;
+    static constexpr int CK = KW * 32;        // keys of a chunk, 32 a wave
+    static constexpr int KP = 2 * D + 16;     // bytes per K row in LDS
+    static constexpr int VP = 2 * D + 64;     // bytes per V row in LDS
+    static constexpr int kBuf = CK * (KP + VP);
+    static constexpr int NB = 2 * kBuf <= 160 * 1024 - 512 ? 2 : 1;  // LDS buffers
+    static constexpr int NP = CK * D / 8 / THREADS;  // 16-byte pieces of K (and of V) a thread stages
+    // final merge: [KW - 1][RW] copies of a wave's accumulators, and (m, l)
+    static constexpr int kMerge = (KW - 1) * RW * D * 32 * 4;
+    static constexpr int kStats = 4 * 32 * 16;  // of the waves of the first half
+    static constexpr int kBytes = (NB * kBuf > kMerge + kStats ? NB * kBuf : kMerge + kStats);
+};
+
+// Byte address of row `key` of the page at `at` on page row `row`, rounded
+// down to whole elements.
+__device__ __forceinline__ uint64_t paged_row(uint64_t at, int key, int log2_page, int64_t row, int row_bytes) {
+    const int64_t in_page = key & ((1 << log2_page) - 1);
+    return (at & ~uint64_t{1}) + static_cast<uint64_t>(((row << log2_page) + in_page) * row_bytes);
+}
+
+// 16 bytes from a row whose start is only element aligned.
+__device__ __forceinline__ u32x4_t load_piece(uint64_t at) {
+    if ((at & 15) == 0) return *reinterpret_cast<const u32x4_t*>(at);
+    const uint16_t* p = reinterpret_cast<const uint16_t*>(at);
+    uint32_t w[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) w[i] = static_cast<uint32_t>(p[2 * i]) | (static_cast<uint32_t>(p[2 * i + 1]) << 16);
+    return u32x4_t{w[0], w[1], w[2], w[3]};
+}
+
+// One row again, a key at a time, where V holds infinities or NaN: every key
+// the row sees adds its normalised probability times V (from the row's known
+// max and 1 / sum), so a non-finite V reaches exactly the rows that see its
+// key.  256 keys at a time through `probs`; q in `qrow`.
+template <int D, bool PAGED>
+__device__ __forceinline__ void careful_row(const PrefillArgs& a, int b, int kh, int row, int first, int last,
+                                                      float m, float inv, float* probs, void* qrow) {
+    const int tid = threadIdx.x;
+    const int t = row / a.group, h = kh * a.group + row % a.group;
+    float* qf = static_cast<float*>(qrow);
+    if (tid < D) qf[tid] = bf16_to_f32(static_cast<const uint16_t*>(a.q)[b * a.qs[0] + h * a.qs[1] + t * a.qs[2] + tid]);
+    auto row_of = [&](bool value, int key) -> const uint16_t* {
+        if constexpr (PAGED) {
+            const uint64_t at = (value ? a.v_pages : a.k_pages)[key >> a.log2_page];
+            return at ? reinterpret_cast<const uint16_t*>(paged_row(at, key, a.log2_page, b * a.kv_rows_b + kh, 2 * D))
+                      : nullptr;
+        } else {
+            const int64_t* st = value ? a.vs : a.ks;
+            return static_cast<const uint16_t*>(value ? a.v : a.k) + b * st[0] + kh * st[1] + key * st[2];
+        }
+    };
+    float acc = 0.0f;
+    for (int k0 = first; k0 <= last; k0 += 256) {
+        __syncthreads();
+        const int n = min(256, last + 1 - k0);
+        if (tid < n) {
+            const uint16_t* kp = row_of(false, k0 + tid);
+            float s = 0.0f;
+#pragma unroll 1
+            for (int d = 0; d < D; d++) s = fmaf(qf[d], kp ? bf16_to_f32(kp[d]) : 0.0f, s);
+            probs[tid] = __builtin_amdgcn_exp2f(fmaf(s, a.scale_log2, -m)) * inv;
+        }
+        __syncthreads();
+        if (tid < D) {
+#pragma unroll 1
+            for (int i = 0; i < n; i++) {
+                const uint16_t* vp = row_of(true, k0 + i);
+                acc = fmaf(probs[i], vp ? bf16_to_f32(vp[tid]) : 0.0f, acc);
+            }
+        }
+    }
+    if (tid < D && first <= last)
+        static_cast<uint16_t*>(a.out)[b * a.os[0] + h * a.os[1] + t * a.os[2] + tid] = f32_to_bf16(acc);
+    __syncthreads();
+}
+
+template <int D, int RW, bool PAGED>
+__global__ __launch_bounds__((Geo<D, RW>::THREADS), 2) void attention_prefill_kernel(PrefillArgs a) {
+    using G_ = Geo<D, RW>;
+    constexpr int KW = G_::KW, SUB = 32, CK = G_::CK, KP = G_::KP, VP = G_::VP, NP = G_::NP, DT = G_::DT;
+    constexpr int kPieces = D / 8;  // 16-byte pieces per row
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rw = wave % RW, kw = (wave & 3) / RW, ds = wave >> 2;
+    const int col = lane & 31, half = lane >> 5;
+    // heads vary fastest: workgroups go round-robin to the 8 XCDs, so one XCD
+    // serves few kv heads; the longest row blocks (latest queries) start first
+    const int heads = a.batch * a.hkv;
+    const int bh = static_cast<int>(blockIdx.x) % heads;
+    const int nth = static_cast<int>(blockIdx.x) / heads;
+    const int b = bh / a.hkv, kh = bh % a.hkv;
+    const int rows = a.group * a.tq;
+    int64_t base = 0;
+    if (a.pos) {
+        base = load_index(a.pos, a.pos_dt, b);
+        if (base < 0) {
+            if (tid == 0) atomicOr(a.errw, static_cast<uint32_t>(SANDY_DEVERR_ATTN_POS));
+            return;
+        }
+    }
+    // keys [first, last] of query t
+    auto last_of = [&](int t) -> int { return static_cast<int>(min<int64_t>(base + t, a.tk - 1)); };
+    auto first_of = [&](int t) -> int {
+        return a.window > 0 ? static_cast<int>(min<int64_t>(max<int64_t>(0, base + t + 1 - a.window), kMaxKeys)) : 0;
+    };
+    const int rb = a.row_blocks - 1 - nth;
+    const int r0 = rb * 32 * RW;
+    const int k_begin = first_of(r0 / a.group);
+    const int k_end = last_of(min(rows - 1, r0 + 32 * RW - 1) / a.group) + 1;
+
+    // this lane's row (clamped: rows past the end repeat the last and are not stored)
+    const int row = r0 + 32 * rw + col;
+    const int rc = min(row, rows - 1);
+    const int qt = rc / a.group, qg = rc - qt * a.group;
+    const int lane_last = last_of(qt), lane_first = first_of(qt);
+    // the wave's rows: keys every row sees, and keys some row sees
+    const int t_lo = min(rows - 1, r0 + 32 * rw) / a.group, t_hi = min(rows - 1, r0 + 32 * rw + 31) / a.group;
+    const int any_first = first_of(t_lo), any_last = last_of(t_hi);
+    const int all_first = first_of(t_hi), all_last = last_of(t_lo);
+
+    bf16x8_t qv[D / 16];  // B operands: column = query, 16 s + 8 half .. + 7
+    {
+        const uint16_t* qp = static_cast<const uint16_t*>(a.q) + b * a.qs[0] + (kh * a.group + qg) * a.qs[1] +
+                             qt * a.qs[2] + 8 * half;
+#pragma unroll
+        for (int s = 0; s < D / 16; s++) qv[s] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(qp + 16 * s));
+    }
+
+    // ---- staging: thread piece i covers chunk row prow + i * (256 / kPieces), 16-byte piece ppc
+    constexpr int kRowStep = G_::THREADS / kPieces;
+    const int prow = tid / kPieces, ppc = tid % kPieces;
+    const uint16_t* kbase = static_cast<const uint16_t*>(a.k) + (PAGED ? 0 : b * a.ks[0] + kh * a.ks[1] + 8 * ppc);
+    const uint16_t* vbase = static_cast<const uint16_t*>(a.v) + (PAGED ? 0 : b * a.vs[0] + kh * a.vs[1] + 8 * ppc);
+    const uint32_t page_row = static_cast<uint32_t>(b * a.kv_rows_b + kh);
+    u32x4_t kr[NP], vr[NP];
+    bool pages_ok = true;
+    // rows past the last key repeat it (they are masked)
+    auto key_of = [&](int c0, int i) -> int { return min(c0 + prow + i * kRowStep, k_end - 1); };
+    // the page addresses of the workgroup's keys, staged in LDS once where they
+    // fit: read from memory per chunk they put a dependent load before each of
+    // the chunk's (D 256: 4.4 us a chunk against 2.4 us)
+    uint64_t* tab = reinterpret_cast<uint64_t*>(lds + G_::kBytes);
+    const int page0 = PAGED ? k_begin >> a.log2_page : 0;
+    if (PAGED && a.table_pages > 0) {
+        const int n = k_begin < k_end ? min(((k_end - 1) >> a.log2_page) - page0 + 1, a.table_pages) : 0;
+        for (int i = tid; i < n; i += G_::THREADS) {
+            tab[2 * i] = a.k_pages[page0 + i];
+            tab[2 * i + 1] = a.v_pages[page0 + i];
+        }
+        __syncthreads();
+    }
+    auto load = [&](int c0) {
+        if constexpr (PAGED) {
+            uint64_t kat[NP], vat[NP];
+            bool plain = true;  // every page there and 16-byte aligned
+#pragma unroll
+            for (int i = 0; i < NP; i++) {
+                const int key = key_of(c0, i), page = key >> a.log2_page;
+                if (a.table_pages > 0) {
+                    kat[i] = tab[2 * (page - page0)];
+                    vat[i] = tab[2 * (page - page0) + 1];
+                } else {
+                    kat[i] = a.k_pages[page];
+                    vat[i] = a.v_pages[page];
+                }
+                // byte offset of the row within the page: below 2^31 (checked on the host)
+                const uint32_t off = ((page_row << a.log2_page) + (key & ((1 << a.log2_page) - 1))) * (2 * D) + 16 * ppc;
+                plain = plain && kat[i] != 0 && vat[i] != 0 && ((kat[i] | vat[i]) & 15) == 0;
+                kat[i] = kat[i] ? (kat[i] & ~uint64_t{1}) + off : 0;
+                vat[i] = vat[i] ? (vat[i] & ~uint64_t{1}) + off : 0;
+            }
+            if (__all(plain)) {
+#pragma unroll
+                for (int i = 0; i < NP; i++) {
+                    kr[i] = *reinterpret_cast<const u32x4_t*>(kat[i]);
+                    vr[i] = *reinterpret_cast<const u32x4_t*>(vat[i]);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < NP; i++) {
+                    pages_ok = pages_ok && kat[i] && vat[i];
+                    kr[i] = kat[i] ? load_piece(kat[i]) : u32x4_t{0, 0, 0, 0};
+                    vr[i] = vat[i] ? load_piece(vat[i]) : u32x4_t{0, 0, 0, 0};
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < NP; i++) {
+                kr[i] = *reinterpret_cast<const u32x4_t*>(kbase + key_of(c0, i) * a.ks[2]);
+                vr[i] = *reinterpret_cast<const u32x4_t*>(vbase + key_of(c0, i) * a.vs[2]);
+            }
+        }
+    };
+    auto store = [&](int buf) {
+        unsigned char* kt = lds + buf * G_::kBuf;
+        unsigned char* vt = kt + CK * KP;
+#pragma unroll
+        for (int i = 0; i < NP; i++) {
+            *reinterpret_cast<u32x4_t*>(kt + (prow + i * kRowStep) * KP + 16 * ppc) = kr[i];
+            *reinterpret_cast<u32x4_t*>(vt + (prow + i * kRowStep) * VP + 16 * ppc) = vr[i];
+        }
+    };
+
+    f32x16_t acc[DT];
+    float m = -INFINITY;  // -inf until a key has been seen
+    double l = 0.0;
+    // P of a masked key is 0 and lo of an exact P is 0, so an infinity in V
+    // would come out as NaN: outputs that are not all finite are computed again
+    // below, one key at a time
+#pragma unroll
+    for (int t = 0; t < DT; t++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[t][i] = 0.0f;
+    if (k_begin < k_end) load(k_begin);
+    int buf = 0;
+    for (int c0 = k_begin; c0 < k_end; c0 += CK, buf ^= G_::NB - 1) {
+        if (G_::NB == 1 && c0 > k_begin) __syncthreads();  // the chunk before has been read
+        store(buf);
+        __syncthreads();
+        if (c0 + CK < k_end) load(c0 + CK);
+        const int k0 = c0 + kw * SUB;
+        if (k0 > any_last || k0 + SUB - 1 < any_first) continue;  // wave-uniform
+        const bool partial = k0 + SUB - 1 > all_last || k0 < all_first;
+        const unsigned char* kt = lds + buf * G_::kBuf + kw * SUB * KP + col * KP + 16 * half;
+        const unsigned char* vt = lds + buf * G_::kBuf + CK * KP + kw * SUB * VP;
+        f32x16_t sc;
+#pragma unroll
+        for (int i = 0; i < 16; i++) sc[i] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < D / 16; s++) {
+            const bf16x8_t kv = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(kt + 32 * s));
+            sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kv, qv[s], sc, 0, 0, 0);
+        }
+        // element i of sc: key k0 + 8 (i / 4) + 4 half + i % 4
+        if (partial) {
+            int key0 = k0 + 4 * half;
+            asm volatile("" : "+v"(key0));  // keeps the compares out of whole tiles
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int key = key0 + 8 * (i >> 2) + (i & 3);
+                if (key > lane_last || key < lane_first) sc[i] = -INFINITY;
+            }
+        }
+        float mx = sc[0];
+#pragma unroll
+        for (int i = 1; i < 16; i++) mx = fmaxf(mx, sc[i]);
+        mx = max_xor32(mx) * a.scale_log2;
+        // the reference point m of a row's exponents moves only when its max has
+        // grown by 2^8 (p stays below that, its relative precision is the same),
+        // so most chunks leave the accumulators alone
+        if (__any(mx > m + 8.0f)) {
+            const float m_new = fmaxf(m, mx);
+            const float alpha = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - m_new);
+            l *= static_cast<double>(alpha);
+            if (__any(m != -INFINITY)) {
+#pragma unroll
+                for (int t = 0; t < DT; t++) acc[t] *= alpha;
+            }
+            m = m_new;
+        }
+        const float shift = m == -INFINITY ? 0.0f : m;
+        float rs = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            sc[i] = __builtin_amdgcn_exp2f(fmaf(sc[i], a.scale_log2, -shift));
+            rs += sc[i];
+        }
+        l += static_cast<double>(rs);
+        // contraction slot 8 half + j of step s2: key 16 s2 + 4 half + j (j < 4) or + 8 + j - 4
+#pragma unroll
+        for (int s2 = 0; s2 < 2; s2++) {
+            bf16x8_t ph, pl;
+#pragma unroll
+            for (int j = 0; j < 8; j += 2) {
+                const f32x2_t p2 = {sc[8 * s2 + j], sc[8 * s2 + j + 1]};
+                const bf16x2_t h2 = __builtin_convertvector(p2, bf16x2_t);
+                const f32x2_t back = __builtin_convertvector(h2, f32x2_t);
+                const bf16x2_t l2 = __builtin_convertvector(f32x2_t{p2[0] - back[0], p2[1] - back[1]}, bf16x2_t);
+                ph[j] = h2[0];
+                ph[j + 1] = h2[1];
+                pl[j] = l2[0];
+                pl[j + 1] = l2[1];
+            }
+            // ds_read_b64_tr_b16: in each 16-lane group, lane i gets element i % 4 of
+            // the 8-byte pieces addressed by lanes 4 n + i / 4 (n = 0..3): pointing
+            // lane i at key kb + i / 4, dims d0 + 4 (i % 4) .. + 3 yields V[kb + n][d0 + i]
+            const int i16 = lane & 15;
+            const unsigned char* src = vt + (16 * s2 + 4 * half + (i16 >> 2)) * VP + 2 * (16 * ((lane >> 4) & 1) + 4 * (i16 & 3));
+#pragma unroll
+            for (int t = 0; t < DT; t++) {
+                const unsigned char* s0 = src + 64 * (DT * ds + t);
+                const short4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (short4_t __attribute__((address_space(3)))*)((unsigned char __attribute__((address_space(3)))*)s0));
+                const short4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (short4_t __attribute__((address_space(3)))*)((unsigned char __attribute__((address_space(3)))*)(s0 + 8 * VP)));
+                const bf16x8_t va = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+                acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, ph, acc[t], 0, 0, 0);
+                acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pl, acc[t], 0, 0, 0);
+            }
+        }
+    }
+    // the two halves of a row's sums; then the key shares of the KW waves
+    l += __shfl_xor(l, 32, 64);
+    __syncthreads();
+    if constexpr (KW > 1) {
+        float* red = reinterpret_cast<float*>(lds);
+        double* ml = reinterpret_cast<double*>(lds + G_::kMerge);  // [wave][32][2]
+        if (half == 0 && ds == 0) {
+            ml[((wave & 3) * 32 + col) * 2] = static_cast<double>(m);
+            ml[((wave & 3) * 32 + col) * 2 + 1] = l;
+        }
+        __syncthreads();
+        float mm = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < KW; w++) mm = fmaxf(mm, static_cast<float>(ml[((w * RW + rw) * 32 + col) * 2]));
+        const float shift = mm == -INFINITY ? 0.0f : mm;
+        double ll = 0.0;
+#pragma unroll
+        for (int w = 0; w < KW; w++) {
+            const double* e = ml + ((w * RW + rw) * 32 + col) * 2;
+            ll += e[1] * static_cast<double>(__builtin_amdgcn_exp2f(static_cast<float>(e[0]) - shift));
+        }
+        const float f = __builtin_amdgcn_exp2f(m - shift);
+#pragma unroll
+        for (int t = 0; t < DT; t++) acc[t] *= f;
+        m = mm;
+        l = ll;
+        if (kw > 0) {
+#pragma unroll
+            for (int t = 0; t < DT; t++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) red[(((kw - 1) * RW + rw) * (D / 2) + 16 * (DT * ds + t) + i) * 64 + lane] = acc[t][i];
+        }
+        __syncthreads();
+        if (kw == 0) {
+#pragma unroll
+            for (int w = 0; w < KW - 1; w++)
+#pragma unroll
+                for (int t = 0; t < DT; t++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) acc[t][i] += red[((w * RW + rw) * (D / 2) + 16 * (DT * ds + t) + i) * 64 + lane];
+        }
+    }
+    if (PAGED && !pages_ok) atomicOr(a.errw, static_cast<uint32_t>(SANDY_DEVERR_BLOCK));
+    const float inv = 1.0f / static_cast<float>(l);
+    // a row that sees no key (or only NaN scores) is zero, as in the general kernel
+    const bool none = m == -INFINITY;
+    bool finite = true;
+    if (kw == 0 && row < rows) {
+        uint16_t* op = static_cast<uint16_t*>(a.out) + b * a.os[0] + (kh * a.group + qg) * a.os[1] + qt * a.os[2] + 32 * DT * ds + 4 * half;
+#pragma unroll
+        for (int t = 0; t < DT; t++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                float o[4];
+#pragma unroll
+                for (int x = 0; x < 4; x++) {
+                    o[x] = none ? 0.0f : acc[t][4 * i + x] * inv;
+                    finite = finite && fabsf(o[x]) < INFINITY;
+                }
+                *reinterpret_cast<uint2*>(op + 32 * t + 8 * i) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+            }
+    }
+    if (!__syncthreads_or(finite ? 0 : 1)) return;
+    float* stats = reinterpret_cast<float*>(lds);  // [32 * RW] max, then 1 / sum
+    if (kw == 0 && half == 0 && ds == 0) {
+        stats[32 * rw + col] = m;
+        stats[32 * RW + 32 * rw + col] = inv;
+    }
+    __syncthreads();
+    for (int i = 0; i < 32 * RW && r0 + i < rows; i++)
+        if (stats[i] != -INFINITY) careful_row<D, PAGED>(a, b, kh, r0 + i, first_of((r0 + i) / a.group), last_of((r0 + i) / a.group), stats[i],
+                              stats[32 * RW + i], reinterpret_cast<float*>(lds) + 64 * RW, lds + 256 * RW + 1024 + 16);
+}
+
+template <int D, int RW, bool PAGED>
+int launch_form(const PrefillArgs& a, hipStream_t stream, Err e) {
+    static_assert(Geo<D, RW>::kBytes + kTablePages * 16 <= 160 * 1024 - 256, "LDS of a workgroup");
+    PrefillArgs args = a;
+    size_t bytes = Geo<D, RW>::kBytes;
+    if (PAGED) {
+        // pages a workgroup's keys can span: the whole list, or a window and its rows' queries
+        int64_t span = (static_cast<int64_t>(a.tk) >> a.log2_page) + 1;
+        if (a.window > 0) span = std::min(span, ((a.window + 32 * RW / a.group + 1) >> a.log2_page) + 2);
+        args.table_pages = span <= kTablePages ? static_cast<int32_t>(span) : 0;
+        bytes += static_cast<size_t>(args.table_pages) * 16;
+    }
+    const void* fn = reinterpret_cast<const void*>(&attention_prefill_kernel<D, RW, PAGED>);
+    if (bytes > 64 * 1024)
+        SANDY_HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)), e,
+                      "attention launch");
+    const int64_t rows = static_cast<int64_t>(a.group) * a.tq;
+    args.row_blocks = static_cast<int32_t>((rows + 32 * RW - 1) / (32 * RW));
+    const int64_t wgs = static_cast<int64_t>(args.row_blocks) * a.batch * a.hkv;
+    void* params[] = {&args};
+    SANDY_HIP_TRY(hipLaunchKernel(fn, dim3(static_cast<unsigned>(wgs)), dim3(Geo<D, RW>::THREADS), params, bytes, stream),
+                  e, "attention launch");
+    return ok(e);
+}
+
+template <int D, bool PAGED>
+int launch_dim(const PrefillArgs& a, hipStream_t stream, Err e) {
+    const int64_t rows = static_cast<int64_t>(a.group) * a.tq;
+    const int64_t heads = static_cast<int64_t>(a.batch) * a.hkv;
+    // 64-row workgroups (two waves share the keys) where they fill the 256 CUs,
+    // else 32-row ones (four share them): 1024 workgroups of 64 rows 43 us
+    // against 94, 114 of them 37 us against 33 at 32 rows (900 queries, D 256).
+    // 128-row workgroups were slower at every size (2048 queries, D 64: 45 us).
+    const int64_t wgs = (rows + 63) / 64 * heads;
+    if (env_int("SANDY_PREFILL_RW", wgs >= 256 ? 2 : 1) == 2) return launch_form<D, 2, PAGED>(a, stream, e);
+    return launch_form<D, 1, PAGED>(a, stream, e);
+}
+
+} // namespace
+
+bool prefill_takes(const PrefillArgs& a, int32_t dtype, int64_t D) {
+    if (dtype != SANDY_BF16 || (D != 64 && D != 128 && D != 256) || a.tq < 2 || a.tk <= 0) return false;
+    // 16-byte q and dense K/V rows, 8-byte output pieces
+    auto aligned = [](const void* p, const int64_t* s, uintptr_t bytes) {
+        return (reinterpret_cast<uintptr_t>(p) & (bytes - 1)) == 0 &&
+               ((s[0] | s[1] | s[2]) & static_cast<int64_t>(bytes / 2 - 1)) == 0;
+    };
+    if (!aligned(a.q, a.qs, 16) || !aligned(a.out, a.os, 8)) return false;
+    if (!a.k_pages && (!aligned(a.k, a.ks, 16) || !aligned(a.v, a.vs, 16))) return false;
+    const int64_t rows = static_cast<int64_t>(a.group) * a.tq;
+    if (a.k_pages && ((a.batch * a.kv_rows_b + a.hkv) << a.log2_page) * D * 2 >= (int64_t{1} << 31)) return false;
+    return rows < kMaxKeys && (rows + 31) / 32 * a.batch * a.hkv < (int64_t{1} << 31) &&
+           env_int("SANDY_PREFILL_GENERAL", 0) == 0;
+}
+
+int launch_prefill(PrefillArgs a, int64_t D, hipStream_t stream, Err e) {
+    const bool paged = a.k_pages != nullptr;
+    switch (D) {
+        case 64: return paged ? launch_dim<64, true>(a, stream, e) : launch_dim<64, false>(a, stream, e);
+        case 128: return paged ? launch_dim<128, true>(a, stream, e) : launch_dim<128, false>(a, stream, e);
+        default: return paged ? launch_dim<256, true>(a, stream, e) : launch_dim<256, false>(a, stream, e);
+    }
+}
+
+} // namespace sandy_hip

@@ -1,0 +1,122 @@
+"""GPU parity of attention over several queries (prompts and prompt chunks)
+against the oracle (src/core/TensorCalc.cpp:1167-1314): the MFMA prefill
+kernel's row and key tile edges, windows, offsets past the keys, page lists,
+and non-finite keys and values."""
+import numpy as np
+import pytest
+import torch
+
+from tests.helpers import assert_close, from_f32, normal, rng, to_oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from sandyrt_amd import ops
+    return ops
+
+
+def pages_of(ops, t, P, shift=0):
+    """A [B, Hkv, T, D] tensor as a page list (its own allocation a page,
+    `shift` elements into it) and the tensors to keep alive."""
+    B, H, T, D = t.shape
+    keep, at = [], []
+    for p in range((T + P - 1) // P):
+        page = torch.zeros(B * H * P * D + shift, dtype=t.dtype, device="cuda")
+        rows = t[:, :, p * P:(p + 1) * P].reshape(B * H, -1, D)
+        page[shift:].view(B * H, P, D)[:, :rows.shape[1]] = rows
+        keep.append(page)
+        at.append(page.data_ptr() + shift * t.element_size())
+    return ops.PagedView(torch.tensor(at, dtype=torch.int64, device="cuda"), t.shape, P, t.dtype), keep
+
+
+def check(ops, oracle, dtype, B, hq, hkv, tq, tk, D, pos, window, P=0, shift=0, spoil=None, heads_inner=False):
+    r = rng(tq * 131 + tk + D + window)
+    q = from_f32(normal(r, (B, hq, tq, D), 0.5), dtype)
+    if heads_inner:  # the engine's [B, T, H, D] rows seen as [B, H, T, D]
+        q = q.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3)
+    k = from_f32(normal(r, (B, hkv, tk, D), 0.5), dtype)
+    v = from_f32(normal(r, (B, hkv, tk, D)), dtype)
+    if spoil:
+        spoil(k, v)
+    p = torch.tensor(pos, device="cuda") if pos is not None else None
+    want = oracle.attention(to_oracle(q.contiguous()), to_oracle(k), to_oracle(v),
+                            np.array(pos, np.int64) if pos is not None else None, window, -1.0)
+    out = torch.empty_like(q)
+    if P:
+        kv, keep_k = pages_of(ops, k, P, shift)
+        vv, keep_v = pages_of(ops, v, P, shift)
+        ops.attention_paged_view(q, kv, vv, p, window, out=out)
+    else:
+        ops.attention(q, k, v, p, window, out=out)
+    ops.check_device_errors()
+    assert_close(out.contiguous(), want, dtype, f"B{B} hq{hq} hkv{hkv} tq{tq} tk{tk} D{D} pos{pos} w{window} P{P}")
+
+
+SHAPES = [
+    # one row tile and less, more keys than queries, several queries a tile column
+    dict(B=1, hq=1, hkv=1, tq=2, tk=2, D=64, pos=None, window=0),
+    dict(B=2, hq=8, hkv=2, tq=9, tk=40, D=64, pos=[31, 5], window=0),
+    dict(B=1, hq=8, hkv=1, tq=37, tk=200, D=64, pos=[163], window=0),
+    # several row tiles with a ragged end; a group that does not divide the tile
+    dict(B=1, hq=6, hkv=2, tq=65, tk=65, D=64, pos=None, window=0),
+    dict(B=1, hq=12, hkv=12, tq=130, tk=130, D=64, pos=[0], window=0),
+    dict(B=1, hq=4, hkv=2, tq=67, tk=131, D=128, pos=[64], window=0),
+    dict(B=2, hq=4, hkv=1, tq=33, tk=97, D=256, pos=[64, 3], window=0),
+    # windows: inside a tile, across tiles; rows that see no key
+    dict(B=1, hq=4, hkv=2, tq=50, tk=150, D=64, pos=[100], window=7),
+    dict(B=1, hq=4, hkv=2, tq=50, tk=250, D=128, pos=[190], window=100),
+    dict(B=2, hq=2, hkv=1, tq=40, tk=60, D=256, pos=[30, 200], window=33),
+    # offsets past the last key
+    dict(B=1, hq=2, hkv=2, tq=35, tk=70, D=64, pos=[500], window=0),
+]
+
+
+@pytest.mark.parametrize("rows", ["", "1", "2"])
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_prefill_matches_oracle(ops, oracle, monkeypatch, shape, rows):
+    """Every row-tile form (32 rows a workgroup with the keys split over four
+    waves, 64 over two) and the one chosen by size."""
+    if rows:
+        monkeypatch.setenv("SANDY_PREFILL_RW", rows)
+    check(ops, oracle, torch.bfloat16, **shape)
+
+
+@pytest.mark.parametrize("shape", [SHAPES[2], SHAPES[5], SHAPES[9]], ids=str)
+def test_prefill_strided_heads_and_pages(ops, oracle, shape):
+    """q and out with the heads inside the tokens; K/V from page lists of 1,
+    16 and 64 rows, also where pages start on odd elements."""
+    check(ops, oracle, torch.bfloat16, heads_inner=True, **shape)
+    for P, shift in ((1, 0), (16, 0), (64, 8), (16, 3)):
+        check(ops, oracle, torch.bfloat16, P=P, shift=shift, **shape)
+
+
+@pytest.mark.parametrize("P", [0, 16])
+def test_prefill_non_finite_values_reach_only_their_rows(ops, oracle, P):
+    """An infinity or NaN in V, or a NaN in K, changes the rows that see its
+    key and no other (the reference never reads a masked key)."""
+    def spoil(k, v):
+        v[0, 0, 70, 3] = float("inf")
+        v[0, 1, 90, 5] = float("nan")
+        v[0, 1, 20, 6] = float("-inf")
+        k[0, 0, 95, 1] = float("nan")
+        k[0, 1, 98, 2] = float("inf")
+    check(ops, oracle, torch.bfloat16, B=1, hq=4, hkv=2, tq=60, tk=100, D=64, pos=[40], window=30, P=P, spoil=spoil)
+
+
+def test_prefill_errors(ops):
+    """A negative offset and a null page are recorded."""
+    from sandyrt_amd._lib import SandyError
+    q = torch.zeros(1, 2, 4, 64, dtype=torch.bfloat16, device="cuda")
+    k = torch.zeros(1, 1, 20, 64, dtype=torch.bfloat16, device="cuda")
+    ops.attention(q, k, k, torch.tensor([-1], device="cuda"))
+    with pytest.raises(SandyError, match="attention position_offsets must be non-negative"):
+        ops.check_device_errors()
+    view, keep = pages_of(ops, k, 16)
+    view.pages[1] = 0
+    ops.attention_paged_view(q, view, view, torch.tensor([4], device="cuda"))  # keys 0..7: page 0 alone
+    ops.check_device_errors()
+    ops.attention_paged_view(q, view, view, torch.tensor([14], device="cuda"))
+    with pytest.raises(SandyError, match="block id outside the pool"):
+        ops.check_device_errors()
