@@ -15,7 +15,7 @@
 //
 // The reference hands both to cuBLAS (cublasGemmEx, CudaMatMulKernels.cu:
 // 173-216; its CUDA linear is not implemented, CudaDevice.cpp:536-537).
-// Here there are three kernels:
+// Here there are four kernels:
 //   - bf16 with the weight read row-major as [n, k] (transpose_rhs, the
 //     layout of every projection and the lm-head) runs on
 //     v_mfma_f32_16x16x32_bf16 with fp32 accumulation:
@@ -25,14 +25,16 @@
 //         the last-arriving workgroup of each output tile summing the fp32
 //         partials in split order -- one launch, no second reduction pass;
 //       gemm_lines_kernel for larger row counts: 64 x 256 tiles;
-//   - gemm_simt_kernel: every other case (f32, either operand transposed,
-//     unaligned shapes).  Register-tiled FMA-free float loops that keep the
-//     reference's k order per output, so f32 results are bit-identical to the
-//     CPU path.
+//   - f32 in the same layout runs gemm_ordered_kernel, FMA-free float loops
+//     that keep the reference's k order per output, so f32 results are
+//     bit-identical to the CPU path;
+//   - gemm_simt_kernel: every other case (other layouts, unaligned shapes),
+//     register-tiled, in the same order.
 #include "gemm.h"
 
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 namespace sandy_hip {
 namespace {
@@ -249,118 +251,148 @@ __global__ __launch_bounds__(256) void gemm_simt_kernel(const void* __restrict__
     }
 }
 
+// f32 products against a weight read as [n, k] (linear, and matmul with
+// transpose_rhs) in the reference's k order: every output is acc = (bias or
+// 0), then acc + x * w rounded at each step (no FMA), so results stay
+// bit-identical to the CPU path and MFMA, which sums in another order, is out.
+// Bound: two VALU instructions a multiply-add, 39 TFLOP/s over 1024 SIMDs; a
+// single output's chain alone takes 8 K cycles, so small products want one
+// output a lane on as many SIMDs as there are, large ones R rows a lane to
+// amortise the operand reads.  A wave owns R rows x 64 columns; chunks of 64 k
+// of its operands go global -> registers (a ring of kRing chunks, so that the
+// weight stream stays in flight over several short chunks) -> LDS.  A lane
+// reads its column 4 k at a time, and of each row the 4 k that its place in a
+// quad of lanes names: the multiply takes the quad's lane j by DPP, so an
+// activation costs one 16-byte LDS read per 16 k and no instruction of its own.
+// Measured (before: 64 x 64 tiles, and one wave per 16 columns up to 8 rows):
+// 64 x 768 x 768 119 -> 12 us, 64 x 768 x 3072 542 -> 36, 1000 x 3072 x 768 at
+// 35 TFLOP/s, 1 x 50257 x 768 62 -> 33.
+typedef float f32v4_t __attribute__((ext_vector_type(4)));
+
+// lane (4 (lane / 4) + Q)'s v
+template <int Q>
+__device__ __forceinline__ float quad_lane(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), Q * 0x55, 0xf, 0xf, true));
+}
+
+template <int R>
+__global__ __launch_bounds__(256, R == 1 ? 2 : 3) void gemm_ordered_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                           const float* __restrict__ bias, float* __restrict__ out,
+                                                           int64_t M, int64_t N, int64_t K, int32_t row_tiles,
+                                                           BatchMap bm) {
+    constexpr int kBK = 64;                      // k per chunk
+    constexpr int kPitch = kBK + 4;              // floats per weight row in LDS: 64 lanes x 16 bytes, no conflict
+    constexpr int kRows = 4 * R;                 // rows and columns of the workgroup
+    constexpr int kCols = 64;
+    constexpr int kW = kCols * kBK / 4 / 256;    // 16-byte pieces of w a thread stages per chunk
+    constexpr int kX = (kRows * kBK / 4 + 255) / 256;
+    constexpr int kRing = R == 1 ? 3 : 2;
+    static_assert(R <= 4, "x pieces of a chunk: at most one a thread");
+    __shared__ __attribute__((aligned(16))) float wl[2][kCols * kPitch];
+    __shared__ __attribute__((aligned(16))) float xl[2][kRows * kBK];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t r0 = static_cast<int64_t>(blockIdx.x % row_tiles) * kRows, m0 = r0 + wave * R;
+    const int64_t n0 = static_cast<int64_t>(blockIdx.x / row_tiles) * kCols, n = n0 + lane;
+    int64_t lo, ro;
+    batch_offsets(bm, blockIdx.z, lo, ro);
+    const int prow = tid / 16, ppc = tid % 16;   // piece (row prow + 16 i, 4 ppc .. + 3) of a chunk
+    const float* wp[kW];
+    const float* xp[kX];
+#pragma unroll
+    for (int i = 0; i < kW; i++) wp[i] = w + ro + min<int64_t>(n0 + prow + 16 * i, N - 1) * K;
+#pragma unroll
+    for (int i = 0; i < kX; i++) xp[i] = x + lo + min<int64_t>(r0 + prow + 16 * i, M - 1) * K;
+    const bool x_on = kRows >= 16 || prow < kRows;
+    f32v4_t wv[kRing][kW], xv[kRing][kX];
+    auto load = [&](int64_t c, int slot) {
+        const int64_t k = min<int64_t>(c * kBK + 4 * ppc, K - 4);  // pieces past K are not used
+#pragma unroll
+        for (int i = 0; i < kW; i++) wv[slot][i] = *reinterpret_cast<const f32v4_t*>(wp[i] + k);
+#pragma unroll
+        for (int i = 0; i < kX; i++) xv[slot][i] = *reinterpret_cast<const f32v4_t*>(xp[i] + k);
+    };
+    float acc[R];
+    float b0 = bias && n < N ? bias[n] : 0.0f;
+    asm volatile("" : "+v"(b0));  // waited for here, not (with the weights in flight) in the loop
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[r] = b0;
+    const float* wr = &wl[0][lane * kPitch];
+    const float* xr = &xl[0][wave * R * kBK + 4 * (lane & 3)];
+    auto put = [&](int slot, int buf) {
+#pragma unroll
+        for (int i = 0; i < kW; i++)
+            *reinterpret_cast<f32v4_t*>(&wl[buf][(prow + 16 * i) * kPitch + 4 * ppc]) = wv[slot][i];
+        if (x_on) {
+#pragma unroll
+            for (int i = 0; i < kX; i++) *reinterpret_cast<f32v4_t*>(&xl[buf][(prow + 16 * i) * kBK + 4 * ppc]) = xv[slot][i];
+        }
+        __syncthreads();
+    };
+    // 16 k (the first 4 `quads` of them) of the chunk in `buf`
+    const bool live = m0 < M;  // a wave past the last row only stages
+    auto sixteen = [&](int buf, int s, int quads) {
+        f32v4_t a[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) a[r] = *reinterpret_cast<const f32v4_t*>(xr + buf * kRows * kBK + r * kBK + 16 * s);
+        auto step = [&](auto quad) {
+            constexpr int q = decltype(quad)::value;
+            if (q >= quads) return;
+            const f32v4_t b = *reinterpret_cast<const f32v4_t*>(wr + buf * kCols * kPitch + 16 * s + 4 * q);
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int r = 0; r < R; r++) acc[r] = __fadd_rn(acc[r], __fmul_rn(quad_lane<q>(a[r][j]), b[j]));
+        };
+        step(std::integral_constant<int, 0>{});
+        step(std::integral_constant<int, 1>{});
+        step(std::integral_constant<int, 2>{});
+        step(std::integral_constant<int, 3>{});
+    };
+    auto whole = [&](int buf) {
+        if (!live) return;
+#pragma unroll
+        for (int s = 0; s < kBK / 16; s++) sixteen(buf, s, 4);
+    };
+    // rings of whole chunks, every load unconditional so that the wait counts
+    // stay exact (past the last chunk its pieces are loaded again); then the
+    // chunks left, the last of them perhaps partial
+    const int64_t chunks = (K + kBK - 1) / kBK, full = K / kBK;
+#pragma unroll
+    for (int q = 0; q < kRing; q++) load(q, q);
+    int64_t c = 0;
+    int buf = 0;
+    for (; c + kRing <= full; c += kRing) {
+#pragma unroll
+        for (int slot = 0; slot < kRing; slot++) {
+            put(slot, buf);
+            load(c + kRing + slot, slot);
+            whole(buf);
+            buf ^= 1;
+        }
+    }
+#pragma unroll
+    for (int slot = 0; slot < kRing; slot++) {
+        if (c + slot < chunks) {
+            put(slot, buf);
+            const int quads = static_cast<int>(min<int64_t>(kBK, K - (c + slot) * kBK) / 4);
+#pragma unroll 1
+            for (int s = 0; live && 4 * s < quads; s++) sixteen(buf, s, quads - 4 * s);
+            buf ^= 1;
+        }
+    }
+    if (n >= N) return;
+#pragma unroll
+    for (int r = 0; r < R; r++)
+        if (m0 + r < M) out[(static_cast<int64_t>(blockIdx.z) * M + m0 + r) * N + n] = acc[r];
+}
+
 // --------------------------------------------------------------------- host
 struct Plan {
     int64_t M, N, K, batches;
     int64_t lrs, rrs;  // row strides (last dims) of lhs and rhs
     BatchMap bm;
 };
-
-// f32 products of a few rows against a weight read as [n, k] (linear, and
-// matmul with transpose_rhs).  Each output column walks k in the reference's
-// order (acc = bias, then acc + x * w rounded at each step, no contraction),
-// so results stay bit-identical to the CPU path.  A wave owns 16 output
-// columns: it loads their weight rows 32 k at a time as whole 128-byte lines
-// (8 lanes per line, Q chunks in flight) into an LDS tile, and lanes 0..15
-// then walk their row in order.  Per-lane row streams (64 distinct lines per
-// load instruction) were bound by the CU's outstanding misses (59 us for
-// 768 x 768); 16 columns per wave also spreads a 768-column output over 48
-// CUs.  The activation rows are staged in LDS per block of k.
-template <int MR, int Q>
-__global__ __launch_bounds__(64) void gemv_seq_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                     const float* __restrict__ bias, float* __restrict__ out,
-                                                     int64_t M, int64_t N, int64_t K, BatchMap bm) {
-    constexpr int kCols = 16;  // output columns per wave
-    constexpr int kXs = 8192;  // activation floats staged in LDS per block of k
-    constexpr int kRow = 33;   // tile row stride in floats (conflict-free column walks)
-    __shared__ float xs[kXs];
-    __shared__ float tile[kCols * kRow];
-    const int lane = threadIdx.x;
-    const int64_t n0 = static_cast<int64_t>(blockIdx.x) * kCols;
-    const int64_t n = n0 + lane;
-    const int64_t bz = blockIdx.z;
-    int64_t lo, ro;
-    batch_offsets(bm, bz, lo, ro);
-    const bool live = lane < kCols && n < N;
-    const float* xr = x + lo;
-    // this lane's two 16-byte pieces of each chunk: rows (lane / 8) and 8 + (lane / 8), piece lane % 8
-    const int prow[2] = {lane >> 3, 8 + (lane >> 3)};
-    const float* wrow[2];
-#pragma unroll
-    for (int i = 0; i < 2; i++) wrow[i] = w + ro + min<int64_t>(n0 + prow[i], N - 1) * K + (lane & 7) * 4;
-    float acc[MR];
-    const float b0 = bias && live ? bias[n] : 0.0f;
-#pragma unroll
-    for (int r = 0; r < MR; r++) acc[r] = b0;
-    const int64_t kb_len = max<int64_t>(32, (kXs / M) & ~int64_t(31));
-    float4 buf[Q][2];
-    for (int64_t kb = 0; kb < K; kb += kb_len) {
-        const int64_t len = min(kb_len, K - kb);
-        __syncthreads();  // the previous block's reads of xs are done
-        for (int64_t j = lane; j < M * len; j += 64) {
-            const int64_t r = j / len, kk = j - r * len;
-            xs[r * len + kk] = xr[r * K + kb + kk];
-        }
-        __syncthreads();
-        const int64_t nch = len / 32;
-        auto load = [&](int64_t c, int slot) {
-#pragma unroll
-            for (int i = 0; i < 2; i++) buf[slot][i] = *reinterpret_cast<const float4*>(wrow[i] + kb + c * 32);
-        };
-#pragma unroll
-        for (int q = 0; q < Q; q++)
-            if (q < nch) load(q, q);
-        for (int64_t c0 = 0; c0 < nch; c0 += Q) {
-#pragma unroll
-            for (int q = 0; q < Q; q++) {
-                const int64_t c = c0 + q;
-                if (c >= nch) break;
-#pragma unroll
-                for (int i = 0; i < 2; i++) {
-                    float* t = tile + prow[i] * kRow + (lane & 7) * 4;
-                    t[0] = buf[q][i].x;
-                    t[1] = buf[q][i].y;
-                    t[2] = buf[q][i].z;
-                    t[3] = buf[q][i].w;
-                }
-                if (c + Q < nch) load(c + Q, q);
-                __syncthreads();
-                if (lane < kCols) {
-                    // every LDS read is unconditional (rows past M read row M - 1), so the
-                    // compiler issues them ahead of the in-order chain; only the
-                    // accumulate is selected
-                    const float* trow = tile + lane * kRow;
-                    float wv[32];
-#pragma unroll
-                    for (int j = 0; j < 32; j++) wv[j] = trow[j];
-#pragma unroll
-                    for (int r = 0; r < MR; r++) {
-                        const float* xc = xs + min<int64_t>(r, M - 1) * len + c * 32;
-                        float xv[32];
-#pragma unroll
-                        for (int j = 0; j < 32; j++) xv[j] = xc[j];
-                        float a_r = acc[r];
-#pragma unroll
-                        for (int j = 0; j < 32; j++) a_r = __fadd_rn(a_r, __fmul_rn(xv[j], wv[j]));
-                        acc[r] = r < M ? a_r : acc[r];
-                    }
-                }
-                __syncthreads();  // the tile is rewritten by the next chunk
-            }
-        }
-        if (live)  // k tail past the 32-wide chunks, in order
-            for (int64_t kk = nch * 32; kk < len; kk++) {
-                const float wv = w[ro + n * K + kb + kk];
-#pragma unroll
-                for (int r = 0; r < MR; r++)
-                    if (r < M) acc[r] = __fadd_rn(acc[r], __fmul_rn(xs[r * len + kk], wv));
-            }
-    }
-    if (!live) return;
-#pragma unroll
-    for (int r = 0; r < MR; r++)
-        if (r < M) out[(bz * M + r) * N + n] = acc[r];
-}
 
 // Fills the plan from operand shapes with the reference's rules; returns an
 // error message or null.
@@ -441,21 +473,24 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
         return fail(e, SANDY_ERR_UNSUPPORTED, "%s needs bf16 operands, k a multiple of 32 and at most 64 rows", what);
     if (fz && p.batches != 1) return fail(e, SANDY_ERR_UNSUPPORTED, "%s takes one [m, k] matrix", what);
     const bool norm = fz && fz->norm_w;
-    // f32, few rows, weight rows contiguous: the exact-order GEMV
-    const bool gemv = l.dtype == SANDY_F32 && !tl && tr && p.M <= 8 && p.K % 4 == 0 && aligned &&
-                      p.lrs == p.K && p.rrs == p.K && env_int("SANDY_GEMM_SIMT", 0) == 0;
-    if (gemv) {
-        const int64_t blocks = (p.N + 15) / 16;
-        if (blocks > 0x7fffffff) return fail(e, SANDY_ERR_UNSUPPORTED, "%s shape exceeds the launch grid", what);
-        const dim3 grid(static_cast<unsigned>(blocks), 1, static_cast<unsigned>(p.batches));
-        const float* x = static_cast<const float*>(pl);
-        const float* w = static_cast<const float*>(pr);
-        const float* b = static_cast<const float*>(pb);
-        float* y = static_cast<float*>(po);
-        if (p.M == 1) hipLaunchKernelGGL((gemv_seq_kernel<1, 8>), grid, dim3(64), 0, stream, x, w, b, y, p.M, p.N, p.K, p.bm);
-        else if (p.M <= 2) hipLaunchKernelGGL((gemv_seq_kernel<2, 8>), grid, dim3(64), 0, stream, x, w, b, y, p.M, p.N, p.K, p.bm);
-        else if (p.M <= 4) hipLaunchKernelGGL((gemv_seq_kernel<4, 8>), grid, dim3(64), 0, stream, x, w, b, y, p.M, p.N, p.K, p.bm);
-        else hipLaunchKernelGGL((gemv_seq_kernel<8, 8>), grid, dim3(64), 0, stream, x, w, b, y, p.M, p.N, p.K, p.bm);
+    // f32 against a weight read as [n, k], in the reference's k order
+    const bool ordered = l.dtype == SANDY_F32 && !tl && tr && p.K % 4 == 0 && p.K > 0 && aligned &&
+                         env_int("SANDY_GEMM_SIMT", 0) == 0;
+    if (ordered) {
+        // one row a lane while that takes at most two waves a SIMD, else four
+        // (one wave alone issues a VALU instruction every 7 cycles, several
+        // every 4, so small products want more waves, not more rows a wave):
+        // us at R = 1 / 4 for rows x columns x k: 64 x 768 x 768 12 / 20,
+        // 64 x 768 x 3072 36 / 71, 1 x 50257 x 768 33 / 43; 64 x 3072 x 768
+        // 25 / 22, 200 x 768 x 768 23 / 21, 1000 x 3072 x 768 258 / 136
+        const int64_t ct = (p.N + 63) / 64;
+        const int R = env_int("SANDY_GEMM_ROWS", p.M * ct * p.batches <= 2048 ? 1 : 4) == 1 ? 1 : 4;
+        const int64_t rt = (p.M + 4 * R - 1) / (4 * R);
+        if (rt * ct > 0x7fffffff) return fail(e, SANDY_ERR_UNSUPPORTED, "%s shape exceeds the launch grid", what);
+        const dim3 grid(static_cast<unsigned>(rt * ct), 1, static_cast<unsigned>(p.batches));
+        hipLaunchKernelGGL(R == 1 ? gemm_ordered_kernel<1> : gemm_ordered_kernel<4>, grid, dim3(256), 0, stream,
+                           static_cast<const float*>(pl), static_cast<const float*>(pr), static_cast<const float*>(pb),
+                           static_cast<float*>(po), p.M, p.N, p.K, static_cast<int32_t>(rt), p.bm);
     } else if (waves) {
         GemmArgs g{};
         g.a = static_cast<const uint16_t*>(pl);

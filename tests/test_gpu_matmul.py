@@ -221,6 +221,24 @@ def test_linear_f32_few_rows_bit_exact(ops, oracle, rows, in_f, out_f):
                  oracle.matmul(to_oracle(x), to_oracle(w), transpose_rhs=True), "matmul transposed rhs")
 
 
+@pytest.mark.parametrize("rows_a_lane", ["1", "4"])
+@pytest.mark.parametrize("rows,in_f,out_f", [(1, 4, 1), (9, 60, 65), (17, 64, 130), (16, 68, 64), (33, 132, 63),
+                                             (5, 196, 70), (70, 380, 129)])
+def test_linear_f32_ordered_tiles_bit_exact(ops, oracle, rows_a_lane, rows, in_f, out_f):
+    """The k-ordered f32 kernel at the edges of its row tiles (4 and 16 rows),
+    column tile (64) and chunk (64 k, rings of 2 and 3 chunks): bit-identical
+    to the CPU, with bias and batched without."""
+    r = rng(rows + in_f * 7 + out_f)
+    x = from_f32(normal(r, (rows, in_f)), torch.float32)
+    w = from_f32(normal(r, (out_f, in_f), 0.02), torch.float32)
+    b = from_f32(normal(r, (out_f,)), torch.float32)
+    x3 = from_f32(normal(r, (3, rows, in_f)), torch.float32)
+    with env(SANDY_GEMM_ROWS=rows_a_lane):
+        got, got3 = ops.linear(x, w, b), ops.matmul(x3, w.unsqueeze(0), transpose_rhs=True)
+    assert_equal(got, oracle.linear(to_oracle(x), to_oracle(w), to_oracle(b)), "linear")
+    assert_equal(got3, oracle.matmul(to_oracle(x3), to_oracle(w.unsqueeze(0)), transpose_rhs=True), "batched matmul")
+
+
 @pytest.mark.parametrize("act", ["silu", "gelu"])
 @pytest.mark.parametrize("m,k,ffn", [(1, 2048, 5632), (5, 64, 80), (32, 2048, 5632), (64, 2560, 1024),
                                      (32, 5632, 96), (3, 128, 40)])
