@@ -7,6 +7,8 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import struct
+import threading
 
 import torch
 
@@ -275,29 +277,43 @@ def dcall(name: str, *args):
         raise SandyError(rc, buf.value.decode(errors="replace"))
 
 
+# SandyTensor as bytes, one layout per rank: data, dtype, rank, dims, strides, storage_offset
+_TENSOR_LAYOUT = [struct.Struct(f"=Qii{r}q{8 * (MAX_RANK - r)}x{r}q{8 * (MAX_RANK - r)}xq") for r in range(MAX_RANK + 1)]
+
+
+def pack(t: torch.Tensor) -> bytes:
+    """The bytes of the SandyTensor describing a torch tensor's view (data is
+    the view's first element, storage_offset 0)."""
+    rank = t.dim()
+    if rank > MAX_RANK:
+        raise SandyError(1, f"tensor rank {rank} exceeds {MAX_RANK}")
+    return _TENSOR_LAYOUT[rank].pack(t.data_ptr(), _TORCH_TO_CODE[t.dtype], rank, *t.shape, *t.stride(), 0)
+
+
+def arg(t: torch.Tensor | None):
+    """A tensor argument of an entry point: its SandyTensor (ctypes passes its
+    address), or NULL.  Packed at once: setting the fields one by one took
+    7 us a tensor, most of a small call."""
+    return None if t is None else SandyTensor.from_buffer_copy(pack(t))
+
+
 def desc(t: torch.Tensor | None):
-    """SandyTensor describing a torch tensor's storage view (or NULL)."""
-    if t is None:
-        return None
-    if t.dim() > MAX_RANK:
-        raise SandyError(1, f"tensor rank {t.dim()} exceeds {MAX_RANK}")
-    d = SandyTensor()
-    d.data = t.untyped_storage().data_ptr() if t.numel() else t.data_ptr()
-    d.dtype = _TORCH_TO_CODE[t.dtype]
-    d.rank = t.dim()
-    for i in range(t.dim()):
-        d.dims[i] = t.shape[i]
-        d.strides[i] = t.stride(i)
-    d.storage_offset = t.storage_offset() if t.numel() else 0
-    return C.pointer(d)
+    """Pointer to a SandyTensor describing a torch tensor's view (or NULL)."""
+    return None if t is None else C.pointer(arg(t))
+
+
+_local = threading.local()
 
 
 def call(name: str, *args, stream=None):
     """Invoke an entry point on `stream` (default: torch's current stream)."""
     if stream is None:
-        stream = torch.cuda.current_stream().cuda_stream
-    buf = C.create_string_buffer(512)
-    rc = getattr(lib(), name)(*args, C.c_void_p(stream), buf, C.c_size_t(512))
+        stream = torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    try:
+        buf = _local.err
+    except AttributeError:
+        buf = _local.err = C.create_string_buffer(512)  # this thread's error text
+    rc = getattr(_lib or lib(), name)(*args, stream, buf, 512)
     if rc != 0:
         raise SandyError(rc, buf.value.decode(errors="replace"))
 

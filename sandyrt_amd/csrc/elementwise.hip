@@ -291,7 +291,7 @@ struct Compiled {
 };
 
 std::mutex g_mu;
-std::map<std::pair<int, std::string>, Compiled> g_cache;
+std::map<std::string, Compiled> g_cache;
 
 int compile(const std::string& src, Compiled* out, Err e) {
     hiprtcProgram prog;
@@ -406,16 +406,37 @@ extern "C" int sandy_hip_elementwise(const SandyScalarNode* nodes, int32_t node_
     }
 
     const int U = vec_chunks(n);
-    const std::string src = generate(nodes, node_count, result, dts, modes, input_count, out->dtype, vec, U);
     int dev = 0;
     SANDY_HIP_TRY(hipGetDevice(&dev), e, "hipGetDevice");
+    // compiled groups by everything the generated source depends on; writing the
+    // source out to look it up took 8 us of host time a call
+    std::string key;
+    auto put = [&key](const auto& v) { key.append(reinterpret_cast<const char*>(&v), sizeof(v)); };
+    put(dev);
+    put(result);
+    put(node_count);
+    for (int i = 0; i < node_count; i++) {
+        put(nodes[i].id);
+        put(nodes[i].op);
+        if (nodes[i].op == 0) put(nodes[i].input_index);
+        if (nodes[i].op == 1) put(nodes[i].constant);
+        const int need = nodes[i].op <= 1 ? 0 : nodes[i].op <= 7 ? 2 : 1;
+        for (int j = 0; j < need; j++) put(nodes[i].operands[j]);
+    }
+    put(input_count);
+    for (int i = 0; i < input_count; i++) {
+        put(dts[i]);
+        put(modes[i]);
+    }
+    put(out->dtype);
+    put(vec);
+    put(U);
     Compiled c;
     {
         std::lock_guard<std::mutex> lock(g_mu);
-        auto key = std::make_pair(dev, src);
         auto it = g_cache.find(key);
         if (it == g_cache.end()) {
-            int st = compile(src, &c, e);
+            int st = compile(generate(nodes, node_count, result, dts, modes, input_count, out->dtype, vec, U), &c, e);
             if (st) return st;
             g_cache.emplace(key, c);
         } else {

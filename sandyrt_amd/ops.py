@@ -13,12 +13,14 @@ torch's current stream and do not synchronise, except `check_device_errors`.
 from __future__ import annotations
 
 import ctypes as C
+import functools
+import struct
 from dataclasses import dataclass
 
 import torch
 
 from . import _lib
-from ._lib import SandyError, call, desc
+from ._lib import SandyError, arg, call, pack
 
 # ScalarOp codes (src/ir/KernelIR.h:317-337)
 LOAD, CONST, ADD, SUB, MUL, DIV, MAX, MIN, NEG, SQRT, RSQRT, EXP, LOG, TANH, RELU, CAST = range(16)
@@ -66,15 +68,16 @@ def paged_to_dense(x: PagedTensor, out=None):
     """The logical elements of a paged tensor as a contiguous tensor (the
     gather every family runs on a paged input before its dense kernel)."""
     out = torch.empty(x.dims, dtype=x.dtype, device=x.device) if out is None else out
-    call("sandy_hip_paged_to_dense", x.struct(), desc(out))
+    call("sandy_hip_paged_to_dense", x.struct(), arg(out))
     return out
+
+
+_NOT_PAGED = frozenset((torch.Tensor, int, float, bool, type(None)))
 
 
 def _reads_paged(fn):
     """Inputs given as PagedTensor (also inside a list of inputs) are gathered
     to dense copies before the family's dense entry point runs."""
-    import functools
-
     def dense(v):
         if isinstance(v, PagedTensor):
             return paged_to_dense(v)
@@ -84,7 +87,11 @@ def _reads_paged(fn):
 
     @functools.wraps(fn)
     def run(*args, **kw):
-        return fn(*[dense(a) for a in args], **{k: (v if k == "out" else dense(v)) for k, v in kw.items()})
+        if not _NOT_PAGED.issuperset(map(type, args)):
+            args = [dense(a) for a in args]
+        if kw and not _NOT_PAGED.issuperset(map(type, kw.values())):
+            kw = {k: (v if k == "out" else dense(v)) for k, v in kw.items()}
+        return fn(*args, **kw)
 
     return run
 
@@ -101,7 +108,7 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor | None, epsilon: float, out=N
     """NormKernelOp RMSNorm (src/core/TensorCalc.cpp:1953-2000)."""
     _require_gpu(x, weight)
     out = torch.empty_like(x) if out is None else out
-    call("sandy_hip_norm", 0, desc(x), desc(weight), None, float(epsilon), desc(out))
+    call("sandy_hip_norm", 0, arg(x), arg(weight), None, float(epsilon), arg(out))
     return out
 
 
@@ -110,7 +117,7 @@ def layer_norm(x, weight, bias, epsilon: float, out=None):
     """NormKernelOp LayerNorm (src/core/TensorCalc.cpp:2010-2077)."""
     _require_gpu(x, weight, bias)
     out = torch.empty_like(x) if out is None else out
-    call("sandy_hip_norm", 1, desc(x), desc(weight), desc(bias), float(epsilon), desc(out))
+    call("sandy_hip_norm", 1, arg(x), arg(weight), arg(bias), float(epsilon), arg(out))
     return out
 
 
@@ -119,7 +126,7 @@ def add_rms_norm(x, residual, weight, epsilon: float, sum_out=None, out=None):
     _require_gpu(x, residual, weight)
     sum_out = torch.empty_like(x) if sum_out is None else sum_out
     out = torch.empty_like(x) if out is None else out
-    call("sandy_hip_add_rms_norm", desc(x), desc(residual), desc(weight), float(epsilon), desc(sum_out), desc(out))
+    call("sandy_hip_add_rms_norm", arg(x), arg(residual), arg(weight), float(epsilon), arg(sum_out), arg(out))
     return sum_out, out
 
 
@@ -129,8 +136,8 @@ def rope(x, theta: float, rotary_dim: int = -1, split_half: bool = False, positi
     """RoPEKernelOp (src/core/TensorCalc.cpp:1823-1951)."""
     _require_gpu(x, position_ids)
     out = torch.empty_like(x) if out is None else out
-    call("sandy_hip_rope", desc(x), desc(position_ids), float(theta), int(rotary_dim), int(bool(split_half)),
-         desc(out))
+    call("sandy_hip_rope", arg(x), arg(position_ids), float(theta), int(rotary_dim), int(bool(split_half)),
+         arg(out))
     return out
 
 
@@ -141,8 +148,8 @@ def rope_pair(q, k, theta: float, rotary_dim: int = -1, split_half: bool = False
     _require_gpu(q, k, position_ids)
     q_out = torch.empty_like(q) if q_out is None else q_out
     k_out = torch.empty_like(k) if k_out is None else k_out
-    call("sandy_hip_rope_pair", desc(q), desc(k), desc(position_ids), float(theta), int(rotary_dim),
-         int(bool(split_half)), desc(q_out), desc(k_out))
+    call("sandy_hip_rope_pair", arg(q), arg(k), arg(position_ids), float(theta), int(rotary_dim),
+         int(bool(split_half)), arg(q_out), arg(k_out))
     return q_out, k_out
 
 
@@ -153,8 +160,8 @@ def rope_cache(seq: int, dim: int, theta: float, rotary_dim: int = -1, split_hal
     _require_gpu(position_ids)
     rd = dim if rotary_dim < 0 else rotary_dim
     out = torch.empty(seq, rd // 2, 2, dtype=torch.float32, device=device) if out is None else out
-    call("sandy_hip_rope_cache", desc(position_ids), int(seq), float(theta), int(rotary_dim), int(dim),
-         int(bool(split_half)), desc(out))
+    call("sandy_hip_rope_cache", arg(position_ids), int(seq), float(theta), int(rotary_dim), int(dim),
+         int(bool(split_half)), arg(out))
     return out
 
 
@@ -163,7 +170,7 @@ def rope_pair_cached(q, k, cache, q_out=None, k_out=None):
     _require_gpu(q, k, cache)
     q_out = torch.empty_like(q) if q_out is None else q_out
     k_out = (torch.empty_like(k) if k_out is None else k_out) if k is not None else None
-    call("sandy_hip_rope_pair_cached", desc(q), desc(k), desc(cache), desc(q_out), desc(k_out))
+    call("sandy_hip_rope_pair_cached", arg(q), arg(k), arg(cache), arg(q_out), arg(k_out))
     return q_out, k_out
 
 
@@ -172,7 +179,7 @@ def softmax(x, axis: int = -1, out=None):
     """SoftmaxKernelOp (src/core/TensorCalc.cpp:1337-1399)."""
     _require_gpu(x)
     out = torch.empty_like(x) if out is None else out
-    call("sandy_hip_softmax", desc(x), int(axis), desc(out))
+    call("sandy_hip_softmax", arg(x), int(axis), arg(out))
     return out
 
 
@@ -187,7 +194,7 @@ def sum(x, axis: int = -1, keep_dims: bool = True, out=None):  # noqa: A001 - re
     else:
         del shape[ax]
     out = torch.empty(shape, dtype=x.dtype, device=x.device) if out is None else out
-    call("sandy_hip_reduce_sum", desc(x), int(axis), int(bool(keep_dims)), desc(out))
+    call("sandy_hip_reduce_sum", arg(x), int(axis), int(bool(keep_dims)), arg(out))
     return out
 
 
@@ -197,7 +204,7 @@ def embedding(ids, weight, out=None):
     _require_gpu(ids, weight)
     shape = list(ids.shape) + list(weight.shape[1:])
     out = torch.empty(shape, dtype=weight.dtype, device=weight.device) if out is None else out
-    call("sandy_hip_gather", desc(ids), desc(weight), desc(out))
+    call("sandy_hip_gather", arg(ids), arg(weight), arg(out))
     return out
 
 
@@ -213,18 +220,26 @@ class ScalarNode:
     operands: tuple = ()
 
 
+_NODE_LAYOUT = struct.Struct("=IiiIdi2I4x")  # SandyScalarNode
+
+
+@functools.lru_cache(maxsize=256)
+def _packed_nodes(key):
+    """SandyScalarNode array of (id, op, input_index, constant, operands) tuples."""
+    def u32(*v):
+        return [x & 0xFFFFFFFF for x in v]  # as a C field takes them: the library rejects what is out of range
+
+    if any(len(operands) > 2 for *_, operands in key):
+        raise IndexError("a scalar node has at most two operands")
+    data = b"".join(_NODE_LAYOUT.pack(*u32(i), op, _lib.F32, *u32(inp), float(const), len(operands),
+                                      *u32(*operands, *(0,) * (2 - len(operands))))
+                    for i, op, inp, const, operands in key)
+    return (_lib.SandyScalarNode * len(key)).from_buffer_copy(data)
+
+
 def _nodes(nodes):
-    arr = (_lib.SandyScalarNode * len(nodes))()
-    for i, n in enumerate(nodes):
-        arr[i].id = n.id
-        arr[i].op = n.op
-        arr[i].dtype = _lib.F32
-        arr[i].input_index = n.input_index
-        arr[i].constant = float(n.constant)
-        arr[i].operand_count = len(n.operands)
-        for j, o in enumerate(n.operands):
-            arr[i].operands[j] = o
-    return arr
+    # looked up by content; zeros by their text, which keeps their sign
+    return _packed_nodes(tuple([(n.id, n.op, n.input_index, n.constant or str(n.constant), tuple(n.operands)) for n in nodes]))
 
 
 @_reads_paged
@@ -238,11 +253,9 @@ def elementwise(nodes, result: int, inputs, broadcast=None, out_shape=None, out_
         dtype = out_dtype if out_dtype is not None else inputs[0].dtype
         out = torch.empty(shape, dtype=dtype, device=inputs[0].device)
     n = len(inputs)
-    arr = (_lib.SandyTensor * max(1, n))()
-    for i, t in enumerate(inputs):
-        arr[i] = desc(t).contents
-    bc = (C.c_int32 * max(1, n))(*[int(bool(b)) for b in broadcast])
-    call("sandy_hip_elementwise", _nodes(nodes), len(nodes), int(result), arr, bc, n, desc(out))
+    arr = (_lib.SandyTensor * n).from_buffer_copy(b"".join([pack(t) for t in inputs])) if n else None
+    bc = (C.c_int32 * n)(*[int(bool(b)) for b in broadcast]) if n else None
+    call("sandy_hip_elementwise", _nodes(nodes), len(nodes), int(result), arr, bc, n, arg(out))
     return out
 
 
@@ -294,8 +307,8 @@ def attention(q, k, v, position_offsets=None, window: int = 0, scale: float = -1
     """AttentionKernelOp over dense K/V (src/core/TensorCalc.cpp:1167-1314)."""
     _require_gpu(q, k, v, position_offsets)
     out = torch.empty_like(q) if out is None else out
-    call("sandy_hip_attention", desc(q), desc(k), desc(v), desc(position_offsets), int(window), float(scale),
-         desc(out))
+    call("sandy_hip_attention", arg(q), arg(k), arg(v), arg(position_offsets), int(window), float(scale),
+         arg(out))
     return out
 
 
@@ -340,8 +353,8 @@ def paged_attention(q, k_cache: PagedCache, v_cache: PagedCache, block_table, po
     """Decode attention (Tq = 1) over paged K/V; block_table [B, max_blocks] int32."""
     _require_gpu(q, block_table, position_offsets, k_cache.pool, v_cache.pool)
     out = torch.empty_like(q) if out is None else out
-    call("sandy_hip_paged_attention", desc(q), k_cache.struct(), v_cache.struct(), desc(block_table),
-         desc(position_offsets), int(window), float(scale), desc(out))
+    call("sandy_hip_paged_attention", arg(q), k_cache.struct(), v_cache.struct(), arg(block_table),
+         arg(position_offsets), int(window), float(scale), arg(out))
     return out
 
 
@@ -354,7 +367,7 @@ def layout_transform(x: torch.Tensor, out: torch.Tensor | None = None, kind: int
     in row-major order, into out (default: a contiguous tensor of x's shape)."""
     _require_gpu(x, out)
     out = torch.empty(x.shape, dtype=x.dtype, device=x.device) if out is None else out
-    call("sandy_hip_layout_transform", desc(x), desc(out), int(kind))
+    call("sandy_hip_layout_transform", arg(x), arg(out), int(kind))
     return out
 
 
@@ -386,8 +399,8 @@ def attention_paged_view(q, k: PagedView, v: PagedView, position_offsets=None, w
     padded T, position_offsets [B])."""
     _require_gpu(q, k.pages, v.pages)
     out = torch.empty_like(q) if out is None else out
-    call("sandy_hip_attention_paged_view", desc(q), k.struct(), v.struct(), desc(position_offsets), int(window),
-         float(scale), desc(out))
+    call("sandy_hip_attention_paged_view", arg(q), k.struct(), v.struct(), arg(position_offsets), int(window),
+         float(scale), arg(out))
     return out
 
 
@@ -398,8 +411,8 @@ def paged_attention_noalloc(q, k_cache: PagedCache, v_cache: PagedCache, block_t
     given by callers that cannot allocate."""
     _require_gpu(q, block_table, position_offsets, k_cache.pool, v_cache.pool)
     out = torch.empty_like(q) if out is None else out
-    call("sandy_hip_paged_attention_noalloc", desc(q), k_cache.struct(), v_cache.struct(), desc(block_table),
-         desc(position_offsets), int(window), float(scale), desc(out))
+    call("sandy_hip_paged_attention_noalloc", arg(q), k_cache.struct(), v_cache.struct(), arg(block_table),
+         arg(position_offsets), int(window), float(scale), arg(out))
     return out
 
 
@@ -412,7 +425,7 @@ def topk(x, k: int, axis: int = -1, index_dtype=torch.int64, values=None, indice
     shape[ax] = k
     values = torch.empty(shape, dtype=x.dtype, device=x.device) if values is None else values
     indices = torch.empty(shape, dtype=index_dtype, device=x.device) if indices is None else indices
-    call("sandy_hip_topk", desc(x), int(k), int(axis), desc(values), desc(indices))
+    call("sandy_hip_topk", arg(x), int(k), int(axis), arg(values), arg(indices))
     return values, indices
 
 
@@ -428,8 +441,8 @@ def moe_gather(x, topk_ids, topk_weights, num_experts: int, index_dtype=torch.in
     packed_w = torch.empty(lead + [rows], dtype=topk_weights.dtype, device=dev)
     token_ids = torch.empty(lead + [rows], dtype=index_dtype, device=dev)
     offsets = torch.empty(lead + [num_experts + 1], dtype=index_dtype, device=dev)
-    call("sandy_hip_moe_gather", desc(x), desc(topk_ids), desc(topk_weights), int(num_experts), int(top_k),
-         desc(packed_x), desc(packed_w), desc(token_ids), desc(offsets))
+    call("sandy_hip_moe_gather", arg(x), arg(topk_ids), arg(topk_weights), int(num_experts), int(top_k),
+         arg(packed_x), arg(packed_w), arg(token_ids), arg(offsets))
     return packed_x, packed_w, token_ids, offsets
 
 
@@ -438,7 +451,7 @@ def moe_matmul(x, expert_offsets, weight, transpose_rhs: bool = True, out=None):
     _require_gpu(x, expert_offsets, weight)
     m = weight.shape[1] if transpose_rhs else weight.shape[2]
     out = torch.empty(list(x.shape[:-1]) + [m], dtype=x.dtype, device=x.device) if out is None else out
-    call("sandy_hip_moe_matmul", desc(x), desc(expert_offsets), desc(weight), int(bool(transpose_rhs)), desc(out))
+    call("sandy_hip_moe_matmul", arg(x), arg(expert_offsets), arg(weight), int(bool(transpose_rhs)), arg(out))
     return out
 
 
@@ -447,7 +460,7 @@ def moe_scatter_sum(packed_out, packed_weights, token_ids, seq: int, out=None):
     _require_gpu(packed_out, packed_weights, token_ids)
     shape = list(packed_out.shape[:-2]) + [seq, packed_out.shape[-1]]
     out = torch.empty(shape, dtype=packed_out.dtype, device=packed_out.device) if out is None else out
-    call("sandy_hip_moe_scatter_sum", desc(packed_out), desc(packed_weights), desc(token_ids), desc(out))
+    call("sandy_hip_moe_scatter_sum", arg(packed_out), arg(packed_weights), arg(token_ids), arg(out))
     return out
 
 
@@ -479,7 +492,7 @@ def matmul(lhs, rhs, transpose_lhs: bool = False, transpose_rhs: bool = False, o
     if out is None:
         shape = _matmul_shape(list(lhs.shape), list(rhs.shape), transpose_lhs, transpose_rhs)
         out = torch.empty(shape, dtype=lhs.dtype, device=lhs.device)
-    call("sandy_hip_matmul", desc(lhs), desc(rhs), int(bool(transpose_lhs)), int(bool(transpose_rhs)), desc(out))
+    call("sandy_hip_matmul", arg(lhs), arg(rhs), int(bool(transpose_lhs)), int(bool(transpose_rhs)), arg(out))
     return out
 
 
@@ -510,7 +523,7 @@ def matmul_glu(x, w_interleaved, activation: str = "silu", out=None):
     code = {"silu": 1, "gelu": 2}[activation]
     shape = list(x.shape[:-1]) + [w_interleaved.shape[0] // 2]
     out = torch.empty(shape, dtype=x.dtype, device=x.device) if out is None else out
-    call("sandy_hip_matmul_glu", desc(x), desc(w_interleaved), code, desc(out))
+    call("sandy_hip_matmul_glu", arg(x), arg(w_interleaved), code, arg(out))
     return out
 
 
@@ -532,7 +545,7 @@ def matmul_residual(x, weight, residual, stats=None, out=None):
     _require_gpu(x, weight, residual)
     out = torch.empty(list(x.shape[:-1]) + [weight.shape[0]], dtype=x.dtype, device=x.device) if out is None else out
     st = C.byref(row_stats(stats)) if stats is not None else None
-    call("sandy_hip_matmul_residual", desc(x), desc(weight), desc(residual), desc(out), st)
+    call("sandy_hip_matmul_residual", arg(x), arg(weight), arg(residual), arg(out), st)
     return out
 
 
@@ -544,8 +557,8 @@ def matmul_rms(x, stats, norm_weight, epsilon: float, weight, activation: str | 
     code = {None: 0, "silu": 1, "gelu": 2}[activation]
     n = weight.shape[0] // (2 if code else 1)
     out = torch.empty(list(x.shape[:-1]) + [n], dtype=x.dtype, device=x.device) if out is None else out
-    call("sandy_hip_matmul_rms", desc(x), C.byref(row_stats(stats)), desc(norm_weight), float(epsilon), desc(weight),
-         code, desc(out))
+    call("sandy_hip_matmul_rms", arg(x), C.byref(row_stats(stats)), arg(norm_weight), float(epsilon), arg(weight),
+         code, arg(out))
     return out
 
 
@@ -557,8 +570,8 @@ def decode_linear(x, weight, bias=None, ln_weight=None, ln_bias=None, epsilon: f
     shape = list(x.shape[:-1]) + [weight.shape[0]]
     out = torch.empty(shape, dtype=x.dtype, device=x.device) if out is None else out
     act = {None: 0, "gelu": 2}[activation]
-    call("sandy_hip_decode_linear", desc(x), desc(ln_weight), desc(ln_bias), C.c_double(epsilon), desc(weight),
-         desc(bias), C.c_int32(act), desc(residual), desc(out))
+    call("sandy_hip_decode_linear", arg(x), arg(ln_weight), arg(ln_bias), C.c_double(epsilon), arg(weight),
+         arg(bias), C.c_int32(act), arg(residual), arg(out))
     return out
 
 
@@ -566,5 +579,5 @@ def linear(x, weight, bias, out=None):
     """LinearKernelOp (TensorCalc.cpp:722-773): bias + x @ weight^T."""
     _require_gpu(x, weight, bias)
     out = torch.empty(list(x.shape[:-1]) + [weight.shape[0]], dtype=x.dtype, device=x.device) if out is None else out
-    call("sandy_hip_linear", desc(x), desc(weight), desc(bias), desc(out))
+    call("sandy_hip_linear", arg(x), arg(weight), arg(bias), arg(out))
     return out

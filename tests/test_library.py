@@ -5,6 +5,8 @@ import ctypes
 import os
 import re
 
+import pytest
+
 from sandyrt_amd import _lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -76,3 +78,32 @@ def test_paged_operand_checks_on_the_host():
         _lib.call("sandy_hip_paged_to_dense", pt(), ctypes.byref(bad), stream=0)
     with pytest.raises(_lib.SandyError, match="slot out of range"):
         _lib.call("sandy_hip_paged_stage", pt(), ctypes.c_int32(-1), ctypes.byref(dst), stream=0)
+
+
+def test_packed_arguments():
+    """Tensor and node arguments packed as bytes: the fields the C structs
+    hold, for every rank and view, and nodes told apart by content (a node
+    list changed in place, the sign of a zero constant)."""
+    import torch
+
+    from sandyrt_amd import _lib, ops
+
+    base = torch.arange(2 * 3 * 4 * 5, dtype=torch.float32).view(2, 3, 4, 5)
+    for t in (base, base[1:, :, 2:].permute(2, 0, 3, 1), base[1, 2, 3, 4], base.view(1, 1, 1, 1, 2, 3, 4, 5).bfloat16(),
+              base[:0], torch.zeros(3, dtype=torch.int64)):
+        d = _lib.desc(t).contents
+        n = t.dim()
+        assert (d.data or 0) == t.data_ptr() and d.storage_offset == 0
+        assert d.dtype == _lib._TORCH_TO_CODE[t.dtype] and d.rank == n
+        assert list(d.dims) == list(t.shape) + [0] * (8 - n) and list(d.strides) == list(t.stride()) + [0] * (8 - n)
+    with pytest.raises(_lib.SandyError, match="rank 9"):
+        _lib.desc(base.view(1, 1, 1, 1, 1, 2, 3, 4, 5))
+
+    nodes = [ops.ScalarNode(0, ops.LOAD, 1), ops.ScalarNode(1, ops.CONST, constant=0.0),
+             ops.ScalarNode(2, ops.MUL, operands=[0, 1])]
+    first = [(n.id, n.op, n.dtype, n.input_index, n.constant, n.operand_count, list(n.operands)) for n in ops._nodes(nodes)]
+    assert first == [(0, 0, 0, 1, 0.0, 0, [0, 0]), (1, 1, 0, 0, 0.0, 0, [0, 0]), (2, 4, 0, 0, 0.0, 2, [0, 1])]
+    nodes[1].constant = -0.0
+    assert str(ops._nodes(nodes)[1].constant) == "-0.0"
+    nodes[1].constant = 3.5
+    assert ops._nodes(nodes)[1].constant == 3.5
