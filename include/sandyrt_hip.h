@@ -285,6 +285,9 @@ int sandy_hip_gather(const SandyTensor* ids, const SandyTensor* table, const San
  * src/device/cuda/CudaAttentionKernels.cu:680-766).  q [B,Hq,Tq,D] (or rank
  * 3), k/v [B,Hkv,Tk,D]; position_offsets (NULL or [B]) shifts query
  * positions; window > 0 is a sliding window; scale <= 0 means 1/sqrt(D).
+ * Several queries of head dim 64 or 128 (bf16 also 256) with 16-byte aligned
+ * rows run on MFMA, float32 sums in another order than the reference's; other
+ * shapes keep its order.
  */
 int sandy_hip_attention(const SandyTensor* q, const SandyTensor* k, const SandyTensor* v,
                         const SandyTensor* position_offsets, int64_t window, double scale,
@@ -312,7 +315,8 @@ int sandy_hip_paged_attention(const SandyTensor* q, const SandyPagedCache* k_cac
  * src/core/TensorCalc.cpp:1167-1314).  q [B,Hq,Tq,D] (or rank 3) and out as
  * in sandy_hip_attention; k and v are reference-layout paged views.  Decode
  * (Tq = 1, bf16, D 64/128/256) runs the MFMA paged decode kernel reading the
- * page table directly; other shapes run the general attention kernel.
+ * page table directly; several queries of D 64/128 (bf16 also 256) run the MFMA
+ * prefill kernel, other shapes the general attention kernel.
  * The decode kernel reads pages with 16-byte loads: a page address that is
  * null or not 16-byte aligned is recorded as SANDY_DEVERR_BLOCK and the page
  * contributes no keys.

@@ -1,5 +1,6 @@
 // attention.hip -- AttentionKernelOp: paged decode on bf16 MFMA, plus a
-// general kernel for dense K/V, fp32 and uncommon shapes.
+// general kernel for fp32 decode and uncommon shapes (prompts:
+// attention_prefill.hip).
 //
 // Semantics: src/core/TensorCalc.cpp:1167-1314 (attention_impl).  Query qi of
 // batch b sits at position offsets[b] + qi; key ki attends when
@@ -1240,9 +1241,12 @@ static bool prefill_args(const GenArgs& g, int64_t B, PrefillArgs* p) {
     p->tq = g.tq;
     p->tk = static_cast<int32_t>(g.tk);
     p->window = g.window;
+    p->scale = g.scale;
     p->scale_log2 = g.scale * kLog2e;
+    p->dtype = g.dt;
+    p->dim = g.d;
     p->errw = g.errw;
-    return prefill_takes(*p, g.dt, g.d);
+    return prefill_takes(*p);
 }
 
 extern "C" int sandy_hip_attention(const SandyTensor* q, const SandyTensor* k, const SandyTensor* v,
@@ -1306,7 +1310,7 @@ extern "C" int sandy_hip_attention(const SandyTensor* q, const SandyTensor* k, c
     a.scale = scale <= 0.0 ? 1.0f / sqrtf(static_cast<float>(D)) : static_cast<float>(scale);
     a.errw = errw;
     PrefillArgs pre;
-    if (prefill_args(a, B, &pre)) return launch_prefill(pre, D, stream, e);
+    if (prefill_args(a, B, &pre)) return launch_prefill(pre, stream, e);
     const size_t sbytes = static_cast<size_t>(B * hq * tq * std::max<int64_t>(tk, 1)) * sizeof(float);
     a.scores = static_cast<float*>(device_workspace(1, sbytes, stream, e, &status));
     if (status) return status;
@@ -1584,7 +1588,8 @@ extern "C" int sandy_hip_paged_attention(const SandyTensor* q, const SandyPagedC
 // with paged = true: page table, logical shape, page size and count).  Same
 // validation and semantics as sandy_hip_attention on the dense tensors the
 // pages hold; decode steps (Tq = 1) of the bf16 MFMA shapes take the paged
-// decode kernel in page-table mode, everything else the general kernel.
+// decode kernel in page-table mode, prompts the prefill kernel
+// (attention_prefill.hip), everything else the general kernel.
 extern "C" int sandy_hip_attention_paged_view(const SandyTensor* q, const SandyPagedView* k, const SandyPagedView* v,
                                               const SandyTensor* position_offsets, int64_t window, double scale,
                                               const SandyTensor* out, void* stream_, char* err, size_t err_cap) {
@@ -1685,7 +1690,7 @@ extern "C" int sandy_hip_attention_paged_view(const SandyTensor* q, const SandyP
     a.scale = sc;
     a.errw = errw;
     PrefillArgs pre;
-    if (prefill_args(a, B, &pre)) return launch_prefill(pre, D, stream, e);
+    if (prefill_args(a, B, &pre)) return launch_prefill(pre, stream, e);
     const size_t sbytes = static_cast<size_t>(B * hq * tq * std::max<int64_t>(tk, 1)) * sizeof(float);
     a.scores = static_cast<float*>(device_workspace(1, sbytes, stream, e, &status));
     if (status) return status;

@@ -27,13 +27,15 @@ struct PrefillArgs {
     int32_t row_blocks;  // row tiles per (b, kh)
     int32_t table_pages; // page addresses staged in LDS (0: read from memory)
     int64_t window;
-    float scale_log2;  // scale * log2(e)
+    float scale, scale_log2;  // scale * log2(e)
+    int32_t dtype;            // F32 or BF16
+    int64_t dim;              // head dim
     uint32_t* errw;
 };
 
 // Whether the kernel takes the shape (the caller's general kernel takes the
 // rest), and its launch.
-bool prefill_takes(const PrefillArgs& a, int32_t dtype, int64_t head_dim);
-int launch_prefill(PrefillArgs a, int64_t head_dim, hipStream_t stream, Err e);
+bool prefill_takes(const PrefillArgs& a);
+int launch_prefill(const PrefillArgs& a, hipStream_t stream, Err e);
 
 } // namespace sandy_hip

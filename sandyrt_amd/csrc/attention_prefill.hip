@@ -1,6 +1,6 @@
 // attention_prefill.hip -- causal attention of prompts and prompt chunks
-// (AttentionKernelOp with Tq > 1, src/core/TensorCalc.cpp:1167-1314), bf16,
-// over dense K/V or the reference's paged K/V.
+// (AttentionKernelOp with Tq > 1, src/core/TensorCalc.cpp:1167-1314), bf16
+// and f32, over dense K/V or the reference's paged K/V.
 //
 // The general kernel (attention.hip) runs one workgroup per (query, head)
 // and walks the keys in the reference's order; every query re-reads its K and
@@ -16,6 +16,9 @@
 //     V^T read by ds_read_b64_tr_b16 in the same key order;
 //   - P enters as two bf16 operands (hi + lo), about 17 bits of each
 //     probability; the row sums are kept in float64.
+// f32 takes v_mfma_f32_32x32x2_f32 for both products (f32 operands throughout,
+// P straight from its registers) and expf; bound by that instruction's rate, a
+// sixteenth of the bf16 one's.
 // Four score waves a workgroup: RW of them own 32 rows each and KW = 4 / RW
 // share the keys of a chunk (merged at the end), so short prompts still fill
 // the chip; at D 256 a second wave per score tile owns half of the head dims.
@@ -24,10 +27,12 @@
 // Bound: softmax VALU work (49% of the cycles at D 64, MFMA 22%).  Measured,
 // us a call (general kernel -> here): 2048 queries, 32 / 4 heads, D 64
 // 14357 -> 44; 777 queries after 1500 keys, window 1024, 8 / 2 heads, D 256,
-// pages of 16: 4896 -> 46; 1500 after 300, 16 / 2 heads, D 128: 54.
+// pages of 16: 4896 -> 46; 1500 after 300, 16 / 2 heads, D 128: 54; f32, 12
+// heads, D 64: 1000 queries 1434 -> 43, 64 queries 23.5 -> 9.8.
 #include "attention_prefill.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace sandy_hip {
 namespace {
@@ -45,9 +50,11 @@ constexpr int kTablePages = 512;  // page addresses of K and V held in LDS
 // Geometry of a variant.  LDS rows are padded so that MFMA-layout reads touch
 // every bank once: 16 lanes x 16 bytes down a K column (pitch 16 bytes past a
 // multiple of 128), 4 rows x 64 bytes of V per transposing read (pitch 64
-// bytes past a multiple of 256 or 128).
-template <int D, int RW>
+// bytes past a multiple of 256 or 128), for f32 two V rows 4 apart x 128 bytes.
+template <typename T, int D, int RW>
 struct Geo {
+    static constexpr bool kF32 = std::is_same_v<T, F32>;
+    static constexpr int ES = kF32 ? 4 : 2;   // bytes of an element
     // D 256: two waves share a score tile and own half of the head dims each,
     // so that two waves fit a SIMD (one wave with all of O^T in its registers
     // had nothing to run behind its waits)
@@ -56,11 +63,13 @@ struct Geo {
     static constexpr int DT = D / 32 / DS;    // 32-dim tiles of O^T a wave owns
     static constexpr int KW = 4 / RW;
     static constexpr int CK = KW * 32;        // keys of a chunk, 32 a wave
-    static constexpr int KP = 2 * D + 16;     // bytes per K row in LDS
-    static constexpr int VP = 2 * D + 64;     // bytes per V row in LDS
+    static constexpr int KP = ES * D + 16;               // bytes per K row in LDS
+    static constexpr int VP = ES * D + (kF32 ? 32 : 64);  // bytes per V row in LDS
     static constexpr int kBuf = CK * (KP + VP);
-    static constexpr int NB = 2 * kBuf <= 160 * 1024 - 512 ? 2 : 1;  // LDS buffers
-    static constexpr int NP = CK * D / 8 / THREADS;  // 16-byte pieces of K (and of V) a thread stages
+    // LDS buffers: two where they fit, for f32 only beside a second workgroup
+    // (its matrix work per chunk is long enough to cover the copy)
+    static constexpr int NB = 2 * kBuf <= (kF32 ? 79 : 159) * 1024 ? 2 : 1;
+    static constexpr int NP = CK * D * ES / 16 / THREADS;  // 16-byte pieces of K (and of V) a thread stages
     // final merge: [KW - 1][RW] copies of a wave's accumulators, and (m, l)
     static constexpr int kMerge = (KW - 1) * RW * D * 32 * 4;
     static constexpr int kStats = 4 * 32 * 16;  // of the waves of the first half
@@ -68,10 +77,10 @@ struct Geo {
 };
 
 // Byte address of row `key` of the page at `at` on page row `row`, rounded
-// down to whole elements.
-__device__ __forceinline__ uint64_t paged_row(uint64_t at, int key, int log2_page, int64_t row, int row_bytes) {
+// down to whole elements of `es` bytes.
+__device__ __forceinline__ uint64_t paged_row(uint64_t at, int key, int log2_page, int64_t row, int row_bytes, int es) {
     const int64_t in_page = key & ((1 << log2_page) - 1);
-    return (at & ~uint64_t{1}) + static_cast<uint64_t>(((row << log2_page) + in_page) * row_bytes);
+    return (at & ~static_cast<uint64_t>(es - 1)) + static_cast<uint64_t>(((row << log2_page) + in_page) * row_bytes);
 }
 
 // 16 bytes from a row whose start is only element aligned.
@@ -88,21 +97,21 @@ __device__ __forceinline__ u32x4_t load_piece(uint64_t at) {
 // the row sees adds its normalised probability times V (from the row's known
 // max and 1 / sum), so a non-finite V reaches exactly the rows that see its
 // key.  256 keys at a time through `probs`; q in `qrow`.
-template <int D, bool PAGED>
-__device__ __forceinline__ void careful_row(const PrefillArgs& a, int b, int kh, int row, int first, int last,
-                                                      float m, float inv, float* probs, void* qrow) {
+template <typename T, int D, bool PAGED>
+__device__ __forceinline__ void careful_row(const PrefillArgs& a, int b, int kh, int row, int first, int last, float m,
+                                            float inv, float* probs, float* qf) {
+    constexpr int ES = Geo<T, D, 1>::ES;
     const int tid = threadIdx.x;
     const int t = row / a.group, h = kh * a.group + row % a.group;
-    float* qf = static_cast<float*>(qrow);
-    if (tid < D) qf[tid] = bf16_to_f32(static_cast<const uint16_t*>(a.q)[b * a.qs[0] + h * a.qs[1] + t * a.qs[2] + tid]);
-    auto row_of = [&](bool value, int key) -> const uint16_t* {
+    if (tid < D) qf[tid] = Vec8<T>::load1(a.q, b * a.qs[0] + h * a.qs[1] + t * a.qs[2] + tid);
+    auto row_of = [&](bool value, int key) -> const void* {
         if constexpr (PAGED) {
             const uint64_t at = (value ? a.v_pages : a.k_pages)[key >> a.log2_page];
-            return at ? reinterpret_cast<const uint16_t*>(paged_row(at, key, a.log2_page, b * a.kv_rows_b + kh, 2 * D))
+            return at ? reinterpret_cast<const void*>(paged_row(at, key, a.log2_page, b * a.kv_rows_b + kh, ES * D, ES))
                       : nullptr;
         } else {
             const int64_t* st = value ? a.vs : a.ks;
-            return static_cast<const uint16_t*>(value ? a.v : a.k) + b * st[0] + kh * st[1] + key * st[2];
+            return static_cast<const char*>(value ? a.v : a.k) + (b * st[0] + kh * st[1] + key * st[2]) * ES;
         }
     };
     float acc = 0.0f;
@@ -110,31 +119,34 @@ __device__ __forceinline__ void careful_row(const PrefillArgs& a, int b, int kh,
         __syncthreads();
         const int n = min(256, last + 1 - k0);
         if (tid < n) {
-            const uint16_t* kp = row_of(false, k0 + tid);
+            const void* kp = row_of(false, k0 + tid);
             float s = 0.0f;
 #pragma unroll 1
-            for (int d = 0; d < D; d++) s = fmaf(qf[d], kp ? bf16_to_f32(kp[d]) : 0.0f, s);
-            probs[tid] = __builtin_amdgcn_exp2f(fmaf(s, a.scale_log2, -m)) * inv;
+            for (int d = 0; d < D; d++) s = fmaf(qf[d], kp ? Vec8<T>::load1(kp, d) : 0.0f, s);
+            probs[tid] = (Geo<T, D, 1>::kF32 ? expf(s * a.scale - m)
+                                             : __builtin_amdgcn_exp2f(fmaf(s, a.scale_log2, -m))) * inv;
         }
         __syncthreads();
         if (tid < D) {
 #pragma unroll 1
             for (int i = 0; i < n; i++) {
-                const uint16_t* vp = row_of(true, k0 + i);
-                acc = fmaf(probs[i], vp ? bf16_to_f32(vp[tid]) : 0.0f, acc);
+                const void* vp = row_of(true, k0 + i);
+                acc = fmaf(probs[i], vp ? Vec8<T>::load1(vp, tid) : 0.0f, acc);
             }
         }
     }
-    if (tid < D && first <= last)
-        static_cast<uint16_t*>(a.out)[b * a.os[0] + h * a.os[1] + t * a.os[2] + tid] = f32_to_bf16(acc);
+    if (tid < D && first <= last) Vec8<T>::store1(a.out, b * a.os[0] + h * a.os[1] + t * a.os[2] + tid, acc);
     __syncthreads();
 }
 
-template <int D, int RW, bool PAGED>
-__global__ __launch_bounds__((Geo<D, RW>::THREADS), 2) void attention_prefill_kernel(PrefillArgs a) {
-    using G_ = Geo<D, RW>;
+template <typename T, int D, int RW, bool PAGED>
+__global__ __launch_bounds__((Geo<T, D, RW>::THREADS), (Geo<T, D, RW>::kF32 && D == 128 ? 1 : 2)) void attention_prefill_kernel(PrefillArgs a) {
+    using G_ = Geo<T, D, RW>;
     constexpr int KW = G_::KW, SUB = 32, CK = G_::CK, KP = G_::KP, VP = G_::VP, NP = G_::NP, DT = G_::DT;
-    constexpr int kPieces = D / 8;  // 16-byte pieces per row
+    constexpr bool kF32 = G_::kF32;
+    constexpr int ES = G_::ES;
+    constexpr int kPieces = D * ES / 16;  // 16-byte pieces per row
+    constexpr int kQ = D * ES / 32;       // 16-byte pieces of q a lane holds
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -175,19 +187,20 @@ __global__ __launch_bounds__((Geo<D, RW>::THREADS), 2) void attention_prefill_ke
     const int any_first = first_of(t_lo), any_last = last_of(t_hi);
     const int all_first = first_of(t_hi), all_last = last_of(t_lo);
 
-    bf16x8_t qv[D / 16];  // B operands: column = query, 16 s + 8 half .. + 7
+    // B operands: column = query; 16 bytes of q from 32 s + 16 half on (bf16: one
+    // step of 16 dims; f32: four steps of 2, slot `half` of step i element i)
+    u32x4_t qv[kQ];
     {
-        const uint16_t* qp = static_cast<const uint16_t*>(a.q) + b * a.qs[0] + (kh * a.group + qg) * a.qs[1] +
-                             qt * a.qs[2] + 8 * half;
+        const char* qp = static_cast<const char*>(a.q) + (b * a.qs[0] + (kh * a.group + qg) * a.qs[1] + qt * a.qs[2]) * ES + 16 * half;
 #pragma unroll
-        for (int s = 0; s < D / 16; s++) qv[s] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(qp + 16 * s));
+        for (int s = 0; s < kQ; s++) qv[s] = *reinterpret_cast<const u32x4_t*>(qp + 32 * s);
     }
 
     // ---- staging: thread piece i covers chunk row prow + i * (256 / kPieces), 16-byte piece ppc
     constexpr int kRowStep = G_::THREADS / kPieces;
     const int prow = tid / kPieces, ppc = tid % kPieces;
-    const uint16_t* kbase = static_cast<const uint16_t*>(a.k) + (PAGED ? 0 : b * a.ks[0] + kh * a.ks[1] + 8 * ppc);
-    const uint16_t* vbase = static_cast<const uint16_t*>(a.v) + (PAGED ? 0 : b * a.vs[0] + kh * a.vs[1] + 8 * ppc);
+    const char* kbase = static_cast<const char*>(a.k) + (PAGED ? 0 : (b * a.ks[0] + kh * a.ks[1]) * ES + 16 * ppc);
+    const char* vbase = static_cast<const char*>(a.v) + (PAGED ? 0 : (b * a.vs[0] + kh * a.vs[1]) * ES + 16 * ppc);
     const uint32_t page_row = static_cast<uint32_t>(b * a.kv_rows_b + kh);
     u32x4_t kr[NP], vr[NP];
     bool pages_ok = true;
@@ -221,10 +234,10 @@ __global__ __launch_bounds__((Geo<D, RW>::THREADS), 2) void attention_prefill_ke
                     vat[i] = a.v_pages[page];
                 }
                 // byte offset of the row within the page: below 2^31 (checked on the host)
-                const uint32_t off = ((page_row << a.log2_page) + (key & ((1 << a.log2_page) - 1))) * (2 * D) + 16 * ppc;
+                const uint32_t off = ((page_row << a.log2_page) + (key & ((1 << a.log2_page) - 1))) * (ES * D) + 16 * ppc;
                 plain = plain && kat[i] != 0 && vat[i] != 0 && ((kat[i] | vat[i]) & 15) == 0;
-                kat[i] = kat[i] ? (kat[i] & ~uint64_t{1}) + off : 0;
-                vat[i] = vat[i] ? (vat[i] & ~uint64_t{1}) + off : 0;
+                kat[i] = kat[i] ? (kat[i] & ~uint64_t{ES - 1}) + off : 0;
+                vat[i] = vat[i] ? (vat[i] & ~uint64_t{ES - 1}) + off : 0;
             }
             if (__all(plain)) {
 #pragma unroll
@@ -243,8 +256,8 @@ __global__ __launch_bounds__((Geo<D, RW>::THREADS), 2) void attention_prefill_ke
         } else {
 #pragma unroll
             for (int i = 0; i < NP; i++) {
-                kr[i] = *reinterpret_cast<const u32x4_t*>(kbase + key_of(c0, i) * a.ks[2]);
-                vr[i] = *reinterpret_cast<const u32x4_t*>(vbase + key_of(c0, i) * a.vs[2]);
+                kr[i] = *reinterpret_cast<const u32x4_t*>(kbase + key_of(c0, i) * a.ks[2] * ES);
+                vr[i] = *reinterpret_cast<const u32x4_t*>(vbase + key_of(c0, i) * a.vs[2] * ES);
             }
         }
     };
@@ -284,9 +297,16 @@ __global__ __launch_bounds__((Geo<D, RW>::THREADS), 2) void attention_prefill_ke
 #pragma unroll
         for (int i = 0; i < 16; i++) sc[i] = 0.0f;
 #pragma unroll
-        for (int s = 0; s < D / 16; s++) {
-            const bf16x8_t kv = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(kt + 32 * s));
-            sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kv, qv[s], sc, 0, 0, 0);
+        for (int s = 0; s < kQ; s++) {
+            const u32x4_t kv = *reinterpret_cast<const u32x4_t*>(kt + 32 * s);
+            if constexpr (kF32) {
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    sc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(kv[i]), __uint_as_float(qv[s][i]), sc, 0, 0, 0);
+            } else {
+                sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kv),
+                                                             __builtin_bit_cast(bf16x8_t, qv[s]), sc, 0, 0, 0);
+            }
         }
         // element i of sc: key k0 + 8 (i / 4) + 4 half + i % 4
         if (partial) {
@@ -301,13 +321,15 @@ __global__ __launch_bounds__((Geo<D, RW>::THREADS), 2) void attention_prefill_ke
         float mx = sc[0];
 #pragma unroll
         for (int i = 1; i < 16; i++) mx = fmaxf(mx, sc[i]);
-        mx = max_xor32(mx) * a.scale_log2;
+        // bf16: exponents in the exp2 domain; f32: expf of scaled scores, as the
+        // general kernel takes them
+        mx = max_xor32(mx) * (kF32 ? a.scale : a.scale_log2);
         // the reference point m of a row's exponents moves only when its max has
         // grown by 2^8 (p stays below that, its relative precision is the same),
         // so most chunks leave the accumulators alone
-        if (__any(mx > m + 8.0f)) {
+        if (__any(mx > m + (kF32 ? 5.5f : 8.0f))) {
             const float m_new = fmaxf(m, mx);
-            const float alpha = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - m_new);
+            const float alpha = m == -INFINITY ? 0.0f : kF32 ? expf(m - m_new) : __builtin_amdgcn_exp2f(m - m_new);
             l *= static_cast<double>(alpha);
             if (__any(m != -INFINITY)) {
 #pragma unroll
@@ -316,6 +338,22 @@ __global__ __launch_bounds__((Geo<D, RW>::THREADS), 2) void attention_prefill_ke
             m = m_new;
         }
         const float shift = m == -INFINITY ? 0.0f : m;
+        if constexpr (kF32) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                sc[i] = expf(sc[i] * a.scale - shift);
+                l += static_cast<double>(sc[i]);
+            }
+            // step i: slot `half` is key 8 (i / 4) + 4 half + i % 4, this lane's element i
+            const unsigned char* src = vt + 4 * half * VP + 4 * col;
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+#pragma unroll
+                for (int t = 0; t < DT; t++)
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                        *reinterpret_cast<const float*>(src + (8 * (i >> 2) + (i & 3)) * VP + 128 * (DT * ds + t)), sc[i], acc[t], 0, 0, 0);
+            continue;
+        }
         float rs = 0.0f;
 #pragma unroll
         for (int i = 0; i < 16; i++) {
@@ -375,9 +413,10 @@ __global__ __launch_bounds__((Geo<D, RW>::THREADS), 2) void attention_prefill_ke
 #pragma unroll
         for (int w = 0; w < KW; w++) {
             const double* e = ml + ((w * RW + rw) * 32 + col) * 2;
-            ll += e[1] * static_cast<double>(__builtin_amdgcn_exp2f(static_cast<float>(e[0]) - shift));
+            const float d = static_cast<float>(e[0]) - shift;
+            ll += e[1] * static_cast<double>(kF32 ? expf(d) : __builtin_amdgcn_exp2f(d));
         }
-        const float f = __builtin_amdgcn_exp2f(m - shift);
+        const float f = kF32 ? expf(m - shift) : __builtin_amdgcn_exp2f(m - shift);
 #pragma unroll
         for (int t = 0; t < DT; t++) acc[t] *= f;
         m = mm;
@@ -404,7 +443,7 @@ __global__ __launch_bounds__((Geo<D, RW>::THREADS), 2) void attention_prefill_ke
     const bool none = m == -INFINITY;
     bool finite = true;
     if (kw == 0 && row < rows) {
-        uint16_t* op = static_cast<uint16_t*>(a.out) + b * a.os[0] + (kh * a.group + qg) * a.os[1] + qt * a.os[2] + 32 * DT * ds + 4 * half;
+        char* op = static_cast<char*>(a.out) + (b * a.os[0] + (kh * a.group + qg) * a.os[1] + qt * a.os[2] + 32 * DT * ds + 4 * half) * ES;
 #pragma unroll
         for (int t = 0; t < DT; t++)
 #pragma unroll
@@ -415,7 +454,9 @@ __global__ __launch_bounds__((Geo<D, RW>::THREADS), 2) void attention_prefill_ke
                     o[x] = none ? 0.0f : acc[t][4 * i + x] * inv;
                     finite = finite && fabsf(o[x]) < INFINITY;
                 }
-                *reinterpret_cast<uint2*>(op + 32 * t + 8 * i) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+                char* to = op + (32 * t + 8 * i) * ES;
+                if constexpr (kF32) *reinterpret_cast<float4*>(to) = make_float4(o[0], o[1], o[2], o[3]);
+                else *reinterpret_cast<uint2*>(to) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
             }
     }
     if (!__syncthreads_or(finite ? 0 : 1)) return;
@@ -426,15 +467,16 @@ __global__ __launch_bounds__((Geo<D, RW>::THREADS), 2) void attention_prefill_ke
     }
     __syncthreads();
     for (int i = 0; i < 32 * RW && r0 + i < rows; i++)
-        if (stats[i] != -INFINITY) careful_row<D, PAGED>(a, b, kh, r0 + i, first_of((r0 + i) / a.group), last_of((r0 + i) / a.group), stats[i],
-                              stats[32 * RW + i], reinterpret_cast<float*>(lds) + 64 * RW, lds + 256 * RW + 1024 + 16);
+        if (stats[i] != -INFINITY)
+            careful_row<T, D, PAGED>(a, b, kh, r0 + i, first_of((r0 + i) / a.group), last_of((r0 + i) / a.group), stats[i],
+                                     stats[32 * RW + i], stats + 64 * RW, stats + 64 * RW + 256);
 }
 
-template <int D, int RW, bool PAGED>
+template <typename T, int D, int RW, bool PAGED>
 int launch_form(const PrefillArgs& a, hipStream_t stream, Err e) {
-    static_assert(Geo<D, RW>::kBytes + kTablePages * 16 <= 160 * 1024 - 256, "LDS of a workgroup");
+    static_assert(Geo<T, D, RW>::kBytes + kTablePages * 16 <= 160 * 1024 - 256, "LDS of a workgroup");
     PrefillArgs args = a;
-    size_t bytes = Geo<D, RW>::kBytes;
+    size_t bytes = Geo<T, D, RW>::kBytes;
     if (PAGED) {
         // pages a workgroup's keys can span: the whole list, or a window and its rows' queries
         int64_t span = (static_cast<int64_t>(a.tk) >> a.log2_page) + 1;
@@ -442,7 +484,7 @@ int launch_form(const PrefillArgs& a, hipStream_t stream, Err e) {
         args.table_pages = span <= kTablePages ? static_cast<int32_t>(span) : 0;
         bytes += static_cast<size_t>(args.table_pages) * 16;
     }
-    const void* fn = reinterpret_cast<const void*>(&attention_prefill_kernel<D, RW, PAGED>);
+    const void* fn = reinterpret_cast<const void*>(&attention_prefill_kernel<T, D, RW, PAGED>);
     if (bytes > 64 * 1024)
         SANDY_HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)), e,
                       "attention launch");
@@ -450,12 +492,12 @@ int launch_form(const PrefillArgs& a, hipStream_t stream, Err e) {
     args.row_blocks = static_cast<int32_t>((rows + 32 * RW - 1) / (32 * RW));
     const int64_t wgs = static_cast<int64_t>(args.row_blocks) * a.batch * a.hkv;
     void* params[] = {&args};
-    SANDY_HIP_TRY(hipLaunchKernel(fn, dim3(static_cast<unsigned>(wgs)), dim3(Geo<D, RW>::THREADS), params, bytes, stream),
+    SANDY_HIP_TRY(hipLaunchKernel(fn, dim3(static_cast<unsigned>(wgs)), dim3(Geo<T, D, RW>::THREADS), params, bytes, stream),
                   e, "attention launch");
     return ok(e);
 }
 
-template <int D, bool PAGED>
+template <typename T, int D, bool PAGED>
 int launch_dim(const PrefillArgs& a, hipStream_t stream, Err e) {
     const int64_t rows = static_cast<int64_t>(a.group) * a.tq;
     const int64_t heads = static_cast<int64_t>(a.batch) * a.hkv;
@@ -463,34 +505,41 @@ int launch_dim(const PrefillArgs& a, hipStream_t stream, Err e) {
     // else 32-row ones (four share them): 1024 workgroups of 64 rows 43 us
     // against 94, 114 of them 37 us against 33 at 32 rows (900 queries, D 256).
     // 128-row workgroups were slower at every size (2048 queries, D 64: 45 us).
+    // f32: 192 workgroups of 64 rows 58 us, 384 of 32 rows 43.
     const int64_t wgs = (rows + 63) / 64 * heads;
-    if (env_int("SANDY_PREFILL_RW", wgs >= 256 ? 2 : 1) == 2) return launch_form<D, 2, PAGED>(a, stream, e);
-    return launch_form<D, 1, PAGED>(a, stream, e);
+    if (env_int("SANDY_PREFILL_RW", wgs >= 256 ? 2 : 1) == 2) return launch_form<T, D, 2, PAGED>(a, stream, e);
+    return launch_form<T, D, 1, PAGED>(a, stream, e);
 }
 
 } // namespace
 
-bool prefill_takes(const PrefillArgs& a, int32_t dtype, int64_t D) {
-    if (dtype != SANDY_BF16 || (D != 64 && D != 128 && D != 256) || a.tq < 2 || a.tk <= 0) return false;
-    // 16-byte q and dense K/V rows, 8-byte output pieces
-    auto aligned = [](const void* p, const int64_t* s, uintptr_t bytes) {
-        return (reinterpret_cast<uintptr_t>(p) & (bytes - 1)) == 0 &&
-               ((s[0] | s[1] | s[2]) & static_cast<int64_t>(bytes / 2 - 1)) == 0;
+bool prefill_takes(const PrefillArgs& a) {
+    const bool f32 = a.dtype == SANDY_F32;
+    const int64_t D = a.dim, es = f32 ? 4 : 2;
+    if ((D != 64 && D != 128 && (D != 256 || f32)) || a.tq < 2 || a.tk <= 0) return false;
+    // 16-byte q and dense K/V rows; output pieces of 4 elements
+    auto aligned = [es](const void* p, const int64_t* s, int64_t bytes) {
+        return (reinterpret_cast<uintptr_t>(p) & static_cast<uintptr_t>(bytes - 1)) == 0 &&
+               ((s[0] | s[1] | s[2]) & (bytes / es - 1)) == 0;
     };
-    if (!aligned(a.q, a.qs, 16) || !aligned(a.out, a.os, 8)) return false;
+    if (!aligned(a.q, a.qs, 16) || !aligned(a.out, a.os, 4 * es)) return false;
     if (!a.k_pages && (!aligned(a.k, a.ks, 16) || !aligned(a.v, a.vs, 16))) return false;
     const int64_t rows = static_cast<int64_t>(a.group) * a.tq;
-    if (a.k_pages && ((a.batch * a.kv_rows_b + a.hkv) << a.log2_page) * D * 2 >= (int64_t{1} << 31)) return false;
+    if (a.k_pages && ((a.batch * a.kv_rows_b + a.hkv) << a.log2_page) * D * es >= (int64_t{1} << 31)) return false;
     return rows < kMaxKeys && (rows + 31) / 32 * a.batch * a.hkv < (int64_t{1} << 31) &&
            env_int("SANDY_PREFILL_GENERAL", 0) == 0;
 }
 
-int launch_prefill(PrefillArgs a, int64_t D, hipStream_t stream, Err e) {
+int launch_prefill(const PrefillArgs& a, hipStream_t stream, Err e) {
     const bool paged = a.k_pages != nullptr;
-    switch (D) {
-        case 64: return paged ? launch_dim<64, true>(a, stream, e) : launch_dim<64, false>(a, stream, e);
-        case 128: return paged ? launch_dim<128, true>(a, stream, e) : launch_dim<128, false>(a, stream, e);
-        default: return paged ? launch_dim<256, true>(a, stream, e) : launch_dim<256, false>(a, stream, e);
+    if (a.dtype == SANDY_F32) {
+        if (a.dim == 64) return paged ? launch_dim<F32, 64, true>(a, stream, e) : launch_dim<F32, 64, false>(a, stream, e);
+        return paged ? launch_dim<F32, 128, true>(a, stream, e) : launch_dim<F32, 128, false>(a, stream, e);
+    }
+    switch (a.dim) {
+        case 64: return paged ? launch_dim<BF16, 64, true>(a, stream, e) : launch_dim<BF16, 64, false>(a, stream, e);
+        case 128: return paged ? launch_dim<BF16, 128, true>(a, stream, e) : launch_dim<BF16, 128, false>(a, stream, e);
+        default: return paged ? launch_dim<BF16, 256, true>(a, stream, e) : launch_dim<BF16, 256, false>(a, stream, e);
     }
 }
 

@@ -14,9 +14,8 @@ recompute.
 
 fp32 throughout, like the reference CPU path (linear, LayerNorm, embedding,
 attention, the GELU group and the lm-head matmul).  The single-token steps
-read their K/V through the device runtime's paged pools (fp32 rows) with the
-general attention kernel, the same arithmetic as the prompt's dense
-attention.  Greedy selection is
+read their K/V through the device runtime's paged pools (fp32 rows); the
+prompt's dense attention runs on f32 MFMA.  Greedy selection is
 sandy_hip_topk with k = 1 (ties -> lowest id, src/server/Sampler.cpp:69-79).
 """
 from __future__ import annotations
