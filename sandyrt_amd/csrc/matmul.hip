@@ -24,7 +24,7 @@
 //         the column tiles alone cannot fill the chip, over workgroups, with
 //         the last-arriving workgroup of each output tile summing the fp32
 //         partials in split order -- one launch, no second reduction pass;
-//       gemm_lines_kernel for larger row counts: 64 x 256 tiles;
+//       gemm_tile_kernel for larger row counts: tiles up to 128 x 192;
 //   - f32 in the same layout runs gemm_ordered_kernel, FMA-free float loops
 //     that keep the reference's k order per output, so f32 results are
 //     bit-identical to the CPU path;
@@ -33,6 +33,7 @@
 #include "gemm.h"
 
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <type_traits>
 
@@ -42,139 +43,210 @@ namespace {
 // decode GEMM workgroups resident at once (two per CU on the 256 CUs)
 constexpr int64_t kWavesResident = 512;
 
-// Prefill-sized products: workgroup = 16 * RT rows x 64 * CT columns of one
-// batch; wave w owns columns n0 = (tile * 4 + w) * 16 * CT .. + 16 * CT.  Per
-// chunk of 64 k the workgroup stages its activation rows once in LDS and
-// each wave its own weight rows, both as whole 128-byte lines (8 rows x 128
-// bytes per load instruction: on gfx950 that streams at about 5.0 TB/s
-// against 3.2 TB/s for MFMA-layout half lines) into tiles whose 16-byte
-// pieces are XOR-swizzled by (row / 2) % 8, so the 128-bit LDS writes and the
-// MFMA-layout 128-bit reads are conflict-free.  Tiles are double buffered:
-// chunk c + 1's loads are in flight while chunk c multiplies.  Loads go
-// through buffer resources whose range checks return zero past the operand's
-// last row; every offset is in the checked vector offset.
-template <int RT, int CT, int OCC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC))) void gemm_lines_kernel(GemmArgs g) {
-    constexpr int kWTile = 16 * CT * 128;
-    constexpr int kXTile = 16 * RT * 128;
-    constexpr int kXPer = (16 * RT * 8 + 255) / 256;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kXTile + 4 * 2 * kWTile];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int ct = static_cast<int>(blockIdx.x);
-    const int64_t r0 = static_cast<int64_t>(blockIdx.y) * 16 * RT;
-    const int64_t bz = blockIdx.z;
+// Prefill-sized products: workgroup tile 64 WM x 64 WN of rows x columns,
+// 2 x 2 waves of 32 WM x 32 WN on v_mfma_f32_32x32x16_bf16; KS such groups of
+// waves take every KS-th chunk of 64 k (their sums added through LDS at the
+// end, in group order).  The weight rows are the A operand, so a lane ends with
+// four consecutive columns of one activation row.  Both operands go global ->
+// registers -> LDS as whole 128-byte lines into XOR-swizzled rows (16-byte
+// piece p of row r at p ^ (r / 2) % 8: conflict-free 128-bit writes and
+// MFMA-layout reads).  While a chunk multiplies, the next moves from registers
+// to the other LDS buffer and the one after is requested, a quarter of each
+// per 16 k, so that the matrix cores never wait for a whole chunk's copies.
+// Bound: LDS and issue slots beside the MFMA (busy 41% at 2048 x 11264 x 2048);
+// see the launch rule for figures.
+template <int WM, int WN, int KS>
+struct TileGeo {
+    static constexpr int BM = 64 * WM, BN = 64 * WN;
+    static constexpr int THREADS = 256 * KS;
+    static constexpr int kX = BM * 128, kW = BN * 128, kGroup = 2 * (kX + kW);
+    static constexpr int XP = BM * 8 / 256, WP = BN * 8 / 256;  // 16-byte pieces a thread stages per chunk
+    static constexpr int kRowPitch = 64 * WN + 16;              // bytes of a wave's output row in LDS
+    static constexpr int kOut = 4 * 32 * WM * kRowPitch;
+    static constexpr int kSums = (KS - 1) * 4 * WM * WN * 64 * 64;
+    static constexpr int kLoop = KS * kGroup;
+    static constexpr int kBytes = kLoop > kOut ? (kLoop > kSums ? kLoop : kSums) : (kOut > kSums ? kOut : kSums);
+};
+
+template <int WM, int WN, int KS>
+__global__ __launch_bounds__(256 * KS, 2) void gemm_tile_kernel(GemmArgs g) {
+    using G_ = TileGeo<WM, WN, KS>;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    typedef float f32x16_t __attribute__((ext_vector_type(16)));
+    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+    const int tid = threadIdx.x & 255, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const int ks = wave >> 2, wm = wave & 1, wn = (wave >> 1) & 1;
+    const int col = lane & 31, half = lane >> 5;
+    // workgroups are dealt round-robin to the 8 XCDs: each XCD takes a run of
+    // neighbouring tiles, rows fastest, so its L2 serves the weight tile to every row tile
+    const int tiles = g.row_tiles * g.col_tiles, per = (tiles + 7) / 8;
+    const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (static_cast<int>(blockIdx.x >> 3) >= per || tile >= tiles) return;
+    const int64_t m0 = static_cast<int64_t>(tile % g.row_tiles) * G_::BM, n0 = static_cast<int64_t>(tile / g.row_tiles) * G_::BN;
     int64_t lo, ro;
-    batch_offsets(g.bm, bz, lo, ro);
+    batch_offsets(g.bm, blockIdx.z, lo, ro);
     const int64_t M = g.M, N = g.N, K = g.K;
-    const int64_t n0 = (static_cast<int64_t>(ct) * 4 + wave) * 16 * CT;
-    const bool wave_live = n0 < N;
-    unsigned char* xt = lds;
-    unsigned char* wt = lds + 2 * kXTile + wave * 2 * kWTile;
-    auto swz = [](int row, int piece) { return row * 128 + ((piece ^ ((row >> 1) & 7)) << 4); };
-    // chunk indices are 32-bit (K <= 2^21): their compares stay on the scalar unit
-    const int ksteps = static_cast<int>(K / 32);
-    const int chunks = (ksteps + 1) / 2;
+    const int chunks = static_cast<int>((K + 63) / 64);
+    unsigned char* mine = lds + ks * G_::kGroup;
 
-    const int64_t wrows = wave_live ? min<int64_t>(16 * CT, N - n0) : 0;
-    const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(g.w + ro + (wave_live ? n0 : 0) * K), 0, static_cast<int>(wrows * K * 2), 0x00020000);
-    const int64_t xrows = min<int64_t>(16 * RT, M - r0);
+    // staging: piece i covers tile row tid / 8 + 32 i, 16-byte piece tid % 8, through
+    // buffer resources over the tile's rows: the lane's offsets stay put, the chunk's is
+    // scalar (no address arithmetic a load), rows past the operand's end read as zero
+    const int prow = tid >> 3, ppc = tid & 7;
+    const int64_t xrows = min<int64_t>(G_::BM, M - m0), wrows = min<int64_t>(G_::BN, N - n0);
     const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(g.a + lo + r0 * K), 0, static_cast<int>(xrows * K * 2), 0x00020000);
-    // weight load i covers tile rows 8i .. 8i + 7 (lane: row 8i + lane/8, piece lane%8)
-    const int wlane = static_cast<int>((lane >> 3) * K * 2 + (lane & 7) * 16);
-    const int wstep = static_cast<int>(8 * K * 2);
-    // tile row 8i + lane/8 swizzles by (4i + lane/16) % 8: one base for even i, one for odd i (+ i * 1024)
-    const int wbase[2] = {swz(lane >> 3, lane & 7), swz(8 + (lane >> 3), lane & 7) - 1024};
-    const bool w_hi = (lane & 7) >= 4;  // this lane's piece lies in the chunk's second k-step
-    int xaddr[kXPer], xoff[kXPer];
-    bool xlive[kXPer], x_hi[kXPer];
+        const_cast<uint16_t*>(g.a + lo + m0 * K), 0, static_cast<int>(xrows * K * 2), 0x00020000);
+    const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(g.w + ro + n0 * K), 0, static_cast<int>(wrows * K * 2), 0x00020000);
+    int xo[G_::XP], wo[G_::WP];
 #pragma unroll
-    for (int q = 0; q < kXPer; q++) {
-        const int p = tid + 256 * q;
-        xlive[q] = p < 16 * RT * 8;
-        const int row = xlive[q] ? p >> 3 : 0;
-        xaddr[q] = swz(row, p & 7);
-        xoff[q] = static_cast<int>(row * K * 2 + (p & 7) * 16);
-        x_hi[q] = (p & 7) >= 4;
-    }
-    int raddr[2][CT], aaddr[2][RT];
+    for (int i = 0; i < G_::XP; i++) xo[i] = static_cast<int>((prow + 32 * i) * K * 2) + 16 * ppc;
 #pragma unroll
-    for (int u = 0; u < 2; u++) {
+    for (int i = 0; i < G_::WP; i++) wo[i] = static_cast<int>((prow + 32 * i) * K * 2) + 16 * ppc;
+    const int put = prow * 128 + ((ppc ^ ((prow >> 1) & 7)) << 4);  // + 4096 i: (prow + 32 i) / 2 % 8 is the same
+    u32x4_t xv[G_::XP], wv[G_::WP];
+    // from the last chunk on, where that is half a chunk (k a multiple of 32, not of
+    // 64): the pieces past K are put out of range and read as zero
+    auto last_half = [&](int c) {
+        if ((K & 63) == 0 || c != chunks - 1 || ppc < 4) return;
 #pragma unroll
-        for (int c = 0; c < CT; c++) raddr[u][c] = swz(16 * c + (lane & 15), 4 * u + (lane >> 4));
+        for (int i = 0; i < G_::XP; i++) xo[i] |= static_cast<int>(0x80000000u);
 #pragma unroll
-        for (int t = 0; t < RT; t++) aaddr[u][t] = swz(16 * t + (lane & 15), 4 * u + (lane >> 4));
-    }
-
-    f32x4_t acc[RT][CT];
-#pragma unroll
-    for (int t = 0; t < RT; t++)
-#pragma unroll
-        for (int c = 0; c < CT; c++) acc[t][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    uint4 wv[2 * CT], xv[kXPer];
-    // the k-tail mask is applied when the registers are written to LDS
-    auto load = [&](int ch) {
-        const int kb = ch * 128;
-#pragma unroll
-        for (int i = 0; i < 2 * CT; i++)
-            wv[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wres, wlane + i * wstep + kb, 0, 0));
-#pragma unroll
-        for (int q = 0; q < kXPer; q++)
-            xv[q] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(xres, xoff[q] + kb, 0, 0));
+        for (int i = 0; i < G_::WP; i++) wo[i] |= static_cast<int>(0x80000000u);
     };
-    auto store = [&](int buf, int ch) {
-        const bool win = 2 * ch + (w_hi ? 1 : 0) < ksteps;
-#pragma unroll
-        for (int i = 0; i < 2 * CT; i++)
-            *reinterpret_cast<uint4*>(wt + buf * kWTile + wbase[i & 1] + i * 1024) = win ? wv[i] : make_uint4(0, 0, 0, 0);
-#pragma unroll
-        for (int q = 0; q < kXPer; q++)
-            if (xlive[q])
-                *reinterpret_cast<uint4*>(xt + buf * kXTile + xaddr[q]) =
-                    2 * ch + (x_hi[q] ? 1 : 0) < ksteps ? xv[q] : make_uint4(0, 0, 0, 0);
+    auto load1 = [&](int c, int i) {
+        if (i < G_::XP)
+            xv[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(xres, xo[i], 128 * c, 0));
+        else
+            wv[i - G_::XP] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(wres, wo[i - G_::XP], 128 * c, 0));
     };
-    auto mma = [&](int buf) {
+    auto store1 = [&](int b, int i) {
+        unsigned char* to = mine + b * (G_::kX + G_::kW) + put;
+        if (i < G_::XP) *reinterpret_cast<u32x4_t*>(to + 4096 * i) = xv[i];
+        else *reinterpret_cast<u32x4_t*>(to + G_::kX + 4096 * (i - G_::XP)) = wv[i - G_::XP];
+    };
+    constexpr int kAll = G_::XP + G_::WP;
+    auto load = [&](int c) {
+        last_half(c);
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
-            uint4 av[RT];
+        for (int i = 0; i < kAll; i++) load1(c, i);
+    };
+    auto store = [&](int b) {
 #pragma unroll
-            for (int t = 0; t < RT; t++) av[t] = *reinterpret_cast<const uint4*>(xt + buf * kXTile + aaddr[u][t]);
+        for (int i = 0; i < kAll; i++) store1(b, i);
+    };
+    f32x16_t acc[WM][WN];
 #pragma unroll
-            for (int c = 0; c < CT; c++) {
-                const uint4 bv = *reinterpret_cast<const uint4*>(wt + buf * kWTile + raddr[u][c]);
+    for (int t = 0; t < WM; t++)
 #pragma unroll
-                for (int t = 0; t < RT; t++)
-                    acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av[t]),
-                                                                        __builtin_bit_cast(bf16x8_t, bv), acc[t][c],
-                                                                        0, 0, 0);
+        for (int c = 0; c < WN; c++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[t][c][i] = 0.0f;
+    const int sw = (col >> 1) & 7;
+    const int rounds = (chunks + KS - 1) / KS;
+    // past the group's last chunk that chunk is repeated: stored and never read
+    const int last = chunks - 1 - (chunks - 1 - ks) % KS;  // this group's last chunk (below ks: none)
+    const int n_mine = ks < chunks ? (last - ks) / KS + 1 : 0;
+    auto nth = [&](int j) -> int { return min(ks + j * KS, max(last, 0)); };
+    load(min(nth(0), chunks - 1));
+    store(0);
+    load(min(nth(1), chunks - 1));
+    __syncthreads();
+    int b = 0;
+    for (int r = 0; r < rounds; r++, b ^= 1) {
+        const unsigned char* xt = mine + b * (G_::kX + G_::kW) + (32 * WM * wm + col) * 128;
+        const unsigned char* wt = mine + b * (G_::kX + G_::kW) + G_::kX + (32 * WN * wn + col) * 128;
+        bf16x8_t xf[2][WM], wf[2][WN];
+        auto frags = [&](int s, int o) {
+            const int at = ((2 * s + half) ^ sw) << 4;  // k 16 s + 8 half .. of a row: piece 2 s + half
+#pragma unroll
+            for (int t = 0; t < WM; t++) xf[o][t] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(xt + 4096 * t + at));
+#pragma unroll
+            for (int q = 0; q < WN; q++) wf[o][q] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(wt + 4096 * q + at));
+        };
+        if (KS == 1 || r < n_mine) {
+            const int next = min(nth(r + 2), chunks - 1);
+            last_half(next);
+            frags(0, 0);
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                if (s < 3) frags(s + 1, (s + 1) & 1);
+#pragma unroll
+                for (int i = kAll * s / 4; i < kAll * (s + 1) / 4; i++) {
+                    store1(b ^ 1, i);
+                    load1(next, i);
+                }
+#pragma unroll
+                for (int q = 0; q < WN; q++)
+#pragma unroll
+                    for (int t = 0; t < WM; t++)
+                        acc[t][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[s & 1][q], xf[s & 1][t], acc[t][q], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
-    };
-    load(0);
-    store(0, 0);
-    __syncthreads();
-    for (int ch = 0; ch < chunks; ch++) {
-        if (ch + 1 < chunks) load(ch + 1);
-        if (wave_live) mma(ch & 1);
-        if (ch + 1 < chunks) store((ch + 1) & 1, ch + 1);
         __syncthreads();
     }
-    if (!wave_live) return;
-    // acc[t][c][i]: row r0 + 16 t + 4 (lane / 16) + i, column n0 + 16 c + lane % 16
-    const int64_t ob = bz * M * N;
+    if constexpr (KS > 1) {
+        float* red = reinterpret_cast<float*>(lds);
+        const int w4 = wave & 3;
+        if (ks > 0) {
 #pragma unroll
-    for (int c = 0; c < CT; c++) {
-        const int64_t nc = n0 + 16 * c + (lane & 15);
-        if (nc >= N) continue;
-        const float bias = g.bias ? bf16_to_f32(g.bias[nc]) : 0.0f;
+            for (int t = 0; t < WM; t++)
 #pragma unroll
-        for (int t = 0; t < RT; t++)
+                for (int c = 0; c < WN; c++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int64_t rr = r0 + 16 * t + 4 * (lane >> 4) + i;
-                if (rr < M) g.out[ob + rr * N + nc] = f32_to_bf16(acc[t][c][i] + bias);  // 2-byte: L2 combines them
-            }
+                    for (int i = 0; i < 16; i++)
+                        red[((((ks - 1) * 4 + w4) * WM * WN + t * WN + c) * 16 + i) * 64 + lane] = acc[t][c][i];
+        }
+        __syncthreads();
+        if (ks == 0) {
+#pragma unroll
+            for (int q = 0; q < KS - 1; q++)
+#pragma unroll
+                for (int t = 0; t < WM; t++)
+#pragma unroll
+                    for (int c = 0; c < WN; c++)
+#pragma unroll
+                        for (int i = 0; i < 16; i++)
+                            acc[t][c][i] += red[(((q * 4 + w4) * WM * WN + t * WN + c) * 16 + i) * 64 + lane];
+        }
+        __syncthreads();
+        if (ks > 0) return;
+    }
+    // acc[t][c][i]: row 32 t + col, column 32 c + 8 (i / 4) + 4 half + i % 4 of the wave's part:
+    // through LDS (wave-private) into whole row segments
+    unsigned char* ot = lds + (wave & 3) * 32 * WM * G_::kRowPitch;
+    const int64_t mw = m0 + 32 * WM * wm, nw = n0 + 32 * WN * wn;
+#pragma unroll
+    for (int c = 0; c < WN; c++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            float bias[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (g.bias)
+#pragma unroll
+                for (int x = 0; x < 4; x++) bias[x] = bf16_to_f32(g.bias[min<int64_t>(nw + 32 * c + 8 * q + 4 * half + x, N - 1)]);
+#pragma unroll
+            for (int t = 0; t < WM; t++)
+                *reinterpret_cast<uint2*>(ot + (32 * t + col) * G_::kRowPitch + 2 * (32 * c + 8 * q + 4 * half)) =
+                    make_uint2(pack_bf16x2(acc[t][c][4 * q] + bias[0], acc[t][c][4 * q + 1] + bias[1]),
+                               pack_bf16x2(acc[t][c][4 * q + 2] + bias[2], acc[t][c][4 * q + 3] + bias[3]));
+        }
+    __builtin_amdgcn_wave_barrier();
+    uint16_t* out = g.out + static_cast<int64_t>(blockIdx.z) * M * N;
+    constexpr int kLanes = 4 * WN;  // lanes per row, 8 columns each
+    const bool wide = (N & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+#pragma unroll
+    for (int i = 0; i < 32 * WM * kLanes / 64; i++) {
+        const int r = (64 * i + lane) / kLanes, c8 = 8 * ((64 * i + lane) % kLanes);
+        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ot + r * G_::kRowPitch + 2 * c8);
+        if (mw + r >= M || nw + c8 >= N) continue;
+        uint16_t* to = out + (mw + r) * N + nw + c8;
+        if (wide) {
+            *reinterpret_cast<u32x4_t*>(to) = v;
+        } else {
+            for (int x = 0; x < 8 && nw + c8 + x < N; x++) to[x] = static_cast<uint16_t>(v[x >> 1] >> (16 * (x & 1)));
+        }
     }
 }
 
@@ -646,8 +718,6 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
         SANDY_HIP_TRY(hipGetLastError(), e, what);
         return ok(e);
     } else if (lines) {
-        // 64 x 256 tiles for prefill-sized products (the K loop is rolled and
-        // the grid never splits K)
         GemmArgs g{};
         g.a = static_cast<const uint16_t*>(pl);
         g.w = static_cast<const uint16_t*>(pr);
@@ -657,17 +727,58 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
         g.N = p.N;
         g.K = p.K;
         g.bm = p.bm;
-        const int64_t row_tiles = (p.M + 63) / 64;
-        const int64_t col_tiles = (p.N + 255) / 256;
-        if (row_tiles > 65535 || col_tiles > 0x7fffffff)
-            return fail(e, SANDY_ERR_UNSUPPORTED, "%s shape exceeds the launch grid", what);
-        g.col_tiles = static_cast<int32_t>(col_tiles);
-        g.row_tiles = static_cast<int32_t>(row_tiles);
-        g.splits = 1;
-        g.split_chunks = static_cast<int32_t>((p.K / 32 + 1) / 2);
-        const dim3 grid(static_cast<unsigned>(col_tiles), static_cast<unsigned>(row_tiles),
-                        static_cast<unsigned>(p.batches));
-        hipLaunchKernelGGL((gemm_lines_kernel<4, 4, 2>), grid, dim3(256), 0, stream, g);
+        // The tile form with the least estimated time: its chunks of 64 k (over its
+        // KS groups) times the time of one, `alone` up to one workgroup a CU, else
+        // `each` for every workgroup of the fullest CU (measured, us).  Cold
+        // operands, 64 x 256 tiles before -> the form taken (us): 2048 x 11264 x
+        // 2048 163 -> 99 (128 x 192 tiles, 960 TFLOP/s), 2040 x 2048 x 5632 -> 57
+        // (128 x 128, two K groups), 2048 x 2048 x 2048 39 -> 24 (128 x 64), 1000 x
+        // 2048 x 5632 93 -> 33 (128 x 64, two groups), 333 x 2048 x 5632 93 -> 22
+        // (64 x 64, two groups), 100 x 520 x 224 9.0 -> 4.2 (the same).
+        struct Form {
+            int bm, bn, groups;
+            double alone, each;
+        };
+        static const Form kForms[] = {{128, 192, 1, 0.75, 0.78}, {128, 64, 1, 0.41, 0.36}, {128, 128, 2, 1.2, 1.4},
+                                      {128, 64, 2, 0.72, 0.8}, {64, 64, 2, 0.5, 0.5}};
+        const int64_t chunks = (p.K + 63) / 64;
+        int form = 0;
+        double best = 0.0;
+        for (int i = 0; i < 5; i++) {
+            const Form& f = kForms[i];
+            const double tiles = static_cast<double>((p.M + f.bm - 1) / f.bm) * static_cast<double>((p.N + f.bn - 1) / f.bn) *
+                                 static_cast<double>(p.batches);
+            const double us = static_cast<double>((chunks + f.groups - 1) / f.groups) *
+                              (tiles <= 256.0 ? f.alone : std::ceil(tiles / 256.0) * f.each);
+            if (i == 0 || us < best) {
+                best = us;
+                form = i;
+            }
+        }
+        form = env_int("SANDY_GEMM_FORM", form);
+        auto go = [&](auto geo, auto kernel) -> int {
+            using G_ = decltype(geo);
+            const int64_t rt = (p.M + G_::BM - 1) / G_::BM, ct = (p.N + G_::BN - 1) / G_::BN;
+            if (rt > 0x7fffffff || ct > 0x7fffffff || rt * ct > 0x7ffffff0)
+                return fail(e, SANDY_ERR_UNSUPPORTED, "%s shape exceeds the launch grid", what);
+            g.row_tiles = static_cast<int32_t>(rt);
+            g.col_tiles = static_cast<int32_t>(ct);
+            if (G_::kBytes > 64 * 1024)
+                SANDY_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, G_::kBytes), e, what);
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((rt * ct + 7) / 8 * 8), 1, static_cast<unsigned>(p.batches)),
+                               dim3(G_::THREADS), G_::kBytes, stream, g);
+            return SANDY_OK;
+        };
+        int st = SANDY_OK;
+        switch (form) {
+            case 0: st = go(TileGeo<2, 3, 1>{}, gemm_tile_kernel<2, 3, 1>); break;
+            case 1: st = go(TileGeo<2, 1, 1>{}, gemm_tile_kernel<2, 1, 1>); break;
+            case 2: st = go(TileGeo<2, 2, 2>{}, gemm_tile_kernel<2, 2, 2>); break;
+            case 3: st = go(TileGeo<2, 1, 2>{}, gemm_tile_kernel<2, 1, 2>); break;
+            default: st = go(TileGeo<1, 1, 2>{}, gemm_tile_kernel<1, 1, 2>); break;
+        }
+        if (st) return st;
     } else {
         const int64_t gy = (p.M + 63) / 64, gx = (p.N + 63) / 64;
         if (gy > 65535 || gx > 0x7fffffff) return fail(e, SANDY_ERR_UNSUPPORTED, "%s shape exceeds the launch grid", what);

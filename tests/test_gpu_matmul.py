@@ -239,6 +239,30 @@ def test_linear_f32_ordered_tiles_bit_exact(ops, oracle, rows_a_lane, rows, in_f
     assert_equal(got3, oracle.matmul(to_oracle(x3), to_oracle(w.unsqueeze(0)), transpose_rhs=True), "batched matmul")
 
 
+@pytest.mark.parametrize("form", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("m,n,k", [(65, 8, 32), (70, 301, 64), (129, 194, 96), (192, 65, 160), (257, 200, 2080)])
+def test_matmul_bf16_prefill_tiles(ops, oracle, form, m, n, k):
+    """Every tile form of the prefill GEMM: ragged rows and columns (odd n:
+    narrow stores), one chunk of k, half chunks at the end, chunk counts that
+    do not divide by the wave groups, a weight shared by a batch, bias, and an
+    output that is only element aligned."""
+    r = rng(m + n + k)
+    x = from_f32(normal(r, (m, k)), torch.bfloat16)
+    x2 = from_f32(normal(r, (2, m, k)), torch.bfloat16)
+    w = from_f32(normal(r, (n, k), 0.05), torch.bfloat16)
+    b = from_f32(normal(r, (n,)), torch.bfloat16)
+    guard = torch.full((m * n + 16,), 7.0, dtype=torch.bfloat16, device="cuda")
+    with env(SANDY_GEMM_FORM=form):
+        got = ops.linear(x, w, b)
+        ops.matmul(x, w, transpose_rhs=True, out=guard[3:3 + m * n].view(m, n))
+        got2 = ops.matmul(x2, w.unsqueeze(0), transpose_rhs=True)
+    want = oracle.matmul(to_oracle(x), to_oracle(w), transpose_rhs=True)
+    assert_close(got, oracle.linear(to_oracle(x), to_oracle(w), to_oracle(b)), torch.bfloat16, "linear")
+    assert_close(guard[3:3 + m * n].view(m, n), want, torch.bfloat16, "unaligned out")
+    assert guard[:3].eq(7).all() and guard[3 + m * n:].eq(7).all()
+    assert_close(got2, oracle.matmul(to_oracle(x2), to_oracle(w.unsqueeze(0)), transpose_rhs=True), torch.bfloat16, "batched")
+
+
 @pytest.mark.parametrize("act", ["silu", "gelu"])
 @pytest.mark.parametrize("m,k,ffn", [(1, 2048, 5632), (5, 64, 80), (32, 2048, 5632), (64, 2560, 1024),
                                      (32, 5632, 96), (3, 128, 40)])
