@@ -1212,6 +1212,167 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
     }
 }
 
+// The same product for few routes (decode batches): a pure weight stream, and
+// only the experts that got a row stream anything -- one workgroup per (expert,
+// tile) of all experts, each with one chunk in flight, spent 50 us on 140 MB
+// (and idle workgroups, 2 us each for their offsets, most of a short launch).
+// Workgroup = (one of the experts with rows, columns); its waves run on their
+// own -- no barrier in the loop -- with Q chunks of whole 128-byte lines in
+// flight, through wave-private swizzled LDS tiles.  KW = 1: each wave owns 16 CT
+// columns; KW = 4: the waves own the same columns and every fourth chunk, their
+// sums meeting in wave order.  Rows past the expert's own read as zero without
+// memory traffic.
+template <int CT, int KW, int Q>
+__global__ __launch_bounds__(256, 2) void moe_gemm_stream_kernel(
+        const uint16_t* __restrict__ x, const void* __restrict__ offs, int32_t off_dt, const uint16_t* __restrict__ w,
+        uint16_t* __restrict__ out, int64_t rows, int64_t K, int64_t M, int64_t experts, int64_t slots, uint32_t* errw) {
+    constexpr int RT = 1;
+    constexpr int kWTile = 16 * CT * 128, kXTile = 16 * RT * 128;
+    constexpr int kWave = kWTile + kXTile;
+    constexpr int kSums = (KW - 1) * RT * CT * 64 * 16;  // the other waves' accumulators
+    __shared__ __attribute__((aligned(16))) unsigned char lds[4 * kWave > kSums ? 4 * kWave : kSums];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t b = blockIdx.x / slots, n0 = (KW == 1 ? static_cast<int64_t>(blockIdx.y) * 4 + wave : static_cast<int64_t>(blockIdx.y)) * 16 * CT;
+    // the expert: the (blockIdx.x % slots)-th that has rows, found by every wave
+    // from the offsets, 128 at a time
+    int64_t e = -1, begin = 0, end = 0;
+    int want = static_cast<int>(blockIdx.x % slots);
+    bool bad = false;
+    const bool check = want == 0 && blockIdx.y == 0;  // scans every expert's offsets
+    for (int64_t e0 = 0; e0 < experts && (e < 0 || check); e0 += 128) {
+        int64_t lo[2], hi[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int64_t at = b * (experts + 1) + min<int64_t>(e0 + 64 * h + lane, experts - 1);
+            lo[h] = load_index(offs, off_dt, at);
+            hi[h] = load_index(offs, off_dt, at + 1);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const bool in = e0 + 64 * h + lane < experts;
+            const bool valid = lo[h] >= 0 && hi[h] >= lo[h] && hi[h] <= rows;
+            bad = bad || (in && !valid);
+            const uint64_t mask = __ballot(in && valid && hi[h] > lo[h]);
+            const int count = __popcll(mask);
+            if (e < 0 && want < count) {
+                const int rank = __popcll(mask & ((1ull << lane) - 1));
+                const int src = __ffsll(static_cast<unsigned long long>(__ballot(((mask >> lane) & 1) && rank == want))) - 1;
+                e = e0 + 64 * h + src;
+                begin = __shfl(lo[h], src, 64);
+                end = __shfl(hi[h], src, 64);
+            }
+            want -= count;
+        }
+    }
+    if (bad) atomicOr(errw, static_cast<uint32_t>(SANDY_DEVERR_OFFSETS));
+    if (e < 0) return;
+    e = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(e)));
+    begin = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(begin)));
+    end = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(end)));
+    unsigned char* wt = lds + wave * kWave;
+    unsigned char* xt = wt + kWTile;
+    auto swz = [](int row, int piece) { return row * 128 + ((piece ^ ((row >> 1) & 7)) << 4); };
+    const int ksteps = static_cast<int>(K / 32), chunks = (ksteps + 1) / 2;
+    const int kw = KW == 1 ? 0 : wave;
+    const int n = kw < chunks ? (chunks - kw + KW - 1) / KW : 0;  // this wave's chunks: kw, kw + KW, ...
+    const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(w + (e * M + min<int64_t>(n0, M - 1)) * K), 0, static_cast<int>(max<int64_t>(0, min<int64_t>(16 * CT, M - n0)) * K * 2), 0x00020000);
+    // load i covers tile rows 8 i .. 8 i + 7 (lane: row 8 i + lane / 8, piece lane % 8)
+    const int at = static_cast<int>((lane >> 3) * K * 2 + (lane & 7) * 16), step = static_cast<int>(8 * K * 2);
+    const int base[2] = {swz(lane >> 3, lane & 7), swz(8 + (lane >> 3), lane & 7) - 1024};
+    int faddr[2];  // fragment of tile 0, k-step u: row lane % 16, piece 4 u + lane / 16
+#pragma unroll
+    for (int u = 0; u < 2; u++) faddr[u] = swz(lane & 15, 4 * u + (lane >> 4));
+    for (int64_t r0 = begin; r0 < end; r0 += 16 * RT) {
+        const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint16_t*>(x + (b * rows + r0) * K), 0, static_cast<int>(min<int64_t>(end - r0, 16 * RT) * K * 2),
+            0x00020000);
+        f32x4_t acc[RT][CT];
+#pragma unroll
+        for (int t = 0; t < RT; t++)
+#pragma unroll
+            for (int c = 0; c < CT; c++) acc[t][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        uint4 wv[Q][2 * CT], xv[Q][2 * RT];
+        // every load unconditional, so the wait counts stay exact: past the wave's
+        // last chunk that chunk again (cached, not multiplied)
+        auto load = [&](int j, int slot) {
+            const int kb = (kw + KW * max(0, min(j, n - 1))) * 128;
+#pragma unroll
+            for (int i = 0; i < 2 * CT; i++)
+                wv[slot][i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wres, at + i * step, kb, 2));
+#pragma unroll
+            for (int i = 0; i < 2 * RT; i++)
+                xv[slot][i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(xres, at + i * step, kb, 0));
+        };
+#pragma unroll
+        for (int q = 0; q < Q; q++) load(q, q);
+        for (int j0 = 0; j0 < n; j0 += Q) {
+#pragma unroll
+            for (int q = 0; q < Q; q++) {
+                // a wave's LDS operations complete in order: the reads of the chunk
+                // before are done before these writes land
+#pragma unroll
+                for (int i = 0; i < 2 * CT; i++) *reinterpret_cast<uint4*>(wt + base[i & 1] + i * 1024) = wv[q][i];
+#pragma unroll
+                for (int i = 0; i < 2 * RT; i++) *reinterpret_cast<uint4*>(xt + base[i & 1] + i * 1024) = xv[q][i];
+                load(j0 + q + Q, q);
+                __builtin_amdgcn_wave_barrier();
+                // uniform: a chunk past the wave's last is not multiplied, nor the second
+                // k-step of a half chunk (its registers lie past K)
+                const int left = j0 + q < n ? ksteps - 2 * (kw + KW * (j0 + q)) : 0;
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    if (u >= left) break;
+                    uint4 av[RT];
+#pragma unroll
+                    for (int t = 0; t < RT; t++) av[t] = *reinterpret_cast<const uint4*>(xt + faddr[u] + 2048 * t);
+#pragma unroll
+                    for (int c = 0; c < CT; c++) {
+                        const uint4 bv = *reinterpret_cast<const uint4*>(wt + faddr[u] + 2048 * c);
+#pragma unroll
+                        for (int t = 0; t < RT; t++)
+                            acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av[t]),
+                                                                                __builtin_bit_cast(bf16x8_t, bv),
+                                                                                acc[t][c], 0, 0, 0);
+                    }
+                }
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+        if constexpr (KW > 1) {
+            __syncthreads();
+            f32x4_t* red = reinterpret_cast<f32x4_t*>(lds);
+            if (wave > 0) {
+#pragma unroll
+                for (int t = 0; t < RT; t++)
+#pragma unroll
+                    for (int c = 0; c < CT; c++) red[((wave - 1) * RT * CT + t * CT + c) * 64 + lane] = acc[t][c];
+            }
+            __syncthreads();
+            if (wave == 0) {
+#pragma unroll
+                for (int q = 0; q < KW - 1; q++)
+#pragma unroll
+                    for (int t = 0; t < RT; t++)
+#pragma unroll
+                        for (int c = 0; c < CT; c++) acc[t][c] += red[(q * RT * CT + t * CT + c) * 64 + lane];
+            }
+            __syncthreads();  // the next rows reuse the LDS
+        }
+        if (KW == 1 || wave == 0) {
+#pragma unroll
+            for (int t = 0; t < RT; t++)
+#pragma unroll
+                for (int c = 0; c < CT; c++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const int64_t rr = r0 + 16 * t + 4 * (lane >> 4) + i, nc = n0 + 16 * c + (lane & 15);
+                        if (rr < end && nc < M) out[(b * rows + rr) * M + nc] = f32_to_bf16(acc[t][c][i]);
+                    }
+        }
+    }
+}
+
 // Any dtype / layout: one thread per (row, column), float accumulation in k
 // order like the reference.
 template <typename T>
@@ -1542,16 +1703,35 @@ extern "C" int sandy_hip_moe_matmul(const SandyTensor* x, const SandyTensor* exp
         const auto* pw = static_cast<const uint16_t*>(base_ptr(*weight));
         auto* po = static_cast<uint16_t*>(base_ptr(*out));
         const void* po_ = base_ptr(*expert_offsets);
-        // tile: 16 rows x 32 columns per wave for decode-sized batches, otherwise
-        // 64 rows x the column tile of moe_column_tile
+        // tile: 16 rows x 32 columns per wave for decode-sized batches, 32 rows where
+        // many experts have more than 16 (each further pass streams the weights
+        // again: gate / down at 9 rows an expert 120 / 98 us -> 78 / 84, at 16
+        // 131 / 145 -> 79 / 90; at 6 the 16-row tile, 76 / 81 against 77 / 82),
+        // otherwise 64 rows x the column tile of moe_column_tile
         const int col_tile = avg <= 16 ? 2 : moe_column_tile(M, batch * experts);
-        const int variant = env_int("SANDY_MOE_GEMM", avg <= 16 ? 0 : col_tile == 3 ? 5 : col_tile == 2 ? 2 : 1);
+        const int variant = env_int("SANDY_MOE_GEMM", avg <= 6 ? 0 : avg <= 16 ? 4 : col_tile == 3 ? 5 : col_tile == 2 ? 2 : 1);
         auto grid_for = [&](int ct) {
             return dim3(static_cast<unsigned>(batch * experts), static_cast<unsigned>((M + 64 * ct - 1) / (64 * ct)));
         };
 #define LINES_LAUNCH(RT, CT)                                                                                        \
     hipLaunchKernelGGL((moe_gemm_lines_kernel<RT, CT>), grid_for(CT), dim3(256), 0, stream, px, po_,               \
                        expert_offsets->dtype, pw, po, rows, K, M, experts, batch, errw)
+        // fewer routes than half the experts: only the experts with rows stream
+        // (gate / down of the 128-expert block, us, one chunk in flight -> here: 8
+        // rows 46 / 19 -> 10 / 9, 40 rows 50 / 42 -> 28 / 30, 64 rows 52 / 47 ->
+        // 40 / 44; 96 rows 55 / 56 against 61 / 62).  Up to 16 rows a long
+        // contraction is split over the waves (8 rows 18 -> 10; 40 rows 28 -> 31)
+        const int stream_form = env_int("SANDY_MOE_STREAM", rows * 2 > experts ? 0 : rows <= 16 && K >= 1536 ? 2 : 1);
+        if (stream_form) {
+            const int64_t slots = std::min(rows, experts);  // at most `rows` experts have a row
+            const int64_t cols = stream_form == 2 ? 32 : 64;
+            const dim3 grid(static_cast<unsigned>(batch * slots), static_cast<unsigned>((M + cols - 1) / cols));
+            hipLaunchKernelGGL((stream_form == 2 ? moe_gemm_stream_kernel<2, 4, 4> : moe_gemm_stream_kernel<1, 1, 4>), grid,
+                               dim3(256), 0, stream, px, po_, expert_offsets->dtype, pw, po, rows, K, M, experts, slots,
+                               errw);
+            SANDY_HIP_TRY(hipGetLastError(), e, "moe_matmul launch");
+            return ok(e);
+        }
         switch (variant) {
             case 0: LINES_LAUNCH(1, 2); break;
             case 2: LINES_LAUNCH(4, 2); break;

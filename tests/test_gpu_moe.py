@@ -273,6 +273,43 @@ def test_moe_matmul_config5(ops, oracle, shape):
         assert_close(got[lo:hi], to_oracle(ref), torch.bfloat16, f"expert {e} vs torch fp32")
 
 
+@pytest.mark.parametrize("form", ["1", "2"])
+@pytest.mark.parametrize("counts,M,K", [
+    ([0, 1, 0, 17, 0, 0, 2], 70, 32),                 # one half chunk; an expert of two row passes
+    ([0] * 130 + [3] + [0] * 60 + [1, 0], 33, 96),    # experts past the first scan of 128; three half chunks
+    ([1, 1, 1, 1, 1], 128, 1600),                     # every route its own expert; 25 chunks over the waves
+    ([40], 65, 2048),
+])
+def test_moe_matmul_few_routes(ops, oracle, monkeypatch, form, counts, M, K):
+    """The weight-streaming form (only experts with rows get workgroups): rows
+    over columns and over the waves' share of k, batched."""
+    monkeypatch.setenv("SANDY_MOE_STREAM", form)
+    r = rng(len(counts) + M + K)
+    E, rows = len(counts), int(np.sum(counts))
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.int64)
+    rev = np.concatenate([[0], np.cumsum(counts[::-1])]).astype(np.int64)
+    x = from_f32(normal(r, (2, rows, K)), torch.bfloat16)
+    w = from_f32(normal(r, (E, M, K), 0.1), torch.bfloat16)
+    offs = np.stack([off, rev])
+    got = ops.moe_matmul(x, torch.from_numpy(offs).cuda(), w, True)
+    ops.check_device_errors()
+    assert_close(got, oracle.moe_matmul(to_oracle(x), offs, to_oracle(w), True), torch.bfloat16, "moe_matmul")
+
+
+@pytest.mark.parametrize("form", ["1", "2"])
+def test_moe_matmul_few_routes_bad_offsets(ops, monkeypatch, form):
+    """An invalid offset past every expert with rows is still recorded."""
+    from sandyrt_amd._lib import SandyError
+    monkeypatch.setenv("SANDY_MOE_STREAM", form)
+    x = torch.zeros(1, 32, dtype=torch.bfloat16, device="cuda")
+    w = torch.zeros(200, 16, 32, dtype=torch.bfloat16, device="cuda")
+    offs = torch.ones(201, dtype=torch.int64, device="cuda")
+    offs[0], offs[190] = 0, -1
+    ops.moe_matmul(x, offs, w, True)
+    with pytest.raises(SandyError, match="moe_matmul invalid expert offsets"):
+        ops.check_device_errors()
+
+
 def test_moe_matmul_bad_offsets_sets_device_error(ops):
     from sandyrt_amd._lib import SandyError
     x = torch.zeros(4, 32, dtype=torch.bfloat16, device="cuda")
