@@ -26,8 +26,8 @@
 // fit, one barrier each.
 // Bound: softmax VALU work (49% of the cycles at D 64, MFMA 22%).  Measured,
 // us a call (general kernel -> here): 2048 queries, 32 / 4 heads, D 64
-// 14357 -> 44; 777 queries after 1500 keys, window 1024, 8 / 2 heads, D 256,
-// pages of 16: 4896 -> 46; 1500 after 300, 16 / 2 heads, D 128: 54; f32, 12
+// 14357 -> 43; 777 queries after 1500 keys, window 1024, 8 / 2 heads, D 256,
+// pages of 16: 4896 -> 41; 1500 after 300, 16 / 2 heads, D 128: 49; f32, 12
 // heads, D 64: 1000 queries 1434 -> 43, 64 queries 23.5 -> 9.8.
 #include "attention_prefill.h"
 
@@ -207,50 +207,45 @@ __global__ __launch_bounds__((Geo<T, D, RW>::THREADS), (Geo<T, D, RW>::kF32 && D
     // rows past the last key repeat it (they are masked)
     auto key_of = [&](int c0, int i) -> int { return min(c0 + prow + i * kRowStep, k_end - 1); };
     // the page addresses of the workgroup's keys, staged in LDS once where they
-    // fit: read from memory per chunk they put a dependent load before each of
-    // the chunk's (D 256: 4.4 us a chunk against 2.4 us)
-    uint64_t* tab = reinterpret_cast<uint64_t*>(lds + G_::kBytes);
+    // fit (read from memory per chunk they put a dependent load before each of
+    // the chunk's: 777 queries, D 256, 74 us a call against 59) and checked
+    // there instead of per piece (46 us against 41)
+    u32x4_t* tab = reinterpret_cast<u32x4_t*>(lds + G_::kBytes);
     const int page0 = PAGED ? k_begin >> a.log2_page : 0;
+    const int page_mask = (1 << a.log2_page) - 1;
+    bool staged = false;
     if (PAGED && a.table_pages > 0) {
         const int n = k_begin < k_end ? min(((k_end - 1) >> a.log2_page) - page0 + 1, a.table_pages) : 0;
+        bool plain = true;  // there and 16-byte aligned
         for (int i = tid; i < n; i += G_::THREADS) {
-            tab[2 * i] = a.k_pages[page0 + i];
-            tab[2 * i + 1] = a.v_pages[page0 + i];
+            const uint64_t kp = a.k_pages[page0 + i], vp = a.v_pages[page0 + i];
+            plain = plain && kp != 0 && vp != 0 && ((kp | vp) & 15) == 0;
+            tab[i] = u32x4_t{static_cast<uint32_t>(kp), static_cast<uint32_t>(kp >> 32), static_cast<uint32_t>(vp),
+                             static_cast<uint32_t>(vp >> 32)};
         }
-        __syncthreads();
+        staged = __syncthreads_and(plain);
     }
     auto load = [&](int c0) {
         if constexpr (PAGED) {
-            uint64_t kat[NP], vat[NP];
-            bool plain = true;  // every page there and 16-byte aligned
-#pragma unroll
-            for (int i = 0; i < NP; i++) {
-                const int key = key_of(c0, i), page = key >> a.log2_page;
-                if (a.table_pages > 0) {
-                    kat[i] = tab[2 * (page - page0)];
-                    vat[i] = tab[2 * (page - page0) + 1];
-                } else {
-                    kat[i] = a.k_pages[page];
-                    vat[i] = a.v_pages[page];
-                }
-                // byte offset of the row within the page: below 2^31 (checked on the host)
-                const uint32_t off = ((page_row << a.log2_page) + (key & ((1 << a.log2_page) - 1))) * (ES * D) + 16 * ppc;
-                plain = plain && kat[i] != 0 && vat[i] != 0 && ((kat[i] | vat[i]) & 15) == 0;
-                kat[i] = kat[i] ? (kat[i] & ~uint64_t{ES - 1}) + off : 0;
-                vat[i] = vat[i] ? (vat[i] & ~uint64_t{ES - 1}) + off : 0;
-            }
-            if (__all(plain)) {
+            if (staged) {
 #pragma unroll
                 for (int i = 0; i < NP; i++) {
-                    kr[i] = *reinterpret_cast<const u32x4_t*>(kat[i]);
-                    vr[i] = *reinterpret_cast<const u32x4_t*>(vat[i]);
+                    const int key = key_of(c0, i);
+                    const u32x4_t at = tab[(key >> a.log2_page) - page0];
+                    // byte offset of the row within the page: below 2^31 (checked on the host)
+                    const uint32_t off = ((page_row << a.log2_page) + (key & page_mask)) * (ES * D) + 16 * ppc;
+                    kr[i] = *reinterpret_cast<const u32x4_t*>((static_cast<uint64_t>(at[1]) << 32 | at[0]) + off);
+                    vr[i] = *reinterpret_cast<const u32x4_t*>((static_cast<uint64_t>(at[3]) << 32 | at[2]) + off);
                 }
             } else {
 #pragma unroll
                 for (int i = 0; i < NP; i++) {
-                    pages_ok = pages_ok && kat[i] && vat[i];
-                    kr[i] = kat[i] ? load_piece(kat[i]) : u32x4_t{0, 0, 0, 0};
-                    vr[i] = vat[i] ? load_piece(vat[i]) : u32x4_t{0, 0, 0, 0};
+                    const int key = key_of(c0, i);
+                    const uint64_t kp = a.k_pages[key >> a.log2_page], vp = a.v_pages[key >> a.log2_page];
+                    pages_ok = pages_ok && kp != 0 && vp != 0;
+                    kr[i] = vr[i] = u32x4_t{0, 0, 0, 0};
+                    if (kp) kr[i] = load_piece(paged_row(kp, key, a.log2_page, page_row, ES * D, ES) + 16 * ppc);
+                    if (vp) vr[i] = load_piece(paged_row(vp, key, a.log2_page, page_row, ES * D, ES) + 16 * ppc);
                 }
             }
         } else {
@@ -501,13 +496,14 @@ template <typename T, int D, bool PAGED>
 int launch_dim(const PrefillArgs& a, hipStream_t stream, Err e) {
     const int64_t rows = static_cast<int64_t>(a.group) * a.tq;
     const int64_t heads = static_cast<int64_t>(a.batch) * a.hkv;
-    // 64-row workgroups (two waves share the keys) where they fill the 256 CUs,
-    // else 32-row ones (four share them): 1024 workgroups of 64 rows 43 us
-    // against 94, 114 of them 37 us against 33 at 32 rows (900 queries, D 256).
+    // 64-row workgroups (two waves share the keys) where they nearly fill the 256
+    // CUs, else 32-row ones (four share them): 1024 workgroups of 64 rows 43 us
+    // against 94, 252 of them 11.5 against 13.4, 114 of them 36 against 32 (900
+    // queries, D 256).
     // 128-row workgroups were slower at every size (2048 queries, D 64: 45 us).
     // f32: 192 workgroups of 64 rows 58 us, 384 of 32 rows 43.
     const int64_t wgs = (rows + 63) / 64 * heads;
-    if (env_int("SANDY_PREFILL_RW", wgs >= 256 ? 2 : 1) == 2) return launch_form<T, D, 2, PAGED>(a, stream, e);
+    if (env_int("SANDY_PREFILL_RW", wgs >= 224 ? 2 : 1) == 2) return launch_form<T, D, 2, PAGED>(a, stream, e);
     return launch_form<T, D, 1, PAGED>(a, stream, e);
 }
 
