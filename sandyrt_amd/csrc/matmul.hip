@@ -31,6 +31,7 @@
 //   - gemm_simt_kernel: every other case (other layouts, unaligned shapes),
 //     register-tiled, in the same order.
 #include "gemm.h"
+#include "gemm_tile.h"
 
 #include <algorithm>
 #include <cmath>
@@ -43,41 +44,11 @@ namespace {
 // decode GEMM workgroups resident at once (two per CU on the 256 CUs)
 constexpr int64_t kWavesResident = 512;
 
-// Prefill-sized products: workgroup tile 64 WM x 64 WN of rows x columns,
-// 2 x 2 waves of 32 WM x 32 WN on v_mfma_f32_32x32x16_bf16; KS such groups of
-// waves take every KS-th chunk of 64 k (their sums added through LDS at the
-// end, in group order).  The weight rows are the A operand, so a lane ends with
-// four consecutive columns of one activation row.  Both operands go global ->
-// registers -> LDS as whole 128-byte lines into XOR-swizzled rows (16-byte
-// piece p of row r at p ^ (r / 2) % 8: conflict-free 128-bit writes and
-// MFMA-layout reads).  While a chunk multiplies, the next moves from registers
-// to the other LDS buffer and the one after is requested, a quarter of each
-// per 16 k, so that the matrix cores never wait for a whole chunk's copies.
-// Bound: LDS and issue slots beside the MFMA (busy 41% at 2048 x 11264 x 2048);
-// see the launch rule for figures.
-template <int WM, int WN, int KS>
-struct TileGeo {
-    static constexpr int BM = 64 * WM, BN = 64 * WN;
-    static constexpr int THREADS = 256 * KS;
-    static constexpr int kX = BM * 128, kW = BN * 128, kGroup = 2 * (kX + kW);
-    static constexpr int XP = BM * 8 / 256, WP = BN * 8 / 256;  // 16-byte pieces a thread stages per chunk
-    static constexpr int kRowPitch = 64 * WN + 16;              // bytes of a wave's output row in LDS
-    static constexpr int kOut = 4 * 32 * WM * kRowPitch;
-    static constexpr int kSums = (KS - 1) * 4 * WM * WN * 64 * 64;
-    static constexpr int kLoop = KS * kGroup;
-    static constexpr int kBytes = kLoop > kOut ? (kLoop > kSums ? kLoop : kSums) : (kOut > kSums ? kOut : kSums);
-};
-
+// The tile of gemm_tile.h over a dense product.
 template <int WM, int WN, int KS>
 __global__ __launch_bounds__(256 * KS, 2) void gemm_tile_kernel(GemmArgs g) {
     using G_ = TileGeo<WM, WN, KS>;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    typedef float f32x16_t __attribute__((ext_vector_type(16)));
-    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-    const int tid = threadIdx.x & 255, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-    const int ks = wave >> 2, wm = wave & 1, wn = (wave >> 1) & 1;
-    const int col = lane & 31, half = lane >> 5;
     // workgroups are dealt round-robin to the 8 XCDs: each XCD takes a run of
     // neighbouring tiles, rows fastest, so its L2 serves the weight tile to every row tile
     const int tiles = g.row_tiles * g.col_tiles, per = (tiles + 7) / 8;
@@ -87,167 +58,9 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_tile_kernel(GemmArgs g) {
     int64_t lo, ro;
     batch_offsets(g.bm, blockIdx.z, lo, ro);
     const int64_t M = g.M, N = g.N, K = g.K;
-    const int chunks = static_cast<int>((K + 63) / 64);
-    unsigned char* mine = lds + ks * G_::kGroup;
-
-    // staging: piece i covers tile row tid / 8 + 32 i, 16-byte piece tid % 8, through
-    // buffer resources over the tile's rows: the lane's offsets stay put, the chunk's is
-    // scalar (no address arithmetic a load), rows past the operand's end read as zero
-    const int prow = tid >> 3, ppc = tid & 7;
-    const int64_t xrows = min<int64_t>(G_::BM, M - m0), wrows = min<int64_t>(G_::BN, N - n0);
-    const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(g.a + lo + m0 * K), 0, static_cast<int>(xrows * K * 2), 0x00020000);
-    const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(g.w + ro + n0 * K), 0, static_cast<int>(wrows * K * 2), 0x00020000);
-    int xo[G_::XP], wo[G_::WP];
-#pragma unroll
-    for (int i = 0; i < G_::XP; i++) xo[i] = static_cast<int>((prow + 32 * i) * K * 2) + 16 * ppc;
-#pragma unroll
-    for (int i = 0; i < G_::WP; i++) wo[i] = static_cast<int>((prow + 32 * i) * K * 2) + 16 * ppc;
-    const int put = prow * 128 + ((ppc ^ ((prow >> 1) & 7)) << 4);  // + 4096 i: (prow + 32 i) / 2 % 8 is the same
-    u32x4_t xv[G_::XP], wv[G_::WP];
-    // from the last chunk on, where that is half a chunk (k a multiple of 32, not of
-    // 64): the pieces past K are put out of range and read as zero
-    auto last_half = [&](int c) {
-        if ((K & 63) == 0 || c != chunks - 1 || ppc < 4) return;
-#pragma unroll
-        for (int i = 0; i < G_::XP; i++) xo[i] |= static_cast<int>(0x80000000u);
-#pragma unroll
-        for (int i = 0; i < G_::WP; i++) wo[i] |= static_cast<int>(0x80000000u);
-    };
-    auto load1 = [&](int c, int i) {
-        if (i < G_::XP)
-            xv[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(xres, xo[i], 128 * c, 0));
-        else
-            wv[i - G_::XP] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(wres, wo[i - G_::XP], 128 * c, 0));
-    };
-    auto store1 = [&](int b, int i) {
-        unsigned char* to = mine + b * (G_::kX + G_::kW) + put;
-        if (i < G_::XP) *reinterpret_cast<u32x4_t*>(to + 4096 * i) = xv[i];
-        else *reinterpret_cast<u32x4_t*>(to + G_::kX + 4096 * (i - G_::XP)) = wv[i - G_::XP];
-    };
-    constexpr int kAll = G_::XP + G_::WP;
-    auto load = [&](int c) {
-        last_half(c);
-#pragma unroll
-        for (int i = 0; i < kAll; i++) load1(c, i);
-    };
-    auto store = [&](int b) {
-#pragma unroll
-        for (int i = 0; i < kAll; i++) store1(b, i);
-    };
-    f32x16_t acc[WM][WN];
-#pragma unroll
-    for (int t = 0; t < WM; t++)
-#pragma unroll
-        for (int c = 0; c < WN; c++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) acc[t][c][i] = 0.0f;
-    const int sw = (col >> 1) & 7;
-    const int rounds = (chunks + KS - 1) / KS;
-    // past the group's last chunk that chunk is repeated: stored and never read
-    const int last = chunks - 1 - (chunks - 1 - ks) % KS;  // this group's last chunk (below ks: none)
-    const int n_mine = ks < chunks ? (last - ks) / KS + 1 : 0;
-    auto nth = [&](int j) -> int { return min(ks + j * KS, max(last, 0)); };
-    load(min(nth(0), chunks - 1));
-    store(0);
-    load(min(nth(1), chunks - 1));
-    __syncthreads();
-    int b = 0;
-    for (int r = 0; r < rounds; r++, b ^= 1) {
-        const unsigned char* xt = mine + b * (G_::kX + G_::kW) + (32 * WM * wm + col) * 128;
-        const unsigned char* wt = mine + b * (G_::kX + G_::kW) + G_::kX + (32 * WN * wn + col) * 128;
-        bf16x8_t xf[2][WM], wf[2][WN];
-        auto frags = [&](int s, int o) {
-            const int at = ((2 * s + half) ^ sw) << 4;  // k 16 s + 8 half .. of a row: piece 2 s + half
-#pragma unroll
-            for (int t = 0; t < WM; t++) xf[o][t] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(xt + 4096 * t + at));
-#pragma unroll
-            for (int q = 0; q < WN; q++) wf[o][q] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(wt + 4096 * q + at));
-        };
-        if (KS == 1 || r < n_mine) {
-            const int next = min(nth(r + 2), chunks - 1);
-            last_half(next);
-            frags(0, 0);
-#pragma unroll
-            for (int s = 0; s < 4; s++) {
-                if (s < 3) frags(s + 1, (s + 1) & 1);
-#pragma unroll
-                for (int i = kAll * s / 4; i < kAll * (s + 1) / 4; i++) {
-                    store1(b ^ 1, i);
-                    load1(next, i);
-                }
-#pragma unroll
-                for (int q = 0; q < WN; q++)
-#pragma unroll
-                    for (int t = 0; t < WM; t++)
-                        acc[t][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[s & 1][q], xf[s & 1][t], acc[t][q], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        __syncthreads();
-    }
-    if constexpr (KS > 1) {
-        float* red = reinterpret_cast<float*>(lds);
-        const int w4 = wave & 3;
-        if (ks > 0) {
-#pragma unroll
-            for (int t = 0; t < WM; t++)
-#pragma unroll
-                for (int c = 0; c < WN; c++)
-#pragma unroll
-                    for (int i = 0; i < 16; i++)
-                        red[((((ks - 1) * 4 + w4) * WM * WN + t * WN + c) * 16 + i) * 64 + lane] = acc[t][c][i];
-        }
-        __syncthreads();
-        if (ks == 0) {
-#pragma unroll
-            for (int q = 0; q < KS - 1; q++)
-#pragma unroll
-                for (int t = 0; t < WM; t++)
-#pragma unroll
-                    for (int c = 0; c < WN; c++)
-#pragma unroll
-                        for (int i = 0; i < 16; i++)
-                            acc[t][c][i] += red[(((q * 4 + w4) * WM * WN + t * WN + c) * 16 + i) * 64 + lane];
-        }
-        __syncthreads();
-        if (ks > 0) return;
-    }
-    // acc[t][c][i]: row 32 t + col, column 32 c + 8 (i / 4) + 4 half + i % 4 of the wave's part:
-    // through LDS (wave-private) into whole row segments
-    unsigned char* ot = lds + (wave & 3) * 32 * WM * G_::kRowPitch;
-    const int64_t mw = m0 + 32 * WM * wm, nw = n0 + 32 * WN * wn;
-#pragma unroll
-    for (int c = 0; c < WN; c++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            float bias[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (g.bias)
-#pragma unroll
-                for (int x = 0; x < 4; x++) bias[x] = bf16_to_f32(g.bias[min<int64_t>(nw + 32 * c + 8 * q + 4 * half + x, N - 1)]);
-#pragma unroll
-            for (int t = 0; t < WM; t++)
-                *reinterpret_cast<uint2*>(ot + (32 * t + col) * G_::kRowPitch + 2 * (32 * c + 8 * q + 4 * half)) =
-                    make_uint2(pack_bf16x2(acc[t][c][4 * q] + bias[0], acc[t][c][4 * q + 1] + bias[1]),
-                               pack_bf16x2(acc[t][c][4 * q + 2] + bias[2], acc[t][c][4 * q + 3] + bias[3]));
-        }
-    __builtin_amdgcn_wave_barrier();
-    uint16_t* out = g.out + static_cast<int64_t>(blockIdx.z) * M * N;
-    constexpr int kLanes = 4 * WN;  // lanes per row, 8 columns each
-    const bool wide = (N & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-#pragma unroll
-    for (int i = 0; i < 32 * WM * kLanes / 64; i++) {
-        const int r = (64 * i + lane) / kLanes, c8 = 8 * ((64 * i + lane) % kLanes);
-        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ot + r * G_::kRowPitch + 2 * c8);
-        if (mw + r >= M || nw + c8 >= N) continue;
-        uint16_t* to = out + (mw + r) * N + nw + c8;
-        if (wide) {
-            *reinterpret_cast<u32x4_t*>(to) = v;
-        } else {
-            for (int x = 0; x < 8 && nw + c8 + x < N; x++) to[x] = static_cast<uint16_t>(v[x >> 1] >> (16 * (x & 1)));
-        }
-    }
+    gemm_tile<WM, WN, KS, false>(lds, g.a + lo + m0 * K, static_cast<int>(min<int64_t>(G_::BM, M - m0)), g.w + ro + n0 * K,
+                                 static_cast<int>(min<int64_t>(G_::BN, N - n0)), K, g.bias ? g.bias + n0 : nullptr,
+                                 g.out + (static_cast<int64_t>(blockIdx.z) * M + m0) * N + n0, N);
 }
 
 // Any dtype, either operand transposed: 64 x 64 output tile per workgroup,

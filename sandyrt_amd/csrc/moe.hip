@@ -26,8 +26,10 @@
 //     reference's per-add rounding -- bit-identical to the CPU, no atomics;
 //   - the grouped GEMM streams each expert's weights once through
 //     v_mfma_f32_16x16x32_bf16 tiles (rows of the expert as the M dimension),
-//     HBM-bound like the reference's cuBLAS grouped GEMM.
+//     HBM-bound like the reference's cuBLAS grouped GEMM; experts with many
+//     rows go through the 32x32x16 tiles of gemm_tile.h.
 #include "common.h"
+#include "gemm_tile.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -1212,6 +1214,72 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
     }
 }
 
+// The same product for many rows an expert: tiles of gemm_tile.h, one workgroup per
+// (expert, row tile, column tile), row tiles numbered over the experts' own counts.
+// Bound: the weight stream up to about 64 rows an expert (508 MB in 106 us, 4.8
+// TB/s), then MFMA issue as in the dense tile (128 rows: 65 GFLOP in 157 us with
+// half of the second row tiles empty).
+template <int WM, int WN, int KS>
+__global__ __launch_bounds__(256 * KS, 2) void moe_gemm_tile_kernel(
+        const uint16_t* __restrict__ x, const void* __restrict__ offs, int32_t off_dt, const uint16_t* __restrict__ w,
+        uint16_t* __restrict__ out, int64_t rows, int64_t K, int64_t M, int64_t experts, int col_tiles, uint32_t* errw) {
+    using G_ = TileGeo<WM, WN, KS>;
+    extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
+    const int lane = threadIdx.x & 63;
+    const int64_t b = blockIdx.y;
+    // runs of 16 neighbouring tiles (row tiles fastest) go to one XCD, so that its L2
+    // serves a weight tile to the expert's row tiles; the tiles past the last row come last
+    const int j = static_cast<int>(blockIdx.x >> 3);
+    int want = (j >> 4) * 128 + static_cast<int>(blockIdx.x & 7) * 16 + (j & 15);
+    const bool check = want == 0;  // scans every expert's offsets
+    int64_t e = -1, begin = 0, end = 0;
+    int mine = 0, n_rt = 1;
+    bool bad = false;
+    for (int64_t e0 = 0; e0 < experts && (e < 0 || check); e0 += 128) {
+        int64_t lo[2], hi[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int64_t at = b * (experts + 1) + min<int64_t>(e0 + 64 * h + lane, experts - 1);
+            lo[h] = load_index(offs, off_dt, at);
+            hi[h] = load_index(offs, off_dt, at + 1);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const bool in = e0 + 64 * h + lane < experts;
+            const bool valid = lo[h] >= 0 && hi[h] >= lo[h] && hi[h] <= rows;
+            bad = bad || (in && !valid);
+            const int nt = in && valid ? static_cast<int>((hi[h] - lo[h] + G_::BM - 1) / G_::BM) : 0;
+            int incl = nt;  // row tiles of this and the lower lanes' experts
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int up = __shfl_up(incl, d, 64);
+                if (lane >= d) incl += up;
+            }
+            const uint64_t past = __ballot(want < incl * col_tiles);
+            if (e < 0 && past) {
+                const int src = __ffsll(static_cast<unsigned long long>(past)) - 1;
+                e = e0 + 64 * h + src;
+                begin = __shfl(lo[h], src, 64);
+                end = __shfl(hi[h], src, 64);
+                n_rt = __shfl(nt, src, 64);
+                mine = want - (__shfl(incl, src, 64) - n_rt) * col_tiles;
+            }
+            want -= __shfl(incl, 63, 64) * col_tiles;
+        }
+    }
+    if (bad) atomicOr(errw, static_cast<uint32_t>(SANDY_DEVERR_OFFSETS));
+    if (e < 0) return;
+    e = __builtin_amdgcn_readfirstlane(static_cast<int>(e));
+    begin = __builtin_amdgcn_readfirstlane(static_cast<int>(begin));
+    end = __builtin_amdgcn_readfirstlane(static_cast<int>(end));
+    n_rt = __builtin_amdgcn_readfirstlane(n_rt);
+    mine = __builtin_amdgcn_readfirstlane(mine);
+    const int64_t m0 = begin + static_cast<int64_t>(mine % n_rt) * G_::BM, n0 = static_cast<int64_t>(mine / n_rt) * G_::BN;
+    gemm_tile<WM, WN, KS, true>(tile_lds, x + (b * rows + m0) * K, static_cast<int>(min<int64_t>(G_::BM, end - m0)),
+                                w + (e * M + n0) * K, static_cast<int>(min<int64_t>(G_::BN, M - n0)), K, nullptr,
+                                out + (b * rows + m0) * M + n0, M);
+}
+
 // The same product for few routes (decode batches): a pure weight stream, and
 // only the experts that got a row stream anything -- one workgroup per (expert,
 // tile) of all experts, each with one chunk in flight, spent 50 us on 140 MB
@@ -1729,6 +1797,28 @@ extern "C" int sandy_hip_moe_matmul(const SandyTensor* x, const SandyTensor* exp
             hipLaunchKernelGGL((stream_form == 2 ? moe_gemm_stream_kernel<2, 4, 4> : moe_gemm_stream_kernel<1, 1, 4>), grid,
                                dim3(256), 0, stream, px, po_, expert_offsets->dtype, pw, po, rows, K, M, experts, slots,
                                errw);
+            SANDY_HIP_TRY(hipGetLastError(), e, "moe_matmul launch");
+            return ok(e);
+        }
+        // more than 44 rows an expert: 128 x 192 tiles over the experts' own row tiles.
+        // The kernel above reads an expert's weights again for every 64 rows, and one
+        // expert past 64 holds up the launch (gate / down, us, there -> here: 128
+        // experts, 42 rows each on average 82-137 / 102 -> 99 / 111, 64 rows 149 / 173
+        // -> 106 / 117, 128 rows 241 / 285 -> 157 / 148, 256 rows 428 / 512 -> 201 /
+        // 214; 37 rows 81 / 100 against 98 / 109).  64 x 192 tiles 132 / 129 at 64
+        // rows, 170 / 175 at 128; 128 x 128 tiles 122 / 129 and 154 / 157.
+        using Tile = TileGeo<2, 3, 1>;
+        const int64_t col_tiles = (M + Tile::BN - 1) / Tile::BN;
+        // row tiles of all experts together: whole ones, and one partial one each
+        const int64_t tiles = (rows / Tile::BM + std::min(rows, experts)) * col_tiles;
+        if (env_int("SANDY_MOE_TILE", rows > 44 * experts) && rows <= 0x7fffffff && batch <= 65535 && K <= (1 << 22) &&
+            tiles <= (1 << 30)) {
+            SANDY_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(moe_gemm_tile_kernel<2, 3, 1>),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, Tile::kBytes), e, "moe_matmul");
+            hipLaunchKernelGGL((moe_gemm_tile_kernel<2, 3, 1>),
+                               dim3(static_cast<unsigned>((tiles + 127) / 128 * 128), static_cast<unsigned>(batch)),
+                               dim3(Tile::THREADS), Tile::kBytes, stream, px, po_, expert_offsets->dtype, pw, po, rows, K, M,
+                               experts, static_cast<int>(col_tiles), errw);
             SANDY_HIP_TRY(hipGetLastError(), e, "moe_matmul launch");
             return ok(e);
         }

@@ -310,6 +310,40 @@ def test_moe_matmul_few_routes_bad_offsets(ops, monkeypatch, form):
         ops.check_device_errors()
 
 
+@pytest.mark.parametrize("counts,M,K", [
+    ([0, 1, 63, 64, 65, 127, 128, 129, 300], 200, 96),  # edges of 64-row halves and 128-row tiles; a ragged column tile
+    ([130] + [0] * 140 + [45, 0, 1], 33, 32),           # experts past the first scan of 128; one half chunk; odd columns
+    ([257], 192, 64),
+    ([100, 100], 385, 416),                             # a column tile of one; seven chunks, the last a half
+])
+def test_moe_matmul_many_rows(ops, oracle, monkeypatch, counts, M, K):
+    """The 128 x 192 tiles over the experts' own row tiles, batched."""
+    monkeypatch.setenv("SANDY_MOE_TILE", "1")
+    monkeypatch.setenv("SANDY_MOE_STREAM", "0")
+    r = rng(len(counts) + M + K)
+    E, rows = len(counts), int(np.sum(counts))
+    offs = np.stack([np.concatenate([[0], np.cumsum(c)]).astype(np.int64) for c in (counts, counts[::-1])])
+    x = from_f32(normal(r, (2, rows, K)), torch.bfloat16)
+    w = from_f32(normal(r, (E, M, K), 0.1), torch.bfloat16)
+    got = ops.moe_matmul(x, torch.from_numpy(offs).cuda(), w, True)
+    ops.check_device_errors()
+    assert_close(got, oracle.moe_matmul(to_oracle(x), offs, to_oracle(w), True), torch.bfloat16, "moe_matmul")
+
+
+def test_moe_matmul_many_rows_bad_offsets(ops, monkeypatch):
+    """An invalid offset past every expert with rows is still recorded."""
+    from sandyrt_amd._lib import SandyError
+    monkeypatch.setenv("SANDY_MOE_STREAM", "0")
+    monkeypatch.setenv("SANDY_MOE_TILE", "1")
+    x = torch.zeros(1, 32, dtype=torch.bfloat16, device="cuda")
+    w = torch.zeros(200, 16, 32, dtype=torch.bfloat16, device="cuda")
+    offs = torch.ones(201, dtype=torch.int64, device="cuda")
+    offs[0], offs[190] = 0, -1
+    ops.moe_matmul(x, offs, w, True)
+    with pytest.raises(SandyError, match="moe_matmul invalid expert offsets"):
+        ops.check_device_errors()
+
+
 def test_moe_matmul_bad_offsets_sets_device_error(ops):
     from sandyrt_amd._lib import SandyError
     x = torch.zeros(4, 32, dtype=torch.bfloat16, device="cuda")
