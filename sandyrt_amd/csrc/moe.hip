@@ -19,8 +19,8 @@
 //   - the permute is a device-side stable counting sort: one workgroup per
 //     (expert, share of its rows) ranks that expert's routes by ballots and
 //     copies its rows in the same launch (one workgroup per batch ranks
-//     longer route lists), so rows come out in exactly the CPU order and no
-//     host round trip is needed;
+//     route lists past 65535), so rows come out in exactly the CPU order and
+//     no host round trip is needed;
 //   - the combine is a gather-reduce: one wave per (token, 512 columns)
 //     finds its rows with ballots in row order and accumulates with the
 //     reference's per-add rounding -- bit-identical to the CPU, no atomics;
@@ -572,6 +572,7 @@ __global__ __launch_bounds__(256) void moe_copy_rows_kernel(const char* __restri
 // with q % C == c (one wave per row).  Share 0 writes e's offset (the last
 // expert also the total).
 constexpr int kDispatchRoutes = 8192;
+constexpr int kTokenRoutes = 65535;  // token-major form: 16-bit counts
 
 // CH chunks of 256 routes per thread in registers (16 up to 4096 routes, 32
 // up to 8192): all their loads are in flight at once, so registers, and with
@@ -696,7 +697,7 @@ __global__ __launch_bounds__(256) void moe_dispatch_kernel(
     }
 }
 
-// Token-major form of the same permute (the default up to 8192 routes):
+// Token-major form of the same permute (the default up to 65535 routes):
 // workgroup = (TPW consecutive tokens, batch).  Every workgroup reads the
 // batch's route ids once and builds in LDS the per-expert count of all valid
 // routes and of those before its first route; an exclusive scan of the
@@ -719,8 +720,9 @@ __global__ __launch_bounds__(256) void moe_dispatch_tokens_kernel(
         int64_t top_k_arg, int64_t experts, int tpw, const char* __restrict__ x, char* __restrict__ packed,
         int64_t row_bytes, void* __restrict__ packed_w, void* __restrict__ token_ids, int32_t tok_dt,
         void* __restrict__ offsets, int32_t off_dt, uint32_t* errw) {
-    // 32-bit route and expert arithmetic: the launch keeps routes <= 8192
+    // 32-bit route and expert arithmetic: the launch keeps routes <= 65535
     // and 2 * experts + 64 <= 16384
+    constexpr bool kLong = CH > 32;  // takes more than CH * 256 routes
     const int top_k = TK > 0 ? TK : static_cast<int>(top_k_arg);
     const int E = static_cast<int>(experts);
     extern __shared__ int32_t sh[];
@@ -787,6 +789,24 @@ __global__ __launch_bounds__(256) void moe_dispatch_tokens_kernel(
         if (in && ok) atomicAdd(&total[e], r < r0 ? 0x10001 : 1);  // both counts in one atomic (routes < 2^16)
     }
 
+    // longer route lists: CH more chunks at a time
+    for (int c0 = 256 * CH; kLong && c0 < routes; c0 += 256 * CH) {
+#pragma unroll
+        for (int j = 0; j < CH; j++) {
+            const int r = c0 + tid + 256 * j;
+            raw[j] = idp[r < routes ? r : 0];
+        }
+#pragma unroll
+        for (int j = 0; j < CH; j++) asm volatile("" : "+v"(raw[j]));
+#pragma unroll
+        for (int j = 0; j < CH; j++) {
+            const int r = c0 + tid + 256 * j;
+            const bool in = r < routes;
+            const bool ok = raw[j] < static_cast<id_t>(E);
+            bad = bad || (in && !ok);
+            if (in && ok) atomicAdd(&total[static_cast<int>(raw[j])], r < r0 ? 0x10001 : 1);
+        }
+    }
     if (bad && blockIdx.x == 0) atomicOr(errw, static_cast<uint32_t>(SANDY_DEVERR_EXPERT_ID));
     __syncthreads();
     if (tid < 64) {
@@ -808,7 +828,7 @@ __global__ __launch_bounds__(256) void moe_dispatch_tokens_kernel(
             if (ex < E) {
                 const int tc = total[ex];
                 if (blockIdx.x == 0) store_index(offsets, off_dt, ob + ex, acc);
-                before[ex] = acc + (tc >> 16);
+                before[ex] = acc + static_cast<int>(static_cast<uint32_t>(tc) >> 16);
                 acc += tc & 0xffff;
             }
         }
@@ -1639,7 +1659,9 @@ extern "C" int sandy_hip_moe_gather(const SandyTensor* x, const SandyTensor* top
     const int64_t row_bytes = hidden * static_cast<int64_t>(dtype_size(x->dtype));
     const int aligned = (row_bytes % 16 == 0) &&
                         ((reinterpret_cast<uintptr_t>(base_ptr(*x)) | reinterpret_cast<uintptr_t>(base_ptr(*packed_x))) & 15) == 0;
-    if (routes <= kDispatchRoutes && batch <= 65535 && aligned && top_k <= 64 && 2 * num_experts + 64 <= 16384 &&
+    // the one-workgroup ranking and row copy below took 167 us for 16384 routes of 8 a
+    // token where this form's workgroups, each reading every id, take 34
+    if (routes <= kTokenRoutes && batch <= 65535 && aligned && top_k <= 64 && 2 * num_experts + 64 <= 16384 &&
         env_int("SANDY_MOE_ROUTE_GENERAL", 0) == 0) {
         // token-major: about 256 workgroups of ceil(seq / 256) tokens (at most 64 routes each)
         const int64_t tpw = std::max<int64_t>(1, std::min<int64_t>(64 / top_k, (seq + 255) / 256));
@@ -1648,7 +1670,9 @@ extern "C" int sandy_hip_moe_gather(const SandyTensor* x, const SandyTensor* top
         const size_t shb = static_cast<size_t>(2 * num_experts + 64) * sizeof(int32_t);
         dim3 grid(static_cast<unsigned>(wgs), static_cast<unsigned>(batch));
         const bool i64 = topk_ids->dtype == SANDY_I64;
-        const void* kern = routes <= 4096 ? dispatch_tokens_ch<16>(top_k, i64) : dispatch_tokens_ch<32>(top_k, i64);
+        const void* kern = routes <= 4096   ? dispatch_tokens_ch<16>(top_k, i64)
+                           : routes <= 8192 ? dispatch_tokens_ch<32>(top_k, i64)
+                                            : dispatch_tokens_ch<48>(top_k, i64);
         const void* ids_p = base_ptr(*topk_ids);
         const void* w_p = base_ptr(*topk_weights);
         int32_t w_dt = topk_weights->dtype, tok_dt = token_ids->dtype, off_dt = expert_offsets->dtype;

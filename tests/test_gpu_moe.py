@@ -132,11 +132,11 @@ def test_router_chain_config5(ops, oracle):
 @pytest.mark.parametrize("idx", [np.int64, np.int32])
 @pytest.mark.parametrize("ranking", ["dispatch", "general"])
 def test_moe_gather_bit_exact(ops, oracle, monkeypatch, dtype, T, H, E, K, idx, ranking):
-    """The token-major dispatch (the default up to 8192 routes with 16-byte
+    """The token-major dispatch (the default up to 65535 routes with 16-byte
     rows), the expert-major dispatch (rows of other widths: H = 20 in bf16)
-    and the single-workgroup ballot ranking plus row copy (the path past 8192
-    routes, forced here by SANDY_MOE_ROUTE_GENERAL) give the reference's
-    packing bit for bit; 1100 x 8 routes always take the general path."""
+    and the single-workgroup ballot ranking plus row copy (the path of longer
+    route lists, forced here by SANDY_MOE_ROUTE_GENERAL) give the reference's
+    packing bit for bit."""
     if ranking == "general":
         monkeypatch.setenv("SANDY_MOE_ROUTE_GENERAL", "1")
     r = rng(T * 7 + E)
@@ -153,6 +153,32 @@ def test_moe_gather_bit_exact(ops, oracle, monkeypatch, dtype, T, H, E, K, idx, 
     assert_equal(tok, wtok, "token_ids")
     assert_equal(pw, wpw, "packed_weights")
     assert_equal(px, wpx, "packed_x")
+
+
+@pytest.mark.parametrize("T,E,K,idx", [(1537, 128, 8, np.int64),   # one route past the ids held at once, times 8
+                                       (4097, 7, 8, np.int32),     # a third pass over the ids
+                                       (13107, 300, 5, np.int64),  # 65535 routes, the last the dispatch takes
+                                       (16384, 4, 4, np.int32)])   # one more than that: ranked by one workgroup
+def test_moe_gather_long(ops, oracle, T, E, K, idx):
+    """Route lists the token-major dispatch reads in several passes, skewed to
+    low experts (counts past 16 bits' sign), repeats and two invalid ids."""
+    from sandyrt_amd._lib import SandyError
+    r = rng(T + E)
+    ids = np.minimum(r.integers(0, E, (T, K)), r.integers(0, E, (T, K))).astype(idx)
+    ids[0, 0], ids[-1, -1] = E, -1
+    x = from_f32(normal(r, (T, 8)), torch.bfloat16)
+    w = from_f32(np.abs(normal(r, (T, K))), torch.float32)
+    px, pw, tok, off = ops.moe_gather(x, torch.from_numpy(ids).cuda(), w, E)
+    with pytest.raises(SandyError, match="moe_gather topk expert id out of range"):
+        ops.check_device_errors()
+    flat = ids.reshape(-1)
+    order = [i for i in np.argsort(np.where((flat < 0) | (flat >= E), E, flat), kind="stable")[:T * K - 2]]
+    n = len(order)
+    assert_equal(tok[:n], (np.array(order) // K).astype(np.int64), "token_ids")
+    assert_equal(pw[:n], to_oracle(w).reshape(-1)[order], "packed_weights")
+    assert_equal(px[:n], to_oracle(x)[np.array(order) // K], "packed_x")
+    counts = np.bincount(flat[(flat >= 0) & (flat < E)], minlength=E)
+    assert_equal(off, np.concatenate([[0], np.cumsum(counts)]).astype(np.int64), "expert_offsets")
 
 
 def test_moe_gather_batched_and_skewed(ops, oracle):
