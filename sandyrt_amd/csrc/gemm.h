@@ -672,7 +672,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC))) void
 
 // Launchers of gemm_waves_kernel, one translation unit per (form, NT) so they
 // compile in parallel: tile variant as in the host heuristic of matmul.hip
-// ((RT, CT) = 0 (1, 1), 1 (2, 1), 3 (2, 2), 4 (1, 2), 5 (2, 4), 6 (1, 4)), run
+// ((RT, CT) = 0 (1, 1), 1 (2, 1), 3 (2, 2), 4 (1, 2), 5 (2, 4), 6 (1, 4), 7 (4, 2)), run
 // length cps, chunks in flight qdepth.
 // plain (matmul_waves.hip, matmul_waves_nt.hip)
 template <bool NT>

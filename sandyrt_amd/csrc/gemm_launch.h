@@ -8,7 +8,7 @@
 
 namespace sandy_hip {
 
-// (RT, CT) = 0 (1, 1), 1 (2, 1), 3 (2, 2), 4 (1, 2), 5 (2, 4), 6 (1, 4); four
+// (RT, CT) = 0 (1, 1), 1 (2, 1), 3 (2, 2), 4 (1, 2), 5 (2, 4), 6 (1, 4), 7 (4, 2); four
 // chunks in flight only for RT * CT <= 2 (register bound)
 #define SANDY_WAVES_RUN(RT_, CT_, OCC_, R_, NORM_)                                                                  \
     case R_:                                                                                                        \
@@ -26,6 +26,9 @@ namespace sandy_hip {
         SANDY_WAVES_RUN(RT_, CT_, OCC_, 6, NORM_) SANDY_WAVES_RUN(RT_, CT_, OCC_, 8, NORM_)                    \
         SANDY_WAVES_RUN(RT_, CT_, OCC_, 10, NORM_) SANDY_WAVES_RUN(RT_, CT_, OCC_, 12, NORM_)                  \
     }
+// the 64-row tile: without the RMSNorm prologue only
+#define SANDY_WAVES_64(NORM_) \
+    if constexpr (!NORM_) SANDY_WAVES_CPS(4, 2, 2, false)
 #define SANDY_WAVES_VARIANTS(NORM_)                    \
     switch (variant) {                                 \
         case 0: SANDY_WAVES_CPS(1, 1, 4, NORM_); break; \
@@ -33,6 +36,7 @@ namespace sandy_hip {
         case 3: SANDY_WAVES_CPS(2, 2, 2, NORM_); break; \
         case 4: SANDY_WAVES_CPS(1, 2, 4, NORM_); break; \
         case 5: SANDY_WAVES_CPS(2, 4, 2, NORM_); break; \
+        case 7: SANDY_WAVES_64(NORM_) break;            \
         default: SANDY_WAVES_CPS(1, 4, 2, NORM_); break; \
     }
 
@@ -78,6 +82,7 @@ void launch_waves_qkv(int variant, int cps, int qdepth, bool norm, dim3 grid, hi
 }
 
 #undef SANDY_WAVES_VARIANTS
+#undef SANDY_WAVES_64
 #undef SANDY_WAVES_CPS
 #undef SANDY_WAVES_RUN
 

@@ -398,13 +398,14 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
             if (fz->qr) g.qr = *fz->qr;
         }
         // tile: 16 * RT rows x 16 * CT columns, variants (RT, CT) = 0 (1, 1),
-        // 1 (2, 1), 3 (2, 2), 4 (1, 2), 5 (2, 4), 6 (1, 4) -- the ones the
-        // heuristic below picks (2 is unused); SANDY_GEMM_TILE / SANDY_GEMM_CPS
+        // 1 (2, 1), 3 (2, 2), 4 (1, 2), 5 (2, 4), 6 (1, 4), 7 (4, 2; no norm
+        // prologue) -- the ones the heuristic below picks (2 is unused); SANDY_GEMM_TILE / SANDY_GEMM_CPS
         // select one of them and a run length for the tests that cover every
         // instantiated form
-        static const int kRT[] = {1, 2, 2, 2, 1, 2, 1};
-        static const int kCT[] = {1, 1, 1, 2, 2, 4, 4};
+        static const int kRT[] = {1, 2, 2, 2, 1, 2, 1, 4};
+        static const int kCT[] = {1, 1, 1, 2, 2, 4, 4, 2};
         const int64_t chunks = (p.K / 32 + 1) / 2;
+        const bool qkv = fz && fz->qr;
         int variant = env_int("SANDY_GEMM_TILE", -1);
         int cps = env_int("SANDY_GEMM_CPS", 0);
         // K: at most 32 chunks (2048 k) per workgroup, split evenly; the
@@ -412,7 +413,7 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
         int64_t ksplits = (chunks + 31) / 32;
         // chunks in flight per wave (4 only for RT * CT <= 2, register bound)
         int qdepth = 2;
-        if (variant < 0 || variant > 6 || variant == 2) {
+        if (variant < 0 || variant > (norm ? 6 : 7) || variant == 2) {
             // Measured on decode shapes with the weights streamed from HBM
             // (rotated over >= 1 GiB of copies):
             //   <= 16 rows: 16 x 16 tiles, 16 x 32 from N >= 16384 (lm-head);
@@ -420,8 +421,21 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
             //     weights from cache), 32 columns from N K >= 5M; 17..32 rows
             //     of N K >= 16M without the norm prologue: one 32-row tile
             //     (weights streamed once);
-            //   weights past 64 MB at 32 rows, and 33..64 rows: 32-row tiles,
-            //     the widest column tile giving >= 120 workgroups;
+            //   weights past 64 MB at 32 rows, and batches of 33..64 rows:
+            //     32-row tiles, the widest column tile giving >= 120 workgroups;
+            //   one product of 33..64 rows (us at 48 / 64 rows, that rule ->
+            //     here; the run length and so the sums stay the same): 16 x 16
+            //     tiles, four chunks in flight, for weights under 6M elements
+            //     (2560 x 2048 8.9 / 9.0 -> 7.5, 1024 x 4096 12.0 / 12.3 -> 8.8,
+            //     with the norm prologue 2048 x 2048 11.3 / 12.3 -> 8.4 / 8.9);
+            //     32 x 16 up to 20M (5632 x 2048 13.1 -> 9.1 / 9.5, 2048 x 5632
+            //     19.4 -> 12.6 / 13.2; not measured with the prologue, which keeps
+            //     that rule); 32 x 32 up to 64 MB (11264 x 2048 20.8 / 22.2 -> 15.2 /
+            //     15.9, with the prologue 23.4 / 24.8 -> 18.3 / 19.6; 2560 x 10240
+            //     30.6 / 32.4 -> 23.1 / 24.7); past it 64 x 32, so that the weights
+            //     stream once (32000 x 2048 43.7 / 44.5 -> 33.3 / 36.3, 14336 x 4096
+            //     52.0 / 54.2 -> 45.9 / 49.3; the prologue's work would grow with the
+            //     rows);
             //   4 chunks in flight per wave for weights under 8M elements
             //   (o projection at 32 rows 8.3 -> 6.1 us, q/k/v at one row
             //   7.4 -> 5.5 us), 2 for the larger ones;
@@ -430,6 +444,7 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
             //   K splits of runs of 12 against three of 8; 32 rows
             //   12.8 -> 11.6 us, one row 9.2 -> 8.7 us).
             const bool big = p.N * p.K * 2 > (int64_t(64) << 20);
+            constexpr int64_t kSmall = 6 << 20, kMiddle = 20 << 20;  // weight elements
             int64_t rt = 1, ct = 1;
             if (p.M <= 16 && !big) {
                 ct = p.N >= 16384 ? 2 : 1;
@@ -451,6 +466,10 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
                     ksplits = (chunks + 47) / 48;
                     qdepth = 4;
                 }
+            } else if (p.M > 32 && p.batches == 1 && !qkv && (!norm || (!big && (p.N * p.K < kSmall || p.N * p.K > kMiddle)))) {
+                rt = p.N * p.K < kSmall ? 1 : big ? 4 : 2;
+                ct = p.N * p.K <= kMiddle ? 1 : 2;
+                qdepth = p.N * p.K < kSmall ? 4 : 2;
             } else {
                 rt = p.M <= 16 ? 1 : 2;
                 const int64_t rows = (p.M + 16 * rt - 1) / (16 * rt) * p.batches;
@@ -462,11 +481,10 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
                 }
             }
             static const int kPick[2][3] = {{0, 4, 6}, {1, 3, 5}};  // [RT 1/2][CT 1/2/4]
-            variant = kPick[rt == 1 ? 0 : 1][ct == 1 ? 0 : ct == 2 ? 1 : 2];
+            variant = rt == 4 ? 7 : kPick[rt == 1 ? 0 : 1][ct == 1 ? 0 : ct == 2 ? 1 : 2];
         }
         qdepth = env_int("SANDY_GEMM_Q", qdepth);
         // the q/k/v epilogue kernels: 16-row tiles of 16 or 32 columns
-        const bool qkv = fz && fz->qr;
         if (qkv) variant = kCT[variant] == 1 ? 0 : 4;
         const int RT = kRT[variant], CT = kCT[variant];
         const int64_t row_tiles = (p.M + 16 * RT - 1) / (16 * RT);

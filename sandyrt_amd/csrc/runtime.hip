@@ -6,6 +6,7 @@
 // flags are read only when the caller asks (sandy_hip_take_device_errors).
 #include "common.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace sandy_hip {
@@ -100,7 +101,9 @@ void* device_counters(int slot, size_t bytes, hipStream_t stream, Err e, int* st
             s.ctr[slot] = nullptr;
             s.ctr_bytes[slot] = 0;
         }
-        size_t grown = bytes + bytes / 4;
+        // enough for the tiles of any usual split product at once: a later, larger
+        // one that grew the buffer would free what a captured graph still counts in
+        size_t grown = std::max<size_t>(bytes + bytes / 4, 64 * 1024);
         hipError_t st = hipMalloc(&s.ctr[slot], grown);
         if (st == hipSuccess) st = hipMemset(s.ctr[slot], 0, grown);
         if (st == hipSuccess) st = hipDeviceSynchronize();

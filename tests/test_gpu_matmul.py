@@ -166,6 +166,41 @@ def test_matmul_bf16_wave_kernel_tiles_and_splits(ops, oracle, variant, cps):
     assert torch.equal(got, again), "split-K result is not deterministic"
 
 
+@pytest.mark.parametrize("m", [33, 49, 64])
+@pytest.mark.parametrize("n,k,cps", [(600, 1248, 2), (600, 1248, 12), (33, 96, 0), (64, 4160, 0)])
+def test_matmul_bf16_wave_kernel_64_rows(ops, oracle, m, n, k, cps):
+    """The decode kernel's 64-row tile: partial row tiles, a column tile of one,
+    split K, half chunks."""
+    r = rng(m + n + k)
+    L = from_f32(normal(r, (m, k)), torch.bfloat16)
+    W = from_f32(normal(r, (n, k), 0.05), torch.bfloat16)
+    want = oracle.matmul(to_oracle(L), to_oracle(W), transpose_rhs=True)
+    with env(SANDY_GEMM_WAVES=1, SANDY_GEMM_TILE=7, SANDY_GEMM_CPS=cps):
+        got = ops.matmul(L, W, transpose_rhs=True)
+    assert_close(got, want, torch.bfloat16, "64-row tile")
+
+
+@pytest.mark.parametrize("m", [33, 64])
+@pytest.mark.parametrize("n,k", [(2048, 2080), (2560, 3072), (7168, 3072), (34000, 1024)])
+def test_matmul_bf16_rows_33_to_64(ops, m, n, k):
+    """Each weight range of the 33..64-row rule against fp32, and the fused
+    residual and norm forms bit-identical to the separate ops."""
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    x = torch.randn(m, k, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(n, k, generator=g, device="cuda") * 0.05).to(torch.bfloat16)
+    res = torch.randn(m, n, generator=g, device="cuda").to(torch.bfloat16)
+    got = ops.matmul(x, w, transpose_rhs=True)
+    assert_close(got, to_oracle((x.float() @ w.float().t()).to(torch.bfloat16)), torch.bfloat16, "fp32 product")
+    assert torch.equal(ops.matmul_residual(x, w, res), (got.float() + res.float()).to(torch.bfloat16))
+    px = (torch.randn(k, 64, generator=g, device="cuda") * 0.1).to(torch.bfloat16)
+    stats = ops.row_stats_buffer(m, k)
+    s = ops.matmul_residual(torch.randn(m, 64, generator=g, device="cuda").to(torch.bfloat16), px,
+                            torch.zeros(m, k, dtype=torch.bfloat16, device="cuda"), stats)
+    nw = torch.randn(k, generator=g, device="cuda").to(torch.bfloat16)
+    assert torch.equal(ops.matmul_rms(s, stats, nw, 1e-5, w),
+                       ops.matmul(ops.rms_norm(s, nw, 1e-5), w, transpose_rhs=True))
+
+
 def test_matmul_bf16_split_counters_rearm(ops, oracle):
     """Back-to-back split-K launches of different shapes: each launch leaves its
     arrival counters at zero for the next."""
