@@ -30,6 +30,7 @@
 // pages of 16: 4896 -> 41; 1500 after 300, 16 / 2 heads, D 128: 49; f32, 12
 // heads, D 64: 1000 queries 1434 -> 43, 64 queries 23.5 -> 9.8.
 #include "attention_prefill.h"
+#include "prefill_span.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -215,8 +216,9 @@ __global__ __launch_bounds__((Geo<T, D, RW>::THREADS), (Geo<T, D, RW>::kF32 && D
     const int page_mask = (1 << a.log2_page) - 1;
     bool staged = false;
     if (PAGED && a.table_pages > 0) {
-        const int n = k_begin < k_end ? min(((k_end - 1) >> a.log2_page) - page0 + 1, a.table_pages) : 0;
-        bool plain = true;  // there and 16-byte aligned
+        const int pages = k_begin < k_end ? ((k_end - 1) >> a.log2_page) - page0 + 1 : 0;
+        const int n = min(pages, a.table_pages);
+        bool plain = pages <= a.table_pages;  // all staged, there and 16-byte aligned
         for (int i = tid; i < n; i += G_::THREADS) {
             const uint64_t kp = a.k_pages[page0 + i], vp = a.v_pages[page0 + i];
             plain = plain && kp != 0 && vp != 0 && ((kp | vp) & 15) == 0;
@@ -473,9 +475,7 @@ int launch_form(const PrefillArgs& a, hipStream_t stream, Err e) {
     PrefillArgs args = a;
     size_t bytes = Geo<T, D, RW>::kBytes;
     if (PAGED) {
-        // pages a workgroup's keys can span: the whole list, or a window and its rows' queries
-        int64_t span = (static_cast<int64_t>(a.tk) >> a.log2_page) + 1;
-        if (a.window > 0) span = std::min(span, ((a.window + 32 * RW / a.group + 1) >> a.log2_page) + 2);
+        const int64_t span = prefill_page_span(a.tk, a.window, RW, a.group, a.log2_page);
         args.table_pages = span <= kTablePages ? static_cast<int32_t>(span) : 0;
         bytes += static_cast<size_t>(args.table_pages) * 16;
     }

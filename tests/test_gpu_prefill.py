@@ -102,6 +102,14 @@ def test_prefill_strided_heads_and_pages(ops, oracle, shape, dtype):
         check(ops, oracle, dtype, P=P, shift=shift, **shape)
 
 
+@pytest.mark.parametrize("rows", ["1", "2"])
+@pytest.mark.parametrize("window", [200, 201, 5000, 2 ** 63 - 66, 2 ** 63 - 2, 2 ** 63 - 1])
+def test_prefill_window_wider_than_the_keys_over_pages(ops, oracle, monkeypatch, window, rows):
+    """Windows of all the keys and more, up to the largest value (no limit)."""
+    monkeypatch.setenv("SANDY_PREFILL_RW", rows)
+    check(ops, oracle, torch.bfloat16, B=1, hq=8, hkv=1, tq=37, tk=200, D=64, pos=[163], window=window, P=16)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("P", [0, 16])
 def test_prefill_non_finite_values_reach_only_their_rows(ops, oracle, P, dtype):
