@@ -439,7 +439,27 @@ __global__ __launch_bounds__((Geo<T, D, RW>::THREADS), (Geo<T, D, RW>::kF32 && D
     // a row that sees no key (or only NaN scores) is zero, as in the general kernel
     const bool none = m == -INFINITY;
     bool finite = true;
-    if (kw == 0 && row < rows) {
+#pragma unroll
+    for (int t = 0; t < DT; t++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            acc[t][i] = none ? 0.0f : acc[t][i] * inv;
+            finite = finite && fabsf(acc[t][i]) < INFINITY;
+        }
+    // nothing is stored before it is known which rows are computed again: those read
+    // their q, and `out` may be `q`
+    const bool redo = __syncthreads_or(kw == 0 && row < rows && !finite);
+    float* stats = reinterpret_cast<float*>(lds);  // [32 * RW] max (-inf: the row stands), then 1 / sum
+    if (redo) {
+        if (kw == 0 && half == 0 && ds == 0) {
+            stats[32 * rw + col] = -INFINITY;
+            stats[32 * RW + 32 * rw + col] = inv;
+        }
+        __syncthreads();
+        if (kw == 0 && row < rows && !finite) stats[32 * rw + col] = m;  // the row's lanes all hold the same
+        __syncthreads();
+    }
+    if (kw == 0 && row < rows && (!redo || stats[32 * rw + col] == -INFINITY)) {
         char* op = static_cast<char*>(a.out) + (b * a.os[0] + (kh * a.group + qg) * a.os[1] + qt * a.os[2] + 32 * DT * ds + 4 * half) * ES;
 #pragma unroll
         for (int t = 0; t < DT; t++)
@@ -447,22 +467,13 @@ __global__ __launch_bounds__((Geo<T, D, RW>::THREADS), (Geo<T, D, RW>::kF32 && D
             for (int i = 0; i < 4; i++) {
                 float o[4];
 #pragma unroll
-                for (int x = 0; x < 4; x++) {
-                    o[x] = none ? 0.0f : acc[t][4 * i + x] * inv;
-                    finite = finite && fabsf(o[x]) < INFINITY;
-                }
+                for (int x = 0; x < 4; x++) o[x] = acc[t][4 * i + x];
                 char* to = op + (32 * t + 8 * i) * ES;
                 if constexpr (kF32) *reinterpret_cast<float4*>(to) = make_float4(o[0], o[1], o[2], o[3]);
                 else *reinterpret_cast<uint2*>(to) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
             }
     }
-    if (!__syncthreads_or(finite ? 0 : 1)) return;
-    float* stats = reinterpret_cast<float*>(lds);  // [32 * RW] max, then 1 / sum
-    if (kw == 0 && half == 0 && ds == 0) {
-        stats[32 * rw + col] = m;
-        stats[32 * RW + 32 * rw + col] = inv;
-    }
-    __syncthreads();
+    if (!redo) return;
     for (int i = 0; i < 32 * RW && r0 + i < rows; i++)
         if (stats[i] != -INFINITY)
             careful_row<T, D, PAGED>(a, b, kh, r0 + i, first_of((r0 + i) / a.group), last_of((r0 + i) / a.group), stats[i],

@@ -124,6 +124,25 @@ def test_prefill_non_finite_values_reach_only_their_rows(ops, oracle, P, dtype):
     check(ops, oracle, dtype, B=1, hq=4, hkv=2, tq=60, tk=100, D=64, pos=[40], window=30, P=P, spoil=spoil)
 
 
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.bfloat16, 256), (torch.float32, 128)])
+@pytest.mark.parametrize("rows", ["1", "2"])
+def test_prefill_in_place(ops, oracle, monkeypatch, rows, dtype, D):
+    """`out` may be `q`, also where rows are computed again for an infinity in V."""
+    monkeypatch.setenv("SANDY_PREFILL_RW", rows)
+    r = rng(D)
+    for bad in (None, float("inf")):
+        q, k = from_f32(normal(r, (1, 4, 70, D), 0.5), dtype), from_f32(normal(r, (1, 2, 90, D), 0.5), dtype)
+        v = from_f32(normal(r, (1, 2, 90, D)), dtype)
+        if bad is not None:
+            v[0, 0, 50, 3] = bad
+            v[0, 1, 2, 5] = bad
+        pos = torch.tensor([20], device="cuda")
+        want = ops.attention(q, k, v, pos)
+        got = ops.attention(q, k, v, pos, out=q)
+        assert got.data_ptr() == q.data_ptr() and torch.equal(got, want)
+        assert torch.isfinite(got).all() == (bad is None)
+
+
 def test_prefill_errors(ops):
     """A negative offset and a null page are recorded."""
     from sandyrt_amd._lib import SandyError
