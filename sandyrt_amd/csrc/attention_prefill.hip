@@ -94,50 +94,143 @@ __device__ __forceinline__ u32x4_t load_piece(uint64_t at) {
     return u32x4_t{w[0], w[1], w[2], w[3]};
 }
 
-// One row again, a key at a time, where V holds infinities or NaN: every key
-// the row sees adds its normalised probability times V (from the row's known
-// max and 1 / sum), so a non-finite V reaches exactly the rows that see its
-// key.  256 keys at a time through `probs`; q in `qrow`.
-template <typename T, int D, bool PAGED>
-__device__ __forceinline__ void careful_row(const PrefillArgs& a, int b, int kh, int row, int first, int last, float m,
-                                            float inv, float* probs, float* qf) {
-    constexpr int ES = Geo<T, D, 1>::ES;
-    const int tid = threadIdx.x;
-    const int t = row / a.group, h = kh * a.group + row % a.group;
-    if (tid < D) qf[tid] = Vec8<T>::load1(a.q, b * a.qs[0] + h * a.qs[1] + t * a.qs[2] + tid);
-    auto row_of = [&](bool value, int key) -> const void* {
+// Up to R neighbouring rows again, by one wave, where outputs were not all finite:
+// the general kernel's steps (scores summed over d in order, the max first, then expf
+// and a float64 sum; the keys a row does not see and those of score -inf add nothing,
+// whatever V holds), so that a non-finite K or V reaches exactly the rows that see its
+// key.  Only the rows in `redo` (bit r)
+// are stored; q of the rows as float in `qf` [R][D].
+// A lane scores one key for all R rows (K is read once for them, twice in all: for
+// the max, then for the sums), then each V row of the 64 keys is read once for the R
+// rows, p coming from its lane as a scalar.  Bound: VALU and the K and V reads' latency.
+// Every row redone (an infinity in V at key 0; us a call through Python: general kernel
+// / rows one after another on the whole workgroup / here): 2048 queries, 32 / 4 heads,
+// D 64 14363 / 26956 / 951; 777 after 1500, 8 / 2, D 256 7860 / 20702 / 947; 16 after
+// 2000, 32 / 4, D 64 447 / 11542 / 451; f32, 12 heads, D 64, 64 queries 28 / 383 / 38,
+// 1000 1427 / 5357 / 281.  More loads in flight (8 pieces of K, 32 V rows) gained
+// nothing and spilled.
+template <typename T, int D, bool PAGED, int R>
+__device__ __forceinline__ void careful_rows(const PrefillArgs& a, int b, int kh, int row0, uint32_t redo, int64_t base,
+                                             const float* qf) {
+    constexpr int ES = std::is_same_v<T, F32> ? 4 : 2;
+    constexpr int PE = 16 / ES, NK = 4;  // elements of a 16-byte piece, pieces of K in flight
+    constexpr int DL = D / 64, NV = 8;   // dims a lane owns (lane + 64 i), V rows in flight
+    const int lane = threadIdx.x & 63;
+    const int rows = a.group * a.tq;
+    auto last_of = [&](int r) -> int { return static_cast<int>(min<int64_t>(base + min(row0 + r, rows - 1) / a.group, a.tk - 1)); };
+    auto first_of = [&](int r) -> int {
+        return a.window > 0 ? static_cast<int>(min<int64_t>(max<int64_t>(0, base + min(row0 + r, rows - 1) / a.group + 1 - a.window), kMaxKeys)) : 0;
+    };
+    // a key's row: null where the page is missing (reported by the caller)
+    auto row_of = [&](bool value, int key) -> const char* {
         if constexpr (PAGED) {
             const uint64_t at = (value ? a.v_pages : a.k_pages)[key >> a.log2_page];
-            return at ? reinterpret_cast<const void*>(paged_row(at, key, a.log2_page, b * a.kv_rows_b + kh, ES * D, ES))
-                      : nullptr;
+            return at ? reinterpret_cast<const char*>(paged_row(at, key, a.log2_page, b * a.kv_rows_b + kh, ES * D, ES)) : nullptr;
         } else {
             const int64_t* st = value ? a.vs : a.ks;
             return static_cast<const char*>(value ? a.v : a.k) + (b * st[0] + kh * st[1] + key * st[2]) * ES;
         }
     };
-    float acc = 0.0f;
-    for (int k0 = first; k0 <= last; k0 += 256) {
-        __syncthreads();
-        const int n = min(256, last + 1 - k0);
-        if (tid < n) {
-            const void* kp = row_of(false, k0 + tid);
-            float s = 0.0f;
+    const int k_first = first_of(0), k_last = last_of(R - 1);
+    // p enters scaled by a power of two of the key count, so that the unnormalised
+    // sums stay below the largest |V|
+    const float fac = ldexpf(1.0f, -(32 - __clz(max(k_last - k_first, 0))));
+    float m[R], acc[R][DL];
+    double l[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        m[r] = -INFINITY;
+        l[r] = 0.0;
+#pragma unroll
+        for (int i = 0; i < DL; i++) acc[r][i] = 0.0f;
+    }
 #pragma unroll 1
-            for (int d = 0; d < D; d++) s = fmaf(qf[d], kp ? Vec8<T>::load1(kp, d) : 0.0f, s);
-            probs[tid] = (Geo<T, D, 1>::kF32 ? expf(s * a.scale - m)
-                                             : __builtin_amdgcn_exp2f(fmaf(s, a.scale_log2, -m))) * inv;
-        }
-        __syncthreads();
-        if (tid < D) {
+    for (int pass = 0; pass < 2; pass++) {
 #pragma unroll 1
-            for (int i = 0; i < n; i++) {
-                const void* vp = row_of(true, k0 + i);
-                acc = fmaf(probs[i], vp ? Vec8<T>::load1(vp, tid) : 0.0f, acc);
+        for (int k0 = k_first; k0 <= k_last; k0 += 64) {
+            const int key = min(k0 + lane, k_last);
+            const char* kp = row_of(false, key);
+            float s[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) s[r] = 0.0f;
+#pragma unroll 1
+            for (int d0 = 0; d0 < D; d0 += NK * PE) {
+                u32x4_t kv[NK];
+#pragma unroll
+                for (int i = 0; i < NK; i++)
+                    kv[i] = !PAGED || kp ? load_piece(reinterpret_cast<uint64_t>(kp) + (d0 + i * PE) * ES) : u32x4_t{0, 0, 0, 0};
+#pragma unroll
+                for (int i = 0; i < NK; i++) {
+                    float kf[PE];
+#pragma unroll
+                    for (int j = 0; j < PE; j++)
+                        kf[j] = ES == 4 ? __uint_as_float(kv[i][j & 3])
+                                        : __uint_as_float(j & 1 ? kv[i][j >> 1] & 0xffff0000u : kv[i][j >> 1] << 16);
+#pragma unroll
+                    for (int r = 0; r < R; r++)
+#pragma unroll
+                        for (int j = 0; j < PE; j++)
+                            s[r] = fmaf(qf[r * D + d0 + i * PE + j], kf[j], s[r]);
+                }
             }
+            uint64_t live[R], all = ~0ull, any = 0;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                s[r] = __fmul_rn(s[r], a.scale);
+                const bool sees = k0 + lane <= last_of(r) && k0 + lane >= first_of(r) && s[r] != -INFINITY;
+                live[r] = __ballot(sees);
+                all &= live[r];
+                any |= live[r];
+                if (pass == 0) {
+                    if (sees) m[r] = fmaxf(m[r], s[r]);
+                } else {
+                    s[r] = sees ? expf(__fsub_rn(s[r], m[r])) : 0.0f;
+                    l[r] += static_cast<double>(s[r]);
+                    s[r] *= fac;
+                }
+            }
+            if (pass == 0) continue;
+            auto weigh = [&](auto whole) {
+#pragma unroll 1
+                for (int j0 = 0; j0 < 64 && k0 + j0 <= k_last; j0 += NV) {
+                    float v[NV][DL];
+#pragma unroll
+                    for (int j = 0; j < NV; j++) {
+                        const char* vp = row_of(true, min(k0 + j0 + j, k_last));
+#pragma unroll
+                        for (int i = 0; i < DL; i++) v[j][i] = !PAGED || vp ? Vec8<T>::load1(vp, lane + 64 * i) : 0.0f;
+                    }
+#pragma unroll
+                    for (int j = 0; j < NV; j++)
+#pragma unroll
+                        for (int r = 0; r < R; r++) {
+                            const float p = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(s[r]), j0 + j));
+                            // all bits where the row takes the key, else none: p is zero there
+                            const int mask = decltype(whole)::value ? -1 : -static_cast<int>((live[r] >> (j0 + j)) & 1);
+#pragma unroll
+                            for (int i = 0; i < DL; i++)
+                                acc[r][i] = fmaf(p, __int_as_float(__float_as_int(v[j][i]) & mask), acc[r][i]);
+                        }
+                }
+            };
+            if (all == ~0ull) weigh(std::true_type{});
+            else if (any) weigh(std::false_type{});
+        }
+        if (pass == 0) {
+#pragma unroll
+            for (int r = 0; r < R; r++) m[r] = wave_max(m[r]);
         }
     }
-    if (tid < D && first <= last) Vec8<T>::store1(a.out, b * a.os[0] + h * a.os[1] + t * a.os[2] + tid, acc);
-    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const double total = wave_sum(l[r]);
+        const float inv = (total != 0.0 ? 1.0f / static_cast<float>(total) : 0.0f) / fac;
+        const int row = row0 + r;
+        if (!((redo >> r) & 1)) continue;
+        const int64_t to = b * a.os[0] + (kh * a.group + row % a.group) * a.os[1] + row / a.group * a.os[2] + lane;
+#pragma unroll
+        for (int i = 0; i < DL; i++) Vec8<T>::store1(a.out, to + 64 * i, m[r] == -INFINITY ? 0.0f : acc[r][i] * inv);
+    }
 }
 
 template <typename T, int D, int RW, bool PAGED>
@@ -449,17 +542,19 @@ __global__ __launch_bounds__((Geo<T, D, RW>::THREADS), (Geo<T, D, RW>::kF32 && D
     // nothing is stored before it is known which rows are computed again: those read
     // their q, and `out` may be `q`
     const bool redo = __syncthreads_or(kw == 0 && row < rows && !finite);
-    float* stats = reinterpret_cast<float*>(lds);  // [32 * RW] max (-inf: the row stands), then 1 / sum
+    int* bad = reinterpret_cast<int*>(lds);           // [32 * RW] rows to compute again
+    float* qf = reinterpret_cast<float*>(lds + 512);  // [32 * RW][D] their q
     if (redo) {
-        if (kw == 0 && half == 0 && ds == 0) {
-            stats[32 * rw + col] = -INFINITY;
-            stats[32 * RW + 32 * rw + col] = inv;
+        for (int i = tid; i < 32 * RW; i += G_::THREADS) bad[i] = 0;
+        for (int i = tid; i < 32 * RW * D; i += G_::THREADS) {
+            const int r = min(r0 + i / D, rows - 1);
+            qf[i] = Vec8<T>::load1(a.q, b * a.qs[0] + (kh * a.group + r % a.group) * a.qs[1] + r / a.group * a.qs[2] + i % D);
         }
         __syncthreads();
-        if (kw == 0 && row < rows && !finite) stats[32 * rw + col] = m;  // the row's lanes all hold the same
+        if (kw == 0 && row < rows && !finite) bad[32 * rw + col] = 1;
         __syncthreads();
     }
-    if (kw == 0 && row < rows && (!redo || stats[32 * rw + col] == -INFINITY)) {
+    if (kw == 0 && row < rows && !(redo && bad[32 * rw + col])) {
         char* op = static_cast<char*>(a.out) + (b * a.os[0] + (kh * a.group + qg) * a.os[1] + qt * a.os[2] + 32 * DT * ds + 4 * half) * ES;
 #pragma unroll
         for (int t = 0; t < DT; t++)
@@ -474,10 +569,14 @@ __global__ __launch_bounds__((Geo<T, D, RW>::THREADS), (Geo<T, D, RW>::kF32 && D
             }
     }
     if (!redo) return;
-    for (int i = 0; i < 32 * RW && r0 + i < rows; i++)
-        if (stats[i] != -INFINITY)
-            careful_row<T, D, PAGED>(a, b, kh, r0 + i, first_of((r0 + i) / a.group), last_of((r0 + i) / a.group), stats[i],
-                                     stats[32 * RW + i], stats + 64 * RW, stats + 64 * RW + 256);
+    constexpr int kMine = 32 * RW / (G_::THREADS / 64);  // rows of a wave
+    constexpr int R = D == 64 ? 8 : 4;
+    static_assert(32 * RW * 4 <= 512 && 512 + 32 * RW * D * 4 <= G_::kBytes && kMine % R == 0, "rows computed again");
+#pragma unroll 1
+    for (int i = wave * kMine; i < (wave + 1) * kMine && r0 + i < rows; i += R) {
+        const uint32_t which = static_cast<uint32_t>(__ballot(lane < R && bad[i + (lane & (R - 1))]));
+        if (which) careful_rows<T, D, PAGED, R>(a, b, kh, r0 + i, which, base, qf + i * D);
+    }
 }
 
 template <typename T, int D, int RW, bool PAGED>

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from tests.helpers import assert_close, from_f32, normal, rng, to_oracle
+from tests.helpers import as_f32, assert_close, from_f32, normal, rng, to_oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -60,6 +60,9 @@ def check(ops, oracle, dtype, B, hq, hkv, tq, tk, D, pos, window, P=0, shift=0, 
         np.testing.assert_allclose(got, want, rtol=1e-5, atol=8 * 2.0 ** -24 * big, err_msg=what)
     else:
         assert_close(out.contiguous(), want, dtype, what)
+        got, want = as_f32(to_oracle(out.contiguous())), as_f32(np.asarray(want))
+        np.testing.assert_array_equal(np.isnan(got), np.isnan(want), err_msg=what)
+        np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)], err_msg=what)
 
 
 SHAPES = [
@@ -122,6 +125,38 @@ def test_prefill_non_finite_values_reach_only_their_rows(ops, oracle, P, dtype):
         k[0, 0, 95, 1] = float("nan")
         k[0, 1, 98, 2] = float("inf")
     check(ops, oracle, dtype, B=1, hq=4, hkv=2, tq=60, tk=100, D=64, pos=[40], window=30, P=P, spoil=spoil)
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.bfloat16, 128), (torch.bfloat16, 256),
+                                     (torch.float32, 64), (torch.float32, 128)])
+@pytest.mark.parametrize("rows", ["1", "2"])
+@pytest.mark.parametrize("window,P,shift", [(0, 0, 0), (130, 16, 0), (0, 16, 3)])
+def test_prefill_non_finite_values_over_several_key_chunks(ops, oracle, monkeypatch, window, P, shift, rows, dtype, D):
+    """The rows computed again, in every form: infinities of both signs in one
+    column, NaN, an infinite key (its score is NaN, an infinity or -inf) and a
+    key of score -inf under an infinite value, at chunk edges."""
+    def spoil(k, v):
+        v[0, 0, 0, 3] = float("inf")
+        v[0, 0, 127, 3] = float("-inf")
+        v[0, 0, 128, D - 1] = float("nan")
+        v[0, 1, 190, 5] = float("-inf")
+        k[0, 1, 200, :] = float("-inf")
+        v[0, 1, 200, 0] = float("inf")
+        k[0, 1, 240, 2] = float("nan")
+    monkeypatch.setenv("SANDY_PREFILL_RW", rows)
+    check(ops, oracle, dtype, B=1, hq=6, hkv=2, tq=90, tk=260, D=D, pos=[165], window=window, P=P, shift=shift, spoil=spoil)
+
+
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** 14, 2.0 ** 20])
+def test_prefill_large_scores(ops, oracle, scale):
+    """Scores up to 2^40: past 2^31 the exponent's rounding alone leaves the range
+    of exp2, and the rows are computed again in the general kernel's arithmetic."""
+    r = rng(5)
+    q, k = (from_f32(normal(r, (1, h, n, 64), scale), torch.bfloat16) for h, n in ((4, 40), (2, 150)))
+    v = from_f32(normal(r, (1, 2, 150, 64)), torch.bfloat16)
+    pos = torch.tensor([110], device="cuda")
+    want = oracle.attention(to_oracle(q), to_oracle(k), to_oracle(v), np.array([110]), 0, -1.0)
+    assert_close(ops.attention(q, k, v, pos), want, torch.bfloat16, f"scale {scale}")
 
 
 @pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.bfloat16, 256), (torch.float32, 128)])
