@@ -39,8 +39,6 @@ namespace sandy_hip {
 namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
@@ -444,27 +442,29 @@ __global__ __launch_bounds__((Geo<T, D, RW>::THREADS), (Geo<T, D, RW>::kF32 && D
                         *reinterpret_cast<const float*>(src + (8 * (i >> 2) + (i & 3)) * VP + 128 * (DT * ds + t)), sc[i], acc[t], 0, 0, 0);
             continue;
         }
-        float rs = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            sc[i] = __builtin_amdgcn_exp2f(fmaf(sc[i], a.scale_log2, -shift));
-            rs += sc[i];
+        for (int i = 0; i < 16; i++) sc[i] = __builtin_amdgcn_exp2f(fmaf(sc[i], a.scale_log2, -shift));
+        {  // pairs first: four roundings deep
+            float rs[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) rs[i] = sc[2 * i] + sc[2 * i + 1];
+            l += static_cast<double>(((rs[0] + rs[1]) + (rs[2] + rs[3])) + ((rs[4] + rs[5]) + (rs[6] + rs[7])));
         }
-        l += static_cast<double>(rs);
         // contraction slot 8 half + j of step s2: key 16 s2 + 4 half + j (j < 4) or + 8 + j - 4
 #pragma unroll
         for (int s2 = 0; s2 < 2; s2++) {
-            bf16x8_t ph, pl;
+            // p = three bf16 of 8 bits each (cut, not rounded: their sum is p exactly)
+            u32x4_t p0, p1, p2;
 #pragma unroll
             for (int j = 0; j < 8; j += 2) {
-                const f32x2_t p2 = {sc[8 * s2 + j], sc[8 * s2 + j + 1]};
-                const bf16x2_t h2 = __builtin_convertvector(p2, bf16x2_t);
-                const f32x2_t back = __builtin_convertvector(h2, f32x2_t);
-                const bf16x2_t l2 = __builtin_convertvector(f32x2_t{p2[0] - back[0], p2[1] - back[1]}, bf16x2_t);
-                ph[j] = h2[0];
-                ph[j + 1] = h2[1];
-                pl[j] = l2[0];
-                pl[j + 1] = l2[1];
+                const float x = sc[8 * s2 + j], y = sc[8 * s2 + j + 1];
+                const uint32_t xb = __float_as_uint(x), yb = __float_as_uint(y);
+                const float x1 = x - __uint_as_float(xb & 0xffff0000u), y1 = y - __uint_as_float(yb & 0xffff0000u);
+                const uint32_t x1b = __float_as_uint(x1), y1b = __float_as_uint(y1);
+                const float x2 = x1 - __uint_as_float(x1b & 0xffff0000u), y2 = y1 - __uint_as_float(y1b & 0xffff0000u);
+                p0[j / 2] = __builtin_amdgcn_perm(yb, xb, 0x07060302u);  // the upper halves of both
+                p1[j / 2] = __builtin_amdgcn_perm(y1b, x1b, 0x07060302u);
+                p2[j / 2] = __builtin_amdgcn_perm(__float_as_uint(y2), __float_as_uint(x2), 0x07060302u);
             }
             // ds_read_b64_tr_b16: in each 16-lane group, lane i gets element i % 4 of
             // the 8-byte pieces addressed by lanes 4 n + i / 4 (n = 0..3): pointing
@@ -479,8 +479,9 @@ __global__ __launch_bounds__((Geo<T, D, RW>::THREADS), (Geo<T, D, RW>::kF32 && D
                 const short4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                     (short4_t __attribute__((address_space(3)))*)((unsigned char __attribute__((address_space(3)))*)(s0 + 8 * VP)));
                 const bf16x8_t va = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
-                acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, ph, acc[t], 0, 0, 0);
-                acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pl, acc[t], 0, 0, 0);
+                acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, __builtin_bit_cast(bf16x8_t, p0), acc[t], 0, 0, 0);
+                acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, __builtin_bit_cast(bf16x8_t, p1), acc[t], 0, 0, 0);
+                acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, __builtin_bit_cast(bf16x8_t, p2), acc[t], 0, 0, 0);
             }
         }
     }
