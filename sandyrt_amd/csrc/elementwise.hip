@@ -418,6 +418,7 @@ extern "C" int sandy_hip_elementwise(const SandyScalarNode* nodes, int32_t node_
     for (int i = 0; i < node_count; i++) {
         put(nodes[i].id);
         put(nodes[i].op);
+        put(nodes[i].operand_count);  // the SiLU pattern's tanh has exactly one
         if (nodes[i].op == 0) put(nodes[i].input_index);
         if (nodes[i].op == 1) put(nodes[i].constant);
         const int need = nodes[i].op <= 1 ? 0 : nodes[i].op <= 7 ? 2 : 1;

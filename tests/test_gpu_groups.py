@@ -39,6 +39,24 @@ def test_fused_group_matches_fused_oracle(ops, oracle, dtype, shape, group):
     assert_close(got, want, dtype, group)
 
 
+def test_group_does_not_depend_on_what_was_compiled_before(ops):
+    """A tanh with a spare operand is accepted and keeps the group out of the
+    SiLU pattern: its kernel and the plain group's are different ones,
+    whichever is compiled first (a dead constant makes the groups new)."""
+    from dataclasses import replace
+    g, u = (from_f32(normal(rng(s), (64, 1000)), torch.float32) for s in (31, 32))
+    got = {}
+    for order in (("plain", "spare"), ("spare", "plain")):
+        nodes, result = ops.silu_mul_nodes()
+        nodes = nodes + [ops.ScalarNode(9, ops.CONST, constant=7.0 if order[0] == "plain" else 9.0)]
+        for kind in order:
+            group = [replace(n, operands=(2, 2)) if kind == "spare" and n.op == ops.TANH else n for n in nodes]
+            got[order[0], kind] = to_oracle(ops.elementwise(group, result, [g, u]))
+    assert not np.array_equal(got["plain", "plain"], got["plain", "spare"]), "the two kernels round differently"
+    for kind in ("plain", "spare"):
+        assert_equal(got["plain", kind], got["spare", kind], kind)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_silu_gate_matches_unfused_reference_chain(ops, oracle, dtype):
     """The fused group against the reference's unfused op chain (each op
