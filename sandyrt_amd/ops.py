@@ -220,26 +220,27 @@ class ScalarNode:
     operands: tuple = ()
 
 
-_NODE_LAYOUT = struct.Struct("=IiiIdi2I4x")  # SandyScalarNode
+_NODE_LAYOUT = struct.Struct("=IiiI8si2I4x")  # SandyScalarNode, its constant as bytes
+_F64 = struct.Struct("=d")
 
 
 @functools.lru_cache(maxsize=256)
 def _packed_nodes(key):
-    """SandyScalarNode array of (id, op, input_index, constant, operands) tuples."""
+    """SandyScalarNode array of (id, op, input_index, constant's bytes, operands) tuples."""
     def u32(*v):
         return [x & 0xFFFFFFFF for x in v]  # as a C field takes them: the library rejects what is out of range
 
     if any(len(operands) > 2 for *_, operands in key):
         raise IndexError("a scalar node has at most two operands")
-    data = b"".join(_NODE_LAYOUT.pack(*u32(i), op, _lib.F32, *u32(inp), float(const), len(operands),
-                                      *u32(*operands, *(0,) * (2 - len(operands))))
+    data = b"".join(_NODE_LAYOUT.pack(*u32(i), (op + 0x80000000 & 0xFFFFFFFF) - 0x80000000, _lib.F32, *u32(inp), const,
+                                      len(operands), *u32(*operands, *(0,) * (2 - len(operands))))
                     for i, op, inp, const, operands in key)
     return (_lib.SandyScalarNode * len(key)).from_buffer_copy(data)
 
 
 def _nodes(nodes):
-    # looked up by content; zeros by their text, which keeps their sign
-    return _packed_nodes(tuple([(n.id, n.op, n.input_index, n.constant or str(n.constant), tuple(n.operands)) for n in nodes]))
+    # looked up by content: a constant by its value now (any object with a float value, zeros with their sign)
+    return _packed_nodes(tuple([(n.id, n.op, n.input_index, _F64.pack(n.constant), tuple(n.operands)) for n in nodes]))
 
 
 @_reads_paged

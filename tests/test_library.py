@@ -107,3 +107,27 @@ def test_packed_arguments():
     assert str(ops._nodes(nodes)[1].constant) == "-0.0"
     nodes[1].constant = 3.5
     assert ops._nodes(nodes)[1].constant == 3.5
+
+
+def test_node_constants_by_value():
+    """A scalar node's constant is any object with a float value, taken at the
+    call: booleans and zeros, numpy scalars, and a tensor changed in place
+    between calls; an op past int32 wraps as a C field does (and is rejected)."""
+    import numpy as np
+    import torch
+
+    from sandyrt_amd import ops
+
+    def constant(v):
+        return ops._nodes([ops.ScalarNode(0, ops.CONST, constant=v)])[0].constant
+
+    for v, want in ((False, 0.0), (True, 1.0), (0, 0.0), (np.float32(0.0), 0.0), (np.float32(1.5), 1.5),
+                    (np.array(2.5), 2.5), (torch.tensor(0.0), 0.0), (float("inf"), float("inf"))):
+        assert constant(v) == want
+    assert constant(float("nan")) != constant(float("nan"))
+    t = torch.tensor(2.0)
+    assert constant(t) == 2.0
+    t.fill_(3.0)
+    assert constant(t) == 3.0
+    assert ops._nodes([ops.ScalarNode(0, 2 ** 31 + 5)])[0].op == 5 - 2 ** 31
+    assert ops._nodes([ops.ScalarNode(0, -1)])[0].op == -1
