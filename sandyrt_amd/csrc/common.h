@@ -110,8 +110,9 @@ uint32_t* device_error_word(Err e, int* status);
 constexpr int kPagedStageSlot0 = 8;
 
 // Per-device, per-purpose grow-only scratch.  The returned memory stays valid
-// until the next call with the same slot and a larger size; callers that
-// need zeroed memory keep it zero themselves.
+// until the next call with the same slot and a larger size, and as long as the
+// process where `stream` is being captured (the graph's replays use it);
+// callers that need zeroed memory keep it zero themselves.
 void* device_workspace(int slot, size_t bytes, hipStream_t stream, Err e, int* status);
 
 // Zero-initialised per-device counters; zeroed when (re)allocated, kept zero

@@ -16,12 +16,15 @@ namespace {
 constexpr int kMaxDevices = 64;
 constexpr int kSlots = kPagedStageSlot0 + SANDY_HIP_PAGED_STAGE_SLOTS;
 
+struct Buffer {
+    void* p = nullptr;
+    size_t bytes = 0;
+    bool in_graph = false;  // its address was given to work under capture
+};
+
 struct DeviceState {
     uint32_t* error_word = nullptr;
-    void* ws[kSlots] = {};
-    size_t ws_bytes[kSlots] = {};
-    void* ctr[kSlots] = {};
-    size_t ctr_bytes[kSlots] = {};
+    Buffer ws[kSlots], ctr[kSlots];
 };
 
 std::mutex g_mu;
@@ -38,6 +41,23 @@ int current_device(Err e, int* dev) {
     if (st != hipSuccess) return fail(e, SANDY_ERR_HIP, "hipGetDevice: %s", hipGetErrorString(st));
     if (*dev < 0 || *dev >= kMaxDevices) return fail(e, SANDY_ERR_HIP, "device ordinal %d out of range", *dev);
     return SANDY_OK;
+}
+
+bool capturing(hipStream_t stream) {
+    if (!stream) return false;  // the legacy stream is never captured
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
+// An outgrown buffer is freed once the work on it is done -- unless a captured graph
+// holds its address: a replay still uses it, so it stays until the process ends (each
+// is at most 0.8 of the next, all of a slot together under five times its last).
+void outgrow(Buffer& b) {
+    if (b.p && !b.in_graph) {
+        hipDeviceSynchronize();  // earlier work on any stream may still use it
+        hipFree(b.p);
+    }
+    b = Buffer{};
 }
 
 } // namespace
@@ -66,25 +86,20 @@ void* device_workspace(int slot, size_t bytes, hipStream_t stream, Err e, int* s
     if (*status) return nullptr;
     if (bytes == 0) bytes = 256;
     std::lock_guard<std::mutex> lock(g_mu);
-    DeviceState& s = g_dev[dev];
-    if (s.ws_bytes[slot] < bytes) {
-        if (s.ws[slot]) {
-            // earlier work on any stream may still read the old buffer
-            hipDeviceSynchronize();
-            hipFree(s.ws[slot]);
-            s.ws[slot] = nullptr;
-            s.ws_bytes[slot] = 0;
-        }
+    Buffer& w = g_dev[dev].ws[slot];
+    if (w.bytes < bytes) {
+        outgrow(w);
         size_t grown = bytes + bytes / 4;
-        hipError_t st = hipMalloc(&s.ws[slot], grown);
+        hipError_t st = hipMalloc(&w.p, grown);
         if (st != hipSuccess) {
+            w.p = nullptr;
             *status = fail(e, SANDY_ERR_HIP, "workspace allocation of %zu bytes: %s", grown, hipGetErrorString(st));
             return nullptr;
         }
-        s.ws_bytes[slot] = grown;
+        w.bytes = grown;
     }
-    (void)stream;
-    return s.ws[slot];
+    w.in_graph = w.in_graph || capturing(stream);
+    return w.p;
 }
 
 void* device_counters(int slot, size_t bytes, hipStream_t stream, Err e, int* status) {
@@ -93,28 +108,22 @@ void* device_counters(int slot, size_t bytes, hipStream_t stream, Err e, int* st
     if (*status) return nullptr;
     if (bytes == 0) bytes = 256;
     std::lock_guard<std::mutex> lock(g_mu);
-    DeviceState& s = g_dev[dev];
-    if (s.ctr_bytes[slot] < bytes) {
-        if (s.ctr[slot]) {
-            hipDeviceSynchronize();
-            hipFree(s.ctr[slot]);
-            s.ctr[slot] = nullptr;
-            s.ctr_bytes[slot] = 0;
-        }
-        // enough for the tiles of any usual split product at once: a later, larger
-        // one that grew the buffer would free what a captured graph still counts in
+    Buffer& c = g_dev[dev].ctr[slot];
+    if (c.bytes < bytes) {
+        outgrow(c);
+        // the tiles of any usual split product at once: growing waits for the device
         size_t grown = std::max<size_t>(bytes + bytes / 4, 64 * 1024);
-        hipError_t st = hipMalloc(&s.ctr[slot], grown);
-        if (st == hipSuccess) st = hipMemset(s.ctr[slot], 0, grown);
+        hipError_t st = hipMalloc(&c.p, grown);
+        if (st == hipSuccess) st = hipMemset(c.p, 0, grown);
         if (st == hipSuccess) st = hipDeviceSynchronize();
         if (st != hipSuccess) {
             *status = fail(e, SANDY_ERR_HIP, "counter allocation of %zu bytes: %s", grown, hipGetErrorString(st));
             return nullptr;
         }
-        s.ctr_bytes[slot] = grown;
+        c.bytes = grown;
     }
-    (void)stream;
-    return s.ctr[slot];
+    c.in_graph = c.in_graph || capturing(stream);
+    return c.p;
 }
 
 } // namespace sandy_hip

@@ -215,6 +215,32 @@ def test_matmul_bf16_split_counters_rearm(ops, oracle):
         assert_close(got, oracle.matmul(to_oracle(L), to_oracle(W), transpose_rhs=True), torch.bfloat16, "rearm")
 
 
+def test_captured_split_product_survives_a_larger_one(ops):
+    """A graph of a split product (fp32 partials and arrival counters in
+    workspaces) is replayed after a far larger product has outgrown both
+    buffers and their size has been allocated and filled anew."""
+    m, n, k = 16, 2048, 10240
+    x, w = (from_f32(normal(rng(s), (r, k), 0.1), torch.bfloat16) for s, r in ((1, m), (2, n)))
+    want = ops.matmul(x, w, transpose_rhs=True)
+    out, s = torch.empty_like(want), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        ops.matmul(x, w, transpose_rhs=True, out=out)
+    for rows, cols in ((64, 16384), (64, 65536)):  # 21 MB, then 84 MB of partials, 512 and 2048 tiles
+        big = torch.full((cols, k), 2.0 ** -7, dtype=torch.bfloat16, device="cuda")
+        got = ops.matmul(torch.ones(rows, k, dtype=torch.bfloat16, device="cuda"), big, transpose_rhs=True)
+        assert torch.all(got == 80.0)
+        fill = [torch.full((b,), 255, dtype=torch.uint8, device="cuda") for b in (64 << 10, 2 << 20, 4 << 20, 32 << 20)]
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want)
+        assert all(torch.all(f == 255) for f in fill)
+        assert torch.equal(ops.matmul(x, w, transpose_rhs=True), want)
+
+
 def test_matmul_bf16_mfma_batched_grouped_heads(ops, oracle):
     """Batched [n, k] rhs with grouped-head broadcast on the MFMA kernel."""
     r = rng(12)
