@@ -3,6 +3,8 @@
 #pragma once
 #include "common.h"
 
+#include <type_traits>
+
 namespace sandy_hip {
 
 // Prefill-sized products: workgroup tile 64 WM x 64 WN of rows x columns,
@@ -32,7 +34,8 @@ struct TileGeo {
 
 // One tile: rows x [xrows, K] times the weight rows w [wrows, K], both packed with
 // K % 32 == 0 and 16-byte aligned, into out (rows `pitch` apart), plus bias [wrows]
-// if given; 1 <= xrows <= BM, 1 <= wrows <= BN.  PART: a wave whose rows all lie past
+// if given; 1 <= xrows <= BM, 1 <= wrows <= BN, and wrows is BN or ends the rows of
+// `out`, so that it divides by what `pitch` divides by.  PART: a wave whose rows all lie past
 // xrows multiplies nothing.
 template <int WM, int WN, int KS, bool PART>
 __device__ __forceinline__ void gemm_tile(unsigned char* lds, const uint16_t* x, int xrows, const uint16_t* w, int wrows,
@@ -52,10 +55,18 @@ __device__ __forceinline__ void gemm_tile(unsigned char* lds, const uint16_t* x,
     // buffer resources over the tile's rows: the lane's offsets stay put, the chunk's is
     // scalar (no address arithmetic a load), rows past the operand's end read as zero
     const int prow = tid >> 3, ppc = tid & 7;
+    // (the resources pinned to scalar registers: left to itself the compiler may compute
+    // them on the vector side and loop over the lanes at every load)
+    auto uniform = [](const uint16_t* p) {
+        const uint64_t v = reinterpret_cast<uint64_t>(p);
+        const uint64_t lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
+        const uint64_t hi = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v >> 32)));
+        return reinterpret_cast<uint16_t*>(hi << 32 | lo);
+    };
     const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(x), 0, static_cast<int>(xrows * K * 2), 0x00020000);
+        uniform(x), 0, __builtin_amdgcn_readfirstlane(static_cast<int>(xrows * K * 2)), 0x00020000);
     const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(w), 0, static_cast<int>(wrows * K * 2), 0x00020000);
+        uniform(w), 0, __builtin_amdgcn_readfirstlane(static_cast<int>(wrows * K * 2)), 0x00020000);
     int xo[G_::XP], wo[G_::WP];
 #pragma unroll
     for (int i = 0; i < G_::XP; i++) xo[i] = static_cast<int>((prow + 32 * i) * K * 2) + 16 * ppc;
@@ -191,20 +202,40 @@ __device__ __forceinline__ void gemm_tile(unsigned char* lds, const uint16_t* x,
                                pack_bf16x2(acc[t][c][4 * q + 2] + bv[2], acc[t][c][4 * q + 3] + bv[3]));
         }
     __builtin_amdgcn_wave_barrier();
-    constexpr int kLanes = 4 * WN;  // lanes per row, 8 columns each
-    const bool wide = (pitch & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+    if ((pitch & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
+        constexpr int kLanes = 4 * WN;  // lanes per row, 8 columns each
 #pragma unroll
-    for (int i = 0; i < 32 * WM * kLanes / 64; i++) {
-        const int r = (64 * i + lane) / kLanes, c8 = 8 * ((64 * i + lane) % kLanes);
-        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ot + r * G_::kRowPitch + 2 * c8);
-        if (mw + r >= xrows || nw + c8 >= wrows) continue;
-        uint16_t* to = out + (mw + r) * pitch + nw + c8;
-        if (wide) {
-            *reinterpret_cast<u32x4_t*>(to) = v;
-        } else {
-            for (int j = 0; j < 8 && nw + c8 + j < wrows; j++) to[j] = static_cast<uint16_t>(v[j >> 1] >> (16 * (j & 1)));
+        for (int i = 0; i < 32 * WM * kLanes / 64; i++) {
+            const int r = (64 * i + lane) / kLanes, c8 = 8 * ((64 * i + lane) % kLanes);
+            const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ot + r * G_::kRowPitch + 2 * c8);
+            if (mw + r >= xrows || nw + c8 >= wrows) continue;
+            *reinterpret_cast<u32x4_t*>(out + (mw + r) * pitch + nw + c8) = v;
         }
+        return;
     }
+    // rows of other alignments: two columns a lane or one, so that neighbouring lanes
+    // still write neighbouring columns (eight two-byte stores a lane, 16 bytes apart, took
+    // 116 us for 2191 x 29614 x 32 where this takes 54; 946 x 13341 x 512 46 -> 37)
+    auto put_rows = [&](auto width) {
+        constexpr int W = decltype(width)::value, kLanes = 32 * WN / W;
+        using Piece = std::conditional_t<W == 2, uint32_t, uint16_t>;
+#pragma unroll 1
+        for (int i0 = 0; i0 < 32 * WM * kLanes / 64; i0 += 8) {
+            Piece v[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const int at = 64 * (i0 + i) + lane;
+                v[i] = *reinterpret_cast<const Piece*>(ot + at / kLanes * G_::kRowPitch + 2 * W * (at % kLanes));
+            }
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const int at = 64 * (i0 + i) + lane, r = mw + at / kLanes, c = nw + W * (at % kLanes);
+                if (r < xrows && c < wrows) *reinterpret_cast<Piece*>(out + r * pitch + c) = v[i];
+            }
+        }
+    };
+    if ((pitch & 1) == 0 && (reinterpret_cast<uintptr_t>(out) & 3) == 0) put_rows(std::integral_constant<int, 2>{});
+    else put_rows(std::integral_constant<int, 1>{});
 }
 
 } // namespace sandy_hip
