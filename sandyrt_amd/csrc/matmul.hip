@@ -559,28 +559,34 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
         g.K = p.K;
         g.bm = p.bm;
         // The tile form with the least estimated time: its chunks of 64 k (over its
-        // KS groups) times the time of one, `alone` up to one workgroup a CU, else
-        // `each` for every workgroup of the fullest CU (measured, us).  Cold
-        // operands, 64 x 256 tiles before -> the form taken (us): 2048 x 11264 x
-        // 2048 163 -> 99 (128 x 192 tiles, 960 TFLOP/s), 2040 x 2048 x 5632 -> 57
-        // (128 x 128, two K groups), 2048 x 2048 x 2048 39 -> 24 (128 x 64), 1000 x
-        // 2048 x 5632 93 -> 33 (128 x 64, two groups), 333 x 2048 x 5632 93 -> 22
-        // (64 x 64, two groups), 100 x 520 x 224 9.0 -> 4.2 (the same).
+        // KS groups) times the time of one plus the tile's own (first loads, output),
+        // `alone` up to one workgroup a CU, else `each` for every workgroup of the
+        // fullest CU (measured, us).  Cold operands, 64 x 256 tiles before -> the form
+        // taken (us): 2048 x 11264 x 2048 163 -> 99 (128 x 192 tiles, 960 TFLOP/s),
+        // 2040 x 2048 x 5632 -> 57 (128 x 128, two K groups), 2048 x 2048 x 2048 39 ->
+        // 24 (128 x 64), 1000 x 2048 x 5632 93 -> 33 (128 x 64, two groups), 333 x 2048
+        // x 5632 93 -> 22 (64 x 64, two groups).  Without the tile's own time short
+        // contractions got too wide tiles, and 64 x 64 of one group suits the smallest
+        // (us, 64 x 256 tiles / that rule / here): 915 x 7338 x 224 16.1 / 17.3 / 13.6,
+        // 946 x 13341 x 512 42 / 37 / 28, 300 products of 80 x 80 x 32 13.5 / 16.6 /
+        // 13.0, 434 x 2385 x 96 - / 7.2 / 6.0.
         struct Form {
             int bm, bn, groups;
-            double alone, each;
+            double alone, each, alone_tile, each_tile;
         };
-        static const Form kForms[] = {{128, 192, 1, 0.75, 0.78}, {128, 64, 1, 0.41, 0.36}, {128, 128, 2, 1.2, 1.4},
-                                      {128, 64, 2, 0.72, 0.8}, {64, 64, 2, 0.5, 0.5}};
+        static const Form kForms[] = {{128, 192, 1, 0.75, 0.78, 2.5, 1.5}, {128, 64, 1, 0.41, 0.36, 0.5, 0.3},
+                                      {128, 128, 2, 1.2, 1.4, 2.0, 1.2},   {128, 64, 2, 0.72, 0.8, 0.9, 1.5},
+                                      {64, 64, 2, 0.5, 0.5, 0.5, 0.5},     {64, 64, 1, 0.27, 0.25, 0.25, 0.05}};
         const int64_t chunks = (p.K + 63) / 64;
         int form = 0;
         double best = 0.0;
-        for (int i = 0; i < 5; i++) {
+        for (int i = 0; i < 6; i++) {
             const Form& f = kForms[i];
             const double tiles = static_cast<double>((p.M + f.bm - 1) / f.bm) * static_cast<double>((p.N + f.bn - 1) / f.bn) *
                                  static_cast<double>(p.batches);
-            const double us = static_cast<double>((chunks + f.groups - 1) / f.groups) *
-                              (tiles <= 256.0 ? f.alone : std::ceil(tiles / 256.0) * f.each);
+            const double steps = static_cast<double>((chunks + f.groups - 1) / f.groups);
+            const double us = tiles <= 256.0 ? steps * f.alone + f.alone_tile
+                                             : std::ceil(tiles / 256.0) * (steps * f.each + f.each_tile);
             if (i == 0 || us < best) {
                 best = us;
                 form = i;
@@ -607,6 +613,7 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
             case 1: st = go(TileGeo<2, 1, 1>{}, gemm_tile_kernel<2, 1, 1>); break;
             case 2: st = go(TileGeo<2, 2, 2>{}, gemm_tile_kernel<2, 2, 2>); break;
             case 3: st = go(TileGeo<2, 1, 2>{}, gemm_tile_kernel<2, 1, 2>); break;
+            case 5: st = go(TileGeo<1, 1, 1>{}, gemm_tile_kernel<1, 1, 1>); break;
             default: st = go(TileGeo<1, 1, 2>{}, gemm_tile_kernel<1, 1, 2>); break;
         }
         if (st) return st;

@@ -300,7 +300,7 @@ def test_linear_f32_ordered_tiles_bit_exact(ops, oracle, rows_a_lane, rows, in_f
     assert_equal(got3, oracle.matmul(to_oracle(x3), to_oracle(w.unsqueeze(0)), transpose_rhs=True), "batched matmul")
 
 
-@pytest.mark.parametrize("form", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("form", [0, 1, 2, 3, 4, 5])
 @pytest.mark.parametrize("m,n,k", [(65, 8, 32), (70, 301, 64), (129, 194, 96), (192, 65, 160), (257, 200, 2080)])
 def test_matmul_bf16_prefill_tiles(ops, oracle, form, m, n, k):
     """Every tile form of the prefill GEMM: ragged rows and columns (odd n:
