@@ -359,7 +359,13 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
     if (fz && p.batches != 1) return fail(e, SANDY_ERR_UNSUPPORTED, "%s takes one [m, k] matrix", what);
     const bool norm = fz && fz->norm_w;
     // f32 against a weight read as [n, k], in the reference's k order
-    const bool ordered = l.dtype == SANDY_F32 && !tl && tr && p.K % 4 == 0 && p.K > 0 && aligned &&
+    // (short contractions with many outputs: the 64 x 64 tiles of gemm_simt_kernel, in the
+    // same order, reread the operands less and fill whole store lines.  us, ordered / simt:
+    // 1000 x 16000 x 16 49 / 26, 1000 x 4000 x 48 21 / 17, 2000 x 8000 x 96 105 / 97,
+    // 1461 x 8606 x 20 44 / 32; k 128 even, 2000 x 8000 x 256 233 / 245; 1000 x 1000 x 24
+    // 7.3 / 8.4)
+    const bool short_wide = p.M > 8 && p.M <= 65535 * 64 && p.K <= 96 && p.M * p.N * p.batches >= (2 << 20);
+    const bool ordered = l.dtype == SANDY_F32 && !tl && tr && p.K % 4 == 0 && p.K > 0 && aligned && !short_wide &&
                          env_int("SANDY_GEMM_SIMT", 0) == 0;
     if (ordered) {
         // one row a lane while that takes at most two waves a SIMD, else four

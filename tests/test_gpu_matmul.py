@@ -300,6 +300,15 @@ def test_linear_f32_ordered_tiles_bit_exact(ops, oracle, rows_a_lane, rows, in_f
     assert_equal(got3, oracle.matmul(to_oracle(x3), to_oracle(w.unsqueeze(0)), transpose_rhs=True), "batched matmul")
 
 
+@pytest.mark.parametrize("rows,in_f,out_f", [(8, 4, 262144), (9, 4, 233017), (128, 96, 16384), (128, 100, 16384)])
+def test_linear_f32_short_contractions_bit_exact(ops, oracle, rows, in_f, out_f):
+    """Both sides of the line between the ordered kernel and the 64 x 64 tiles."""
+    r = rng(rows + in_f)
+    x, w = (from_f32(normal(r, (n, in_f)), torch.float32) for n in (rows, out_f))
+    b = from_f32(normal(r, (out_f,)), torch.float32)
+    assert_equal(ops.linear(x, w, b), oracle.linear(to_oracle(x), to_oracle(w), to_oracle(b)), "linear")
+
+
 @pytest.mark.parametrize("form", [0, 1, 2, 3, 4, 5])
 @pytest.mark.parametrize("m,n,k", [(65, 8, 32), (70, 301, 64), (129, 194, 96), (192, 65, 160), (257, 200, 2080)])
 def test_matmul_bf16_prefill_tiles(ops, oracle, form, m, n, k):
