@@ -441,7 +441,9 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
             //     30.6 / 32.4 -> 23.1 / 24.7); past it 64 x 32, so that the weights
             //     stream once (32000 x 2048 43.7 / 44.5 -> 33.3 / 36.3, 14336 x 4096
             //     52.0 / 54.2 -> 45.9 / 49.3; the prologue's work would grow with the
-            //     rows);
+            //     rows) -- up to k 4096: with more, and so more splits of K, it loses
+            //     (42 x 7616 x 6368 55 against 62, 45 x 14578 x 5408 71 against 76; with
+            //     the prologue 33 x 4512 x 5536 41 against 43) and that rule stays;
             //   4 chunks in flight per wave for weights under 8M elements
             //   (o projection at 32 rows 8.3 -> 6.1 us, q/k/v at one row
             //   7.4 -> 5.5 us), 2 for the larger ones;
@@ -451,6 +453,7 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
             //   12.8 -> 11.6 us, one row 9.2 -> 8.7 us).
             const bool big = p.N * p.K * 2 > (int64_t(64) << 20);
             constexpr int64_t kSmall = 6 << 20, kMiddle = 20 << 20;  // weight elements
+            const bool long_big = p.K > 4096 && (big || (norm && p.N * p.K > kMiddle));
             int64_t rt = 1, ct = 1;
             if (p.M <= 16 && !big) {
                 ct = p.N >= 16384 ? 2 : 1;
@@ -472,7 +475,7 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
                     ksplits = (chunks + 47) / 48;
                     qdepth = 4;
                 }
-            } else if (p.M > 32 && p.batches == 1 && !qkv && (!norm || (!big && (p.N * p.K < kSmall || p.N * p.K > kMiddle)))) {
+            } else if (p.M > 32 && p.batches == 1 && !qkv && !long_big && (!norm || (!big && (p.N * p.K < kSmall || p.N * p.K > kMiddle)))) {
                 rt = p.N * p.K < kSmall ? 1 : big ? 4 : 2;
                 ct = p.N * p.K <= kMiddle ? 1 : 2;
                 qdepth = p.N * p.K < kSmall ? 4 : 2;
