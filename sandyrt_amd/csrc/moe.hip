@@ -1659,13 +1659,18 @@ extern "C" int sandy_hip_moe_gather(const SandyTensor* x, const SandyTensor* top
     const int64_t row_bytes = hidden * static_cast<int64_t>(dtype_size(x->dtype));
     const int aligned = (row_bytes % 16 == 0) &&
                         ((reinterpret_cast<uintptr_t>(base_ptr(*x)) | reinterpret_cast<uintptr_t>(base_ptr(*packed_x))) & 15) == 0;
+    // token-major: about 256 workgroups of ceil(seq / 256) tokens (at most 64 routes each)
+    const int64_t tpw = std::max<int64_t>(1, std::min<int64_t>(64 / std::max<int64_t>(1, top_k), (seq + 255) / 256));
+    const int64_t wgs = (seq + tpw - 1) / tpw;
     // the one-workgroup ranking and row copy below took 167 us for 16384 routes of 8 a
-    // token where this form's workgroups, each reading every id, take 34
-    if (routes <= kTokenRoutes && batch <= 65535 && aligned && top_k <= 64 && 2 * num_experts + 64 <= 16384 &&
+    // token where this form's workgroups, each reading every id, take 34; but those of
+    // several sequences queue up while the ranking runs one workgroup a sequence (us, here
+    // / ranking: 60000 routes of 1 a token, 938 workgroups a sequence, 3 sequences 172 /
+    // 262, 6 325 / 294, 64 3274 / 1044; 64000 of 8, 1000 workgroups, 3 210 / 533, 16 1030 /
+    // 682; 16384 of 4, 256 workgroups, 8 94 / 100, 12 133 / 125)
+    const bool ranked = routes > kDispatchRoutes && batch * wgs > 3000;
+    if (routes <= kTokenRoutes && !ranked && batch <= 65535 && aligned && top_k <= 64 && 2 * num_experts + 64 <= 16384 &&
         env_int("SANDY_MOE_ROUTE_GENERAL", 0) == 0) {
-        // token-major: about 256 workgroups of ceil(seq / 256) tokens (at most 64 routes each)
-        const int64_t tpw = std::max<int64_t>(1, std::min<int64_t>(64 / top_k, (seq + 255) / 256));
-        const int64_t wgs = (seq + tpw - 1) / tpw;
         if (wgs > 0x7fffffff) return fail(e, SANDY_ERR_UNSUPPORTED, "moe_gather too many tokens");
         const size_t shb = static_cast<size_t>(2 * num_experts + 64) * sizeof(int32_t);
         dim3 grid(static_cast<unsigned>(wgs), static_cast<unsigned>(batch));
@@ -1812,8 +1817,12 @@ extern "C" int sandy_hip_moe_matmul(const SandyTensor* x, const SandyTensor* exp
         // (gate / down of the 128-expert block, us, one chunk in flight -> here: 8
         // rows 46 / 19 -> 10 / 9, 40 rows 50 / 42 -> 28 / 30, 64 rows 52 / 47 ->
         // 40 / 44; 96 rows 55 / 56 against 61 / 62).  Up to 16 rows a long
-        // contraction is split over the waves (8 rows 18 -> 10; 40 rows 28 -> 31)
-        const int stream_form = env_int("SANDY_MOE_STREAM", rows * 2 > experts ? 0 : rows <= 16 && K >= 1536 ? 2 : 1);
+        // contraction is split over the waves (8 rows 18 -> 10; 40 rows 28 -> 31).
+        // Short contractions have too few chunks to keep in flight: k 64 4.3 / 5.1 (3
+        // sequences, 128 experts x 3703 x 192, 60 rows 49 / 68), k 512 13.7 / 7.2 for 4
+        // rows of 64 experts x 1577 and 18.5 / 20.3 for 60 of 200 x 1483
+        const bool few = rows * 2 <= experts && (K >= 640 || (K >= 512 && rows * 4 <= experts)) && M <= 65535 * 32;
+        const int stream_form = env_int("SANDY_MOE_STREAM", !few ? 0 : rows <= 16 && K >= 1536 ? 2 : 1);
         if (stream_form) {
             const int64_t slots = std::min(rows, experts);  // at most `rows` experts have a row
             const int64_t cols = stream_form == 2 ? 32 : 64;
@@ -1831,11 +1840,17 @@ extern "C" int sandy_hip_moe_matmul(const SandyTensor* x, const SandyTensor* exp
         // -> 106 / 117, 128 rows 241 / 285 -> 157 / 148, 256 rows 428 / 512 -> 201 /
         // 214; 37 rows 81 / 100 against 98 / 109).  64 x 192 tiles 132 / 129 at 64
         // rows, 170 / 175 at 128; 128 x 128 tiles 122 / 129 and 154 / 157.
+        // A tile's first loads and its output weigh more the shorter the contraction, and
+        // several sequences fill the chip with either kernel: the line moves up (there /
+        // here: k 1408, 3 sequences x 64 experts x 3436 at 50 rows 348 / 402, at 62 rows
+        // 32 x 2816 201 / 125; k 512, 16 x 1028 at 45 12.5 / 14.6, 128 x 704 at 68 38 /
+        // 25; k 192, 8 x 751 at 173 17.6 / 19.8; k 64, 200 x 366 at 82 11.7 / 15.0)
+        const int64_t tile_rows = K >= 640 ? (batch == 1 ? 44 : 56) : K >= 512 ? 64 : K >= 256 ? 128 : rows;
         using Tile = TileGeo<2, 3, 1>;
         const int64_t col_tiles = (M + Tile::BN - 1) / Tile::BN;
         // row tiles of all experts together: whole ones, and one partial one each
         const int64_t tiles = (rows / Tile::BM + std::min(rows, experts)) * col_tiles;
-        if (env_int("SANDY_MOE_TILE", rows > 44 * experts) && rows <= 0x7fffffff && batch <= 65535 && K <= (1 << 22) &&
+        if (env_int("SANDY_MOE_TILE", rows > tile_rows * experts) && rows <= 0x7fffffff && batch <= 65535 && K <= (1 << 22) &&
             tiles <= (1 << 30)) {
             SANDY_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(moe_gemm_tile_kernel<2, 3, 1>),
                                               hipFuncAttributeMaxDynamicSharedMemorySize, Tile::kBytes), e, "moe_matmul");

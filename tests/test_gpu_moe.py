@@ -181,6 +181,21 @@ def test_moe_gather_long(ops, oracle, T, E, K, idx):
     assert_equal(off, np.concatenate([[0], np.cumsum(counts)]).astype(np.int64), "expert_offsets")
 
 
+@pytest.mark.parametrize("B", [11, 12])
+def test_moe_gather_long_batched(ops, oracle, B):
+    """Long route lists of several sequences: in one launch up to 3000 workgroups
+    together (11 x 257), ranked one workgroup a sequence past it."""
+    r = rng(B)
+    T, E, K = 4100, 9, 4
+    ids = r.integers(0, E, (B, T, K)).astype(np.int64)
+    x = from_f32(normal(r, (B, T, 8)), torch.bfloat16)
+    w = from_f32(np.abs(normal(r, (B, T, K))), torch.bfloat16)
+    got = ops.moe_gather(x, torch.from_numpy(ids).cuda(), w, E)
+    want = oracle.moe_gather(to_oracle(x), ids, to_oracle(w), E)
+    for g, wnt, name in zip(got, want, ["packed_x", "packed_weights", "token_ids", "offsets"]):
+        assert_equal(g, wnt, name)
+
+
 def test_moe_gather_batched_and_skewed(ops, oracle):
     """Rank-3 inputs, and routes concentrated on few experts (long same-expert
     runs inside a wave exercise the ballot ranking)."""
@@ -351,6 +366,20 @@ def test_moe_matmul_many_rows(ops, oracle, monkeypatch, counts, M, K):
     offs = np.stack([np.concatenate([[0], np.cumsum(c)]).astype(np.int64) for c in (counts, counts[::-1])])
     x = from_f32(normal(r, (2, rows, K)), torch.bfloat16)
     w = from_f32(normal(r, (E, M, K), 0.1), torch.bfloat16)
+    got = ops.moe_matmul(x, torch.from_numpy(offs).cuda(), w, True)
+    ops.check_device_errors()
+    assert_close(got, oracle.moe_matmul(to_oracle(x), offs, to_oracle(w), True), torch.bfloat16, "moe_matmul")
+
+
+@pytest.mark.parametrize("B,rows,K", [(1, 88, 640), (1, 90, 640), (2, 112, 640), (2, 114, 640), (1, 128, 608), (1, 130, 608),
+                                      (1, 258, 256), (1, 300, 224), (1, 1, 608), (1, 1, 640), (2, 1, 480)])
+def test_moe_matmul_kernel_choice_edges(ops, oracle, B, rows, K):
+    """Both sides of the lines at which the kernel for an expert's rows changes
+    (2 experts; contraction length, rows an expert, sequences)."""
+    r = rng(rows + K)
+    offs = np.stack([np.array([0, rows // 2 + b, rows]) for b in range(B)]).astype(np.int64)
+    x = from_f32(normal(r, (B, rows, K)), torch.bfloat16)
+    w = from_f32(normal(r, (2, 70, K), 0.1), torch.bfloat16)
     got = ops.moe_matmul(x, torch.from_numpy(offs).cuda(), w, True)
     ops.check_device_errors()
     assert_close(got, oracle.moe_matmul(to_oracle(x), offs, to_oracle(w), True), torch.bfloat16, "moe_matmul")
