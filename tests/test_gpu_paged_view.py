@@ -71,7 +71,18 @@ def test_f32_decode_general_kernel(ops, oracle):
     run(ops, oracle, 5, 3, 4, 2, 64, 8, 300, 1, torch.float32)
 
 
-def test_prefill_over_pages_general_kernel(ops, oracle):
+@pytest.mark.parametrize("D,unstaged", [(64, False), (64, True), (96, False), (96, True)])
+def test_prefill_over_pages_general_kernel(ops, oracle, monkeypatch, D, unstaged):
+    """Both forms of the general kernel over pages with several queries: at a
+    head dim that the MFMA prefill kernel does not take, and at one that it
+    does with that kernel switched off."""
+    monkeypatch.setenv("SANDY_PREFILL_GENERAL", "1")
+    if unstaged:
+        monkeypatch.setenv("SANDY_ATTN_UNSTAGED", "1")
+    run(ops, oracle, 6, 2, 8, 2, D, 16, 200, 5, torch.bfloat16)
+
+
+def test_prefill_over_pages(ops, oracle):
     run(ops, oracle, 6, 2, 8, 2, 64, 16, 200, 5, torch.bfloat16)
 
 
@@ -93,13 +104,17 @@ def test_paged_view_errors(ops):
 
 @pytest.mark.parametrize("dtype,tq,D,unstaged", [(torch.float32, 1, 64, False), (torch.bfloat16, 5, 64, False),
                                                  (torch.bfloat16, 1, 64, False), (torch.bfloat16, 1, 96, False),
-                                                 (torch.float32, 1, 64, True), (torch.bfloat16, 5, 64, True)])
+                                                 (torch.float32, 1, 64, True), (torch.bfloat16, 5, 96, False),
+                                                 (torch.bfloat16, 5, 96, True)])
 def test_null_page_is_a_device_error(ops, monkeypatch, dtype, tq, D, unstaged):
     """A page-table entry of 0 inside the attended range is reported as a
-    device error by every kernel that reads the view (f32 decode and prefill
-    through the general kernels, bf16 decode through the MFMA kernel, a head
-    dim the MFMA kernel does not take), and nothing is read from address 0."""
+    device error by every kernel that reads the view (bf16 decode and prompts
+    through the MFMA kernels, f32 decode and a head dim that those do not take
+    through the general kernel, in both its forms), and nothing is read from
+    address 0."""
     from sandyrt_amd._lib import SandyError
+    if unstaged:
+        monkeypatch.setenv("SANDY_ATTN_UNSTAGED", "1")
     r = rng(11)
     kv, _, keep_k = make_view(ops, r, [2, 2], 40, D, 16, dtype)
     vv, _, keep_v = make_view(ops, r, [2, 2], 40, D, 16, dtype)

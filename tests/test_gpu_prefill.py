@@ -31,7 +31,7 @@ def pages_of(ops, t, P, shift=0):
     return ops.PagedView(torch.tensor(at, dtype=torch.int64, device="cuda"), t.shape, P, t.dtype), keep
 
 
-def check(ops, oracle, dtype, B, hq, hkv, tq, tk, D, pos, window, P=0, shift=0, spoil=None, heads_inner=False):
+def check(ops, oracle, dtype, B, hq, hkv, tq, tk, D, pos, window, P=0, shift=0, spoil=None, heads_inner=False, kv_room=0):
     r = rng(tq * 131 + tk + D + window)
     q = from_f32(normal(r, (B, hq, tq, D), 0.5), dtype)
     if heads_inner:  # the engine's [B, T, H, D] rows seen as [B, H, T, D]
@@ -40,6 +40,10 @@ def check(ops, oracle, dtype, B, hq, hkv, tq, tk, D, pos, window, P=0, shift=0, 
     v = from_f32(normal(r, (B, hkv, tk, D)), dtype)
     if spoil:
         spoil(k, v)
+    if kv_room:  # views of [B, T + room, Hkv, D] caches: the heads inside the tokens, keys past the last
+        k, v = (torch.cat([t, torch.full_like(t[:, :, :1], float("nan")).expand(-1, -1, kv_room, -1)], 2)
+                .permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3)[:, :, :tk] for t in (k, v))
+        assert not k.is_contiguous() and k.stride(2) == hkv * D
     p = torch.tensor(pos, device="cuda") if pos is not None else None
     want = oracle.attention(to_oracle(q.contiguous()), to_oracle(k), to_oracle(v),
                             np.array(pos, np.int64) if pos is not None else None, window, -1.0)
@@ -103,6 +107,28 @@ def test_prefill_strided_heads_and_pages(ops, oracle, shape, dtype):
     check(ops, oracle, dtype, heads_inner=True, **shape)
     for P, shift in ((1, 0), (16, 0), (64, 8), (16, 3)):
         check(ops, oracle, dtype, P=P, shift=shift, **shape)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape", [SHAPES[1], SHAPES[5], SHAPES[8]], ids=str)
+def test_prefill_strided_keys_and_values(ops, oracle, monkeypatch, shape, dtype):
+    """Dense K/V that are views of larger caches with the heads inside the
+    tokens; what lies past the keys is never used.  The general kernel takes
+    the same views."""
+    check(ops, oracle, dtype, kv_room=5, **shape)
+    monkeypatch.setenv("SANDY_PREFILL_GENERAL", "1")
+    check(ops, oracle, dtype, kv_room=5, **shape)
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.bfloat16, 256), (torch.float32, 64)])
+@pytest.mark.parametrize("rows", ["1", "2"])
+@pytest.mark.parametrize("tk,window", [(511, 0), (512, 0), (700, 0), (700, 300), (700, 600)])
+def test_prefill_long_page_lists(ops, oracle, monkeypatch, tk, window, rows, dtype, D):
+    """Pages of one key: 512 page addresses, the most that are held in LDS, and
+    more (read from memory per chunk), aligned ones too; a window that brings a
+    longer list under the line and one that does not."""
+    monkeypatch.setenv("SANDY_PREFILL_RW", rows)
+    check(ops, oracle, dtype, B=1, hq=4, hkv=2, tq=40, tk=tk, D=D, pos=[tk - 40], window=window, P=1)
 
 
 @pytest.mark.parametrize("rows", ["1", "2"])
