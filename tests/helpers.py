@@ -7,7 +7,7 @@ the pure relative bound for every element of at least FLOOR times the
 tensor's RMS, and for the elements below that (results of cancellation, where
 a relative bound measures only the rounding of the terms that cancelled) the
 same relative bound on FLOOR * rms.  FLOOR is 1/16 (SANDY_TEST_FLOOR
-overrides it).  Integer and index outputs are compared exactly.
+overrides it).  Infinities keep their sign and NaN is NaN.  Integer and index outputs are compared exactly.
 """
 from __future__ import annotations
 
@@ -67,11 +67,12 @@ def assert_close(got, want, dtype, what="", rtol=None, floor=None):
     assert g.shape == w.shape, f"{what}: shape {g.shape} != {w.shape}"
     rtol = rtol if rtol is not None else RTOL[dtype]
     finite = np.isfinite(w)
-    assert np.array_equal(np.isfinite(g), finite), f"{what}: non-finite pattern differs"
+    np.testing.assert_array_equal(g[~finite], w[~finite], err_msg=f"{what}: non-finite values")
+    assert np.isfinite(g[finite]).all(), f"{what}: non-finite where the reference is finite"
     if not finite.any():
         return
-    scale = float(np.sqrt(np.mean(w[finite] ** 2))) if finite.any() else 0.0
-    err = np.abs(g - w)
+    scale = float(np.sqrt(np.mean(w[finite] ** 2)))
+    err = np.abs(np.where(finite, g, 0.0) - np.where(finite, w, 0.0))
     bound = rtol * np.maximum(np.abs(w), (FLOOR if floor is None else floor) * scale)
     bad = finite & (err > bound)
     if bad.any():

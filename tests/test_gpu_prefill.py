@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from tests.helpers import as_f32, assert_close, from_f32, normal, rng, to_oracle
+from tests.helpers import assert_close, from_f32, normal, rng, to_oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -64,9 +64,6 @@ def check(ops, oracle, dtype, B, hq, hkv, tq, tk, D, pos, window, P=0, shift=0, 
         np.testing.assert_allclose(got, want, rtol=1e-5, atol=8 * 2.0 ** -24 * big, err_msg=what)
     else:
         assert_close(out.contiguous(), want, dtype, what)
-        got, want = as_f32(to_oracle(out.contiguous())), as_f32(np.asarray(want))
-        np.testing.assert_array_equal(np.isnan(got), np.isnan(want), err_msg=what)
-        np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)], err_msg=what)
 
 
 SHAPES = [
