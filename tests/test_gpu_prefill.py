@@ -216,3 +216,32 @@ def test_prefill_errors(ops):
     ops.attention_paged_view(q, view, view, torch.tensor([14], device="cuda"))
     with pytest.raises(SandyError, match="block id outside the pool"):
         ops.check_device_errors()
+
+
+@pytest.mark.parametrize("dtype,D,tq,past,spread", [
+    (torch.float32, 64, 2, 0, 1.0), (torch.float32, 128, 2, 0, 3.0), (torch.float32, 64, 64, 0, 1.0),
+    (torch.float32, 128, 5, 300, 1.0), (torch.bfloat16, 64, 64, 0, 1.0), (torch.bfloat16, 128, 40, 200, 1.0),
+    (torch.bfloat16, 256, 33, 100, 1.0)])
+def test_prefill_error_against_64_bits(ops, monkeypatch, dtype, D, tq, past, spread):
+    """No further from the exact outputs than the general kernel, over enough
+    rows for the difference to show: the 2-norm of the error in f32, in bf16
+    the share of outputs that are not the nearest value to the exact one."""
+    g = torch.Generator(device="cuda").manual_seed(D + tq + past)
+    B, tk = max(4, min(512, 6000 // (tq + past))), tq + past
+    q, k, v = (torch.randn(B, 12, n, D, generator=g, device="cuda") for n in (tq, tk, tk))
+    q, k, v = (q * spread).to(dtype), k.to(dtype), v.to(dtype)
+    pos = torch.full((B,), past, dtype=torch.int64, device="cuda")
+    s = q.double() @ k.double().transpose(2, 3).contiguous() / D ** 0.5
+    seen = torch.arange(tk, device="cuda") <= past + torch.arange(tq, device="cuda")[:, None]
+    want = torch.softmax(s.masked_fill(~seen, float("-inf")), -1) @ v.double()
+
+    def error():
+        out = ops.attention(q, k, v, pos)
+        if dtype == torch.float32:
+            return ((out.double() - want).norm() / want.norm()).item()
+        return (out != want.to(dtype)).double().mean().item()
+
+    here = error()
+    monkeypatch.setenv("SANDY_PREFILL_GENERAL", "1")
+    general = error()
+    assert here <= general, f"{here:.4e} against {general:.4e}"
