@@ -14,8 +14,9 @@
 //     scores of one query and the softmax needs one cross-lane exchange;
 //   - P^T leaves the product in the B-operand layout of O^T += V^T P^T, with
 //     V^T read by ds_read_b64_tr_b16 in the same key order;
-//   - P enters as two bf16 operands (hi + lo), about 17 bits of each
-//     probability; the row sums are kept in float64.
+//   - P enters as three bf16 operands that together are p exactly (two of them
+//     kept about 17 bits and were 17% faster at 2048 queries); the row sums are
+//     kept in float64.
 // f32 takes v_mfma_f32_32x32x2_f32 for both products (f32 operands throughout,
 // P straight from its registers) and expf; bound by that instruction's rate, a
 // sixteenth of the bf16 one's.
@@ -24,11 +25,15 @@
 // the chip; at D 256 a second wave per score tile owns half of the head dims.
 // Chunks of K and V go global -> registers -> LDS, double buffered where they
 // fit, one barrier each.
-// Bound: softmax VALU work (49% of the cycles at D 64, MFMA 22%).  Measured,
-// us a call (general kernel -> here): 2048 queries, 32 / 4 heads, D 64
-// 14357 -> 43; 777 queries after 1500 keys, window 1024, 8 / 2 heads, D 256,
-// pages of 16: 4896 -> 41; 1500 after 300, 16 / 2 heads, D 128: 49; f32, 12
-// heads, D 64: 1000 queries 1434 -> 43, 64 queries 23.5 -> 9.8.
+// Bound: softmax VALU work, the cutting of P included (52% of the cycles at D 64,
+// MFMA 26%).  Measured, us a call (general kernel -> here): 2048 queries, 32 / 4
+// heads, D 64 14357 -> 50; 777 queries after 1500 keys, window 1024, 8 / 2 heads,
+// D 256, pages of 16: 4896 -> 42; 1500 after 300, 16 / 2 heads, D 128: 48; f32, 12
+// heads, D 64: 1000 queries 1434 -> 43, 64 queries 23.5 -> 10.
+// Against 64 bits (2 to 130 queries after 0 to 2000 keys, scores of three spreads)
+// f32 outputs are off by 0.50 to 1.00 of the general kernel's error; of the bf16
+// ones that are not the nearest value there are 0.5 to 0.95 as many wherever there
+// are enough to count.
 #include "attention_prefill.h"
 #include "prefill_span.h"
 
@@ -610,10 +615,12 @@ int launch_dim(const PrefillArgs& a, hipStream_t stream, Err e) {
     const int64_t rows = static_cast<int64_t>(a.group) * a.tq;
     const int64_t heads = static_cast<int64_t>(a.batch) * a.hkv;
     // 64-row workgroups (two waves share the keys) where they nearly fill the 256
-    // CUs, else 32-row ones (four share them): 1024 workgroups of 64 rows 43 us
-    // against 94, 252 of them 11.5 against 13.4, 114 of them 36 against 32 (900
-    // queries, D 256).
-    // 128-row workgroups were slower at every size (2048 queries, D 64: 45 us).
+    // CUs, else 32-row ones (four share them).  us, 64 / 32 rows, by the number of
+    // 64-row workgroups: D 64 100 of them 10.8 / 11.1, 220 12.3 / 13.8, 300 15.4 /
+    // 20.5, 1024 50 / 100; D 128 100 15.7 / 13.7, 200 23.8 / 23.2, 226 25.6 / 26.3,
+    // 300 33 / 42; D 256 114 41 / 35, 200 64 / 56, 224 72 / 62 and with a window of
+    // 1024 54 / 80.  128-row workgroups were slower at every size (two operands of
+    // P, 2048 queries, D 64: 45 against 43).
     // f32: 192 workgroups of 64 rows 58 us, 384 of 32 rows 43.
     const int64_t wgs = (rows + 63) / 64 * heads;
     if (env_int("SANDY_PREFILL_RW", wgs >= 224 ? 2 : 1) == 2) return launch_form<T, D, 2, PAGED>(a, stream, e);

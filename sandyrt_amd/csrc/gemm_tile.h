@@ -17,7 +17,7 @@ namespace sandy_hip {
 // MFMA-layout reads).  While a chunk multiplies, the next moves from registers
 // to the other LDS buffer and the one after is requested, a quarter of each
 // per 16 k, so that the matrix cores never wait for a whole chunk's copies.
-// Bound: LDS and issue slots beside the MFMA (busy 41% at 2048 x 11264 x 2048);
+// Bound: LDS and issue slots beside the MFMA (busy 47% at 2048 x 11264 x 2048);
 // see the launch rule for figures.
 template <int WM, int WN, int KS>
 struct TileGeo {

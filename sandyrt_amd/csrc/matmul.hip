@@ -17,19 +17,20 @@
 // 173-216; its CUDA linear is not implemented, CudaDevice.cpp:536-537).
 // Here there are four kernels:
 //   - bf16 with the weight read row-major as [n, k] (transpose_rhs, the
-//     layout of every projection and the lm-head) runs on
-//     v_mfma_f32_16x16x32_bf16 with fp32 accumulation:
-//       gemm_waves_kernel for decode-sized products (up to 64 rows): weight
-//         streams, HBM-bound, K split over the waves of a workgroup and, when
+//     layout of every projection and the lm-head) runs on bf16 MFMA with fp32
+//     accumulation:
+//       gemm_waves_kernel for decode-sized products (up to 64 rows),
+//         v_mfma_f32_16x16x32_bf16: weight streams, HBM-bound, K split over the waves of a workgroup and, when
 //         the column tiles alone cannot fill the chip, over workgroups, with
 //         the last-arriving workgroup of each output tile summing the fp32
 //         partials in split order -- one launch, no second reduction pass;
-//       gemm_tile_kernel for larger row counts: tiles up to 128 x 192;
+//       gemm_tile_kernel for larger row counts, v_mfma_f32_32x32x16_bf16: tiles
+//         up to 128 x 192;
 //   - f32 in the same layout runs gemm_ordered_kernel, FMA-free float loops
 //     that keep the reference's k order per output, so f32 results are
 //     bit-identical to the CPU path;
-//   - gemm_simt_kernel: every other case (other layouts, unaligned shapes),
-//     register-tiled, in the same order.
+//   - gemm_simt_kernel: every other case (other layouts, unaligned shapes, f32 of
+//     short contractions and many outputs), register-tiled, in the same order.
 #include "gemm.h"
 #include "gemm_tile.h"
 
@@ -571,7 +572,7 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
         // KS groups) times the time of one plus the tile's own (first loads, output),
         // `alone` up to one workgroup a CU, else `each` for every workgroup of the
         // fullest CU (measured, us).  Cold operands, 64 x 256 tiles before -> the form
-        // taken (us): 2048 x 11264 x 2048 163 -> 99 (128 x 192 tiles, 960 TFLOP/s),
+        // taken (us): 2048 x 11264 x 2048 163 -> 95-99 (128 x 192 tiles, 955-995 TFLOP/s),
         // 2040 x 2048 x 5632 -> 57 (128 x 128, two K groups), 2048 x 2048 x 2048 39 ->
         // 24 (128 x 64), 1000 x 2048 x 5632 93 -> 33 (128 x 64, two groups), 333 x 2048
         // x 5632 93 -> 22 (64 x 64, two groups).  Without the tile's own time short

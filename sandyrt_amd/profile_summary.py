@@ -120,25 +120,25 @@ def traffic(fetch_path, write_path, copy_bytes=256 << 20):
 # in a `bench.py --no-decode-step` run (config 2/3 step kernels and extras)
 BENCH_DISPATCH = {
     "add_rms_norm": ("rms_rows_kernel<sandy_hip::BF16, 4, true, true, true, false>", "262144"),
-    "rope_qk": ("rope_split_lines_kernel<sandy_hip::BF16, 6, true, false>", "196608"),
+    "rope_qk": ("rope_split_lines_kernel<sandy_hip::BF16, 6, true, false, 321>", "196608"),
     "silu_gate": ("sandy_ew", "524288"),
-    "paged_decode": ("paged_decode_units_kernel<64, 2, 8, 2, 1>", "262144"),
-    "c4_paged_decode": ("paged_decode_units_kernel<256, 1, 8, 2, 2>", "524288"),
+    "paged_decode": ("paged_decode_units_kernel<64, 2, 8, 2, 1, false>", "262144"),
+    "c4_paged_decode": ("paged_decode_units_kernel<256, 1, 8, 2, 2, true>", "524288"),
     "c4_rms_norm": ("rms_rows_kernel<sandy_hip::BF16, 8, false, true, false, true>", "4096"),
-    "c4_geglu": ("sandy_ew", "40960"),
+    "c4_geglu": ("sandy_ew", "81920"),
     "c4_greedy_argmax": ("argmax_wide_kernel<sandy_hip::BF16, 4, true>", "524288"),
     "c1_greedy_argmax": ("argmax_wide_kernel<sandy_hip::F32, 2, false>", "3328"),
-    "c3_qkv_proj": ("sandy_hip::gemm_waves_kernel<1, 2, 4, 8, 1, false, false>", "40960"),
-    "c3_o_proj": ("sandy_hip::gemm_waves_kernel<1, 1, 4, 8, 1, false, false>", "65536"),
-    "c3_gate_up_proj": ("sandy_hip::gemm_waves_kernel<1, 2, 2, 8, 4, false, false>", "180224"),
-    "c3_down_proj": ("sandy_hip::gemm_waves_kernel<1, 2, 2, 8, 4, false, false>", "98304"),
-    "c3_lm_head": ("sandy_hip::gemm_waves_kernel<2, 4, 2, 8, 2, false, false>", "128000"),
-    "c2_rope_qk_cached": ("rope_split_lines_kernel<sandy_hip::BF16, 6, true, true>", "196608"),
+    "c3_qkv_proj": ("sandy_hip::gemm_waves_kernel<1, 2, 4, 8, 1, false, false, true>", "40960"),
+    "c3_o_proj": ("sandy_hip::gemm_waves_kernel<1, 1, 4, 8, 1, false, false, true>", "65536"),
+    "c3_gate_up_proj": ("sandy_hip::gemm_waves_kernel<2, 1, 4, 8, 1, false, false, true>", "180224"),
+    "c3_down_proj": ("sandy_hip::gemm_waves_kernel<1, 2, 4, 12, 1, false, false, true>", "65536"),
+    "c3_lm_head": ("sandy_hip::gemm_waves_kernel<2, 4, 2, 8, 2, false, false, true>", "128000"),
+    "c2_rope_qk_cached": ("rope_split_lines_kernel<sandy_hip::BF16, 6, true, true, 321>", "196608"),
     "c2_rope_cache": ("rope_cache_kernel", "131072"),
     "c2_copy_rope_bytes": ("layout_copy16_kernel", "1179648"),
     "c5_topk": ("topk_rank4_kernel<sandy_hip::F32, 2>", "131072"),
     "c5_moe_gather": ("moe_dispatch_tokens_kernel<16, 8, true>", "65536"),
-    "c5_moe_matmul_gate": ("moe_gemm_lines_kernel<4, 4>", "98304"),
+    "c5_moe_matmul_gate": ("moe_gemm_lines_kernel<4, 3>", "131072"),
     "c5_swiglu": ("sandy_ew", "180224"),
     "c5_moe_matmul_down": ("moe_gemm_lines_kernel<4, 4>", "360448"),
     "c5_moe_scatter_sum": ("moe_combine_kernel<sandy_hip::BF16>", "196608"),
