@@ -364,8 +364,14 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
     // same order, reread the operands less and fill whole store lines.  us, ordered / simt:
     // 1000 x 16000 x 16 49 / 26, 1000 x 4000 x 48 21 / 17, 2000 x 8000 x 96 105 / 97,
     // 1461 x 8606 x 20 44 / 32; k 128 even, 2000 x 8000 x 256 233 / 245; 1000 x 1000 x 24
-    // 7.3 / 8.4)
-    const bool short_wide = p.M > 8 && p.M <= 65535 * 64 && p.K <= 96 && p.M * p.N * p.batches >= (2 << 20);
+    // 7.3 / 8.4.  The shorter the contraction, the sooner, and few columns count as the
+    // tiles they fill: k 8 235 products of 149 x 12 10.6 / 6.1, 395 x 4689 8.4 / 6.2, k 12
+    // 2375 x 834 11.0 / 8.0, k 32 298 of 151 x 5 15.0 / 11.2; k 16 364 x 1849 5.3 / 6.6,
+    // 500 x 1837 even, k 24 1012 x 950 7.6 / 8.5, k 32 148 x 9429 9.8 / 10.2)
+    const int64_t filled = (p.M + 15) / 16 * 16 * ((p.N + 63) / 64 * 64) * p.batches;
+    const bool short_wide = p.M > 8 && p.M <= 65535 * 64 &&
+                            ((p.K <= 96 && p.M * p.N * p.batches >= (2 << 20)) || (p.K <= 32 && filled >= (2 << 20)) ||
+                             (p.K <= 16 && filled >= 1000000));
     const bool ordered = l.dtype == SANDY_F32 && !tl && tr && p.K % 4 == 0 && p.K > 0 && aligned && !short_wide &&
                          env_int("SANDY_GEMM_SIMT", 0) == 0;
     if (ordered) {

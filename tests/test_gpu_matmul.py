@@ -300,7 +300,8 @@ def test_linear_f32_ordered_tiles_bit_exact(ops, oracle, rows_a_lane, rows, in_f
     assert_equal(got3, oracle.matmul(to_oracle(x3), to_oracle(w.unsqueeze(0)), transpose_rhs=True), "batched matmul")
 
 
-@pytest.mark.parametrize("rows,in_f,out_f", [(8, 4, 262144), (9, 4, 233017), (128, 96, 16384), (128, 100, 16384)])
+@pytest.mark.parametrize("rows,in_f,out_f", [(8, 4, 262144), (9, 4, 233017), (128, 96, 16384), (128, 100, 16384),
+                                             (9, 16, 62465), (9, 16, 62464), (17, 32, 65473), (17, 32, 65472)])
 def test_linear_f32_short_contractions_bit_exact(ops, oracle, rows, in_f, out_f):
     """Both sides of the line between the ordered kernel and the 64 x 64 tiles."""
     r = rng(rows + in_f)
