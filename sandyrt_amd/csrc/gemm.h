@@ -72,6 +72,7 @@ struct GemmArgs {
     uint16_t* out;         // [batch, M, N]
     int64_t M, N, K;
     int32_t col_tiles, row_tiles, splits, split_chunks;
+    int32_t fold;          // gemm_tile_kernel: products in one run of workgroups (else one a grid layer)
     float* part;           // [tiles, splits, 4 waves, RT * CT * 64 lanes * 4]
     uint32_t* counters;    // [tiles] arrivals (zero between launches)
     BatchMap bm;

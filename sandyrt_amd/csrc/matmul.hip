@@ -51,17 +51,24 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_tile_kernel(GemmArgs g) {
     using G_ = TileGeo<WM, WN, KS>;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     // workgroups are dealt round-robin to the 8 XCDs: each XCD takes a run of
-    // neighbouring tiles, rows fastest, so its L2 serves the weight tile to every row tile
-    const int tiles = g.row_tiles * g.col_tiles, per = (tiles + 7) / 8;
-    const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if (static_cast<int>(blockIdx.x >> 3) >= per || tile >= tiles) return;
+    // neighbouring tiles, rows fastest, so its L2 serves the weight tile to every row
+    // tile.  The products of a batch follow one another in that run: each product's
+    // tiles dealt out by themselves, those of one to eight tiles left XCDs idle
+    const int tiles = g.row_tiles * g.col_tiles, all = tiles * g.fold, per = (all + 7) / 8;
+    int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (static_cast<int>(blockIdx.x >> 3) >= per || tile >= all) return;
+    int64_t product = blockIdx.z;
+    if (g.fold > 1) {
+        product = tile / tiles;
+        tile -= static_cast<int>(product) * tiles;
+    }
     const int64_t m0 = static_cast<int64_t>(tile % g.row_tiles) * G_::BM, n0 = static_cast<int64_t>(tile / g.row_tiles) * G_::BN;
     int64_t lo, ro;
-    batch_offsets(g.bm, blockIdx.z, lo, ro);
+    batch_offsets(g.bm, product, lo, ro);
     const int64_t M = g.M, N = g.N, K = g.K;
     gemm_tile<WM, WN, KS, false>(lds, g.a + lo + m0 * K, static_cast<int>(min<int64_t>(G_::BM, M - m0)), g.w + ro + n0 * K,
                                  static_cast<int>(min<int64_t>(G_::BN, N - n0)), K, g.bias ? g.bias + n0 : nullptr,
-                                 g.out + (static_cast<int64_t>(blockIdx.z) * M + m0) * N + n0, N);
+                                 g.out + (product * M + m0) * N + n0, N);
 }
 
 // Any dtype, either operand transposed: 64 x 64 output tile per workgroup,
@@ -584,8 +591,10 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
         // x 5632 93 -> 22 (64 x 64, two groups).  Without the tile's own time short
         // contractions got too wide tiles, and 64 x 64 of one group suits the smallest
         // (us, 64 x 256 tiles / that rule / here): 915 x 7338 x 224 16.1 / 17.3 / 13.6,
-        // 946 x 13341 x 512 42 / 37 / 28, 300 products of 80 x 80 x 32 13.5 / 16.6 /
-        // 13.0, 434 x 2385 x 96 - / 7.2 / 6.0.
+        // 946 x 13341 x 512 42 / 37 / 28, 434 x 2385 x 96 - / 7.2 / 6.0.  Batches (64 x 256
+        // tiles / products dealt to the XCDs one by one / here): 185 of 141 x 165 x 576
+        // 35 / 47 / 19, 137 of 116 x 5 x 1088 22 / 52 / 12, 164 of 73 x 35 x 160 9.3 / 12 /
+        // 5.9, 40 of 85 x 109 x 800 20 / 13 / 7.7.
         struct Form {
             int bm, bn, groups;
             double alone, each, alone_tile, each_tile;
@@ -616,10 +625,13 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
                 return fail(e, SANDY_ERR_UNSUPPORTED, "%s shape exceeds the launch grid", what);
             g.row_tiles = static_cast<int32_t>(rt);
             g.col_tiles = static_cast<int32_t>(ct);
+            const bool fold = rt * ct * p.batches <= 0x7ffffff0;
+            g.fold = fold ? static_cast<int32_t>(p.batches) : 1;
             if (G_::kBytes > 64 * 1024)
                 SANDY_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, G_::kBytes), e, what);
-            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((rt * ct + 7) / 8 * 8), 1, static_cast<unsigned>(p.batches)),
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((rt * ct * g.fold + 7) / 8 * 8), 1,
+                                            static_cast<unsigned>(fold ? 1 : p.batches)),
                                dim3(G_::THREADS), G_::kBytes, stream, g);
             return SANDY_OK;
         };

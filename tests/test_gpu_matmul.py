@@ -547,3 +547,18 @@ def test_decode_linear_rejects(ops):
     sq = torch.zeros(1, 64, device="cuda")
     with pytest.raises(SandyError, match="out must not alias x"):
         ops.decode_linear(sq, torch.zeros(64, 64, device="cuda"), out=sq)
+
+
+@pytest.mark.parametrize("form", ["", 0, 1, 2, 3, 4, 5])
+@pytest.mark.parametrize("B,H,m,n,k", [(3, 1, 65, 5, 32), (2, 9, 70, 66, 96), (13, 1, 193, 200, 64), (1, 40, 66, 4, 160)])
+def test_matmul_bf16_batched_tiles(ops, oracle, monkeypatch, form, B, H, m, n, k):
+    """Batches of products of one to a dozen tiles each: every product's tiles lie
+    in one run over the whole batch; the second operand shared by groups of three
+    heads where they divide."""
+    if form != "":
+        monkeypatch.setenv("SANDY_GEMM_FORM", str(form))
+    r = rng(B * H + n)
+    kv = H // 3 if H % 3 == 0 else H
+    x, w = from_f32(normal(r, (B, H, m, k)), torch.bfloat16), from_f32(normal(r, (B, kv, n, k), 0.1), torch.bfloat16)
+    got = ops.matmul(x, w, transpose_rhs=True)
+    assert_close(got, oracle.matmul(to_oracle(x), to_oracle(w), transpose_rhs=True), torch.bfloat16, "batched tiles")
