@@ -1242,15 +1242,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
 template <int WM, int WN, int KS>
 __global__ __launch_bounds__(256 * KS, 2) void moe_gemm_tile_kernel(
         const uint16_t* __restrict__ x, const void* __restrict__ offs, int32_t off_dt, const uint16_t* __restrict__ w,
-        uint16_t* __restrict__ out, int64_t rows, int64_t K, int64_t M, int64_t experts, int col_tiles, uint32_t* errw) {
+        uint16_t* __restrict__ out, int64_t rows, int64_t K, int64_t M, int64_t experts, int col_tiles, int run_log, int turn,
+        uint32_t* errw) {
     using G_ = TileGeo<WM, WN, KS>;
     extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];
     const int lane = threadIdx.x & 63;
     const int64_t b = blockIdx.y;
-    // runs of 16 neighbouring tiles (row tiles fastest) go to one XCD, so that its L2
-    // serves a weight tile to the expert's row tiles; the tiles past the last row come last
+    // runs of 2^run_log neighbouring tiles (row tiles fastest) go to one XCD, so that its
+    // L2 serves a weight tile to the expert's row tiles; the tiles past the last row come
+    // last.  A sequence's tiles start on the first XCD like the others' (their weights are
+    // the same), or, with fewer tiles than XCDs, `turn` XCDs after the one before
     const int j = static_cast<int>(blockIdx.x >> 3);
-    int want = (j >> 4) * 128 + static_cast<int>(blockIdx.x & 7) * 16 + (j & 15);
+    int want = ((j >> run_log) << (run_log + 3)) + (static_cast<int>((blockIdx.x + blockIdx.y * turn) & 7) << run_log) +
+               (j & ((1 << run_log) - 1));
     const bool check = want == 0;  // scans every expert's offsets
     int64_t e = -1, begin = 0, end = 0;
     int mine = 0, n_rt = 1;
@@ -1840,24 +1844,32 @@ extern "C" int sandy_hip_moe_matmul(const SandyTensor* x, const SandyTensor* exp
         // -> 106 / 117, 128 rows 241 / 285 -> 157 / 148, 256 rows 428 / 512 -> 201 /
         // 214; 37 rows 81 / 100 against 98 / 109).  64 x 192 tiles 132 / 129 at 64
         // rows, 170 / 175 at 128; 128 x 128 tiles 122 / 129 and 154 / 157.
-        // A tile's first loads and its output weigh more the shorter the contraction, and
-        // several sequences fill the chip with either kernel: the line moves up (there /
-        // here: k 1408, 3 sequences x 64 experts x 3436 at 50 rows 348 / 402, at 62 rows
-        // 32 x 2816 201 / 125; k 512, 16 x 1028 at 45 12.5 / 14.6, 128 x 704 at 68 38 /
+        // A tile's first loads and its output weigh more the shorter the contraction, several
+        // sequences of many tiles fill the chip with either kernel, and of few experts none
+        // may pass 64 (one never does up to 64 rows in all): the line moves up (there / here:
+        // k 1408, 3 sequences x 64 experts x 3436 at 50 rows each 285 / 364, but 8 x 6 x 516,
+        // k 2432, at 52 41 / 35, with one expert past 64 76 / 37; k 768, 2 x 2 x 148 at 54 11 /
+        // 16, 2 x 3 x 67 at 50 14 / 20, 2 x 26 x 298 at 51 with one past 64 22 / 15; k 1600,
+        // 4 x 1 x 441 at 60 26 / 33; k 512, 16 x 1028 at 45 12.5 / 14.6, 128 x 704 at 68 38 /
         // 25; k 192, 8 x 751 at 173 17.6 / 19.8; k 64, 200 x 366 at 82 11.7 / 15.0)
-        const int64_t tile_rows = K >= 640 ? (batch == 1 ? 44 : 56) : K >= 512 ? 64 : K >= 256 ? 128 : rows;
         using Tile = TileGeo<2, 3, 1>;
         const int64_t col_tiles = (M + Tile::BN - 1) / Tile::BN;
+        const int64_t owners = batch * experts;
+        const bool late = (batch > 1 && owners * col_tiles >= 2048) || (K < 1024 && owners < 24);
+        const int64_t tile_rows = K >= 640 ? (late ? 56 : 44) : K >= 512 ? 64 : K >= 256 ? 128 : rows;
         // row tiles of all experts together: whole ones, and one partial one each
         const int64_t tiles = (rows / Tile::BM + std::min(rows, experts)) * col_tiles;
-        if (env_int("SANDY_MOE_TILE", rows > tile_rows * experts) && rows <= 0x7fffffff && batch <= 65535 && K <= (1 << 22) &&
+        if (env_int("SANDY_MOE_TILE", rows > std::max<int64_t>(64, tile_rows * experts)) && rows <= 0x7fffffff && batch <= 65535 && K <= (1 << 22) &&
             tiles <= (1 << 30)) {
             SANDY_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(moe_gemm_tile_kernel<2, 3, 1>),
                                               hipFuncAttributeMaxDynamicSharedMemorySize, Tile::kBytes), e, "moe_matmul");
+            int run_log = 0;  // 16 tiles a run where there are that many for each XCD
+            while (run_log < 4 && (int64_t{16} << run_log) <= tiles) run_log++;
+            const int64_t round = int64_t{8} << run_log;
             hipLaunchKernelGGL((moe_gemm_tile_kernel<2, 3, 1>),
-                               dim3(static_cast<unsigned>((tiles + 127) / 128 * 128), static_cast<unsigned>(batch)),
+                               dim3(static_cast<unsigned>((tiles + round - 1) / round * round), static_cast<unsigned>(batch)),
                                dim3(Tile::THREADS), Tile::kBytes, stream, px, po_, expert_offsets->dtype, pw, po, rows, K, M,
-                               experts, static_cast<int>(col_tiles), errw);
+                               experts, static_cast<int>(col_tiles), run_log, tiles < 8 ? 1 : 0, errw);
             SANDY_HIP_TRY(hipGetLastError(), e, "moe_matmul launch");
             return ok(e);
         }

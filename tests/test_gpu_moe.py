@@ -371,7 +371,26 @@ def test_moe_matmul_many_rows(ops, oracle, monkeypatch, counts, M, K):
     assert_close(got, oracle.moe_matmul(to_oracle(x), offs, to_oracle(w), True), torch.bfloat16, "moe_matmul")
 
 
-@pytest.mark.parametrize("B,rows,K", [(1, 88, 640), (1, 90, 640), (2, 112, 640), (2, 114, 640), (1, 128, 608), (1, 130, 608),
+@pytest.mark.parametrize("B,E,rows,M,K", [(1, 1, 64, 40, 1024), (1, 1, 65, 40, 1024), (9, 1, 130, 200, 640), (1, 1, 2100, 400, 640),
+                                          (3, 11, 700, 1000, 1024), (2, 40, 4200, 400, 640)])
+def test_moe_matmul_tile_runs(ops, oracle, B, E, rows, M, K):
+    """The many-rows tiles with fewer tiles than XCDs, in sequences that take
+    turns, and in runs of every length up to 16; one expert up to 64 rows is
+    the other kernel's."""
+    r = rng(rows + M)
+    offs = np.stack([np.array([0, *sorted(r.integers(0, rows + 1, E - 1)), rows]) for _ in range(B)]).astype(np.int64)
+    x = from_f32(normal(r, (B, rows, K)), torch.bfloat16)
+    w = from_f32(normal(r, (E, M, K), 0.1), torch.bfloat16)
+    got = ops.moe_matmul(x, torch.from_numpy(offs).cuda(), w, True)
+    ops.check_device_errors()
+    for b in range(B):  # oracle: the products in fp64, expert by expert
+        for e in range(E):
+            lo, hi = offs[b, e], offs[b, e + 1]
+            want = (x[b, lo:hi].double() @ w[e].double().t().contiguous()).float().bfloat16()
+            assert_close(got[b, lo:hi], to_oracle(want), torch.bfloat16, f"sequence {b} expert {e}")
+
+
+@pytest.mark.parametrize("B,rows,K", [(1, 112, 640), (1, 114, 640), (2, 114, 960), (1, 88, 1024), (1, 90, 1024), (2, 90, 1024), (1, 128, 608), (1, 130, 608),
                                       (1, 258, 256), (1, 300, 224), (1, 1, 608), (1, 1, 640), (2, 1, 480)])
 def test_moe_matmul_kernel_choice_edges(ops, oracle, B, rows, K):
     """Both sides of the lines at which the kernel for an expert's rows changes
