@@ -1850,13 +1850,17 @@ extern "C" int sandy_hip_moe_matmul(const SandyTensor* x, const SandyTensor* exp
         // k 1408, 3 sequences x 64 experts x 3436 at 50 rows each 285 / 364, but 8 x 6 x 516,
         // k 2432, at 52 41 / 35, with one expert past 64 76 / 37; k 768, 2 x 2 x 148 at 54 11 /
         // 16, 2 x 3 x 67 at 50 14 / 20, 2 x 26 x 298 at 51 with one past 64 22 / 15; k 1600,
-        // 4 x 1 x 441 at 60 26 / 33; k 512, 16 x 1028 at 45 12.5 / 14.6, 128 x 704 at 68 38 /
-        // 25; k 192, 8 x 751 at 173 17.6 / 19.8; k 64, 200 x 366 at 82 11.7 / 15.0)
+        // 4 x 1 x 441 at 60 26 / 33.  Even routes: k 512, 53 x 17 at 66 16 / 16, 4 x 25 x 1327
+        // at 182 110 / 72; k 448, 48 x 19 at 63 9 / 15, 23 x 150 at 92 15 / 13; k 320, 5 x 143
+        // at 80 12 / 14, 3 x 524 at 192 19 / 11; k 256, 18 x 124 at 74 10 / 10, 17 x 626 at 120
+        // 16 / 11; k 128, 6 x 83 at 125 10 / 12, 3 x 820 at 198 13 / 9, 13 x 291 at 876 43 /
+        // 14; k 64, 52 x 1893 at 139 22 / 36, 21 x 924 at 205 23 / 24, 3 x 1722 at 298 14 / 9)
         using Tile = TileGeo<2, 3, 1>;
         const int64_t col_tiles = (M + Tile::BN - 1) / Tile::BN;
         const int64_t owners = batch * experts;
         const bool late = (batch > 1 && owners * col_tiles >= 2048) || (K < 1024 && owners < 24);
-        const int64_t tile_rows = K >= 640 ? (late ? 56 : 44) : K >= 512 ? 64 : K >= 256 ? 128 : rows;
+        const int64_t tile_rows = K >= 640 ? (late ? 56 : 44) : K >= 512 ? 64 : K >= 384 ? 72
+                                  : K >= 256 ? 96 : K >= 160 ? 128 : K >= 96 ? 160 : 200;
         // row tiles of all experts together: whole ones, and one partial one each
         const int64_t tiles = (rows / Tile::BM + std::min(rows, experts)) * col_tiles;
         if (env_int("SANDY_MOE_TILE", rows > std::max<int64_t>(64, tile_rows * experts)) && rows <= 0x7fffffff && batch <= 65535 && K <= (1 << 22) &&

@@ -391,7 +391,8 @@ def test_moe_matmul_tile_runs(ops, oracle, B, E, rows, M, K):
 
 
 @pytest.mark.parametrize("B,rows,K", [(1, 112, 640), (1, 114, 640), (2, 114, 960), (1, 88, 1024), (1, 90, 1024), (2, 90, 1024), (1, 128, 608), (1, 130, 608),
-                                      (1, 258, 256), (1, 300, 224), (1, 1, 608), (1, 1, 640), (2, 1, 480)])
+                                      (1, 144, 448), (1, 146, 448), (1, 192, 256), (1, 194, 256), (1, 258, 224), (1, 320, 128),
+                                      (1, 322, 128), (1, 400, 64), (1, 402, 64), (1, 1, 608), (1, 1, 640), (2, 1, 480)])
 def test_moe_matmul_kernel_choice_edges(ops, oracle, B, rows, K):
     """Both sides of the lines at which the kernel for an expert's rows changes
     (2 experts; contraction length, rows an expert, sequences)."""
