@@ -1824,8 +1824,12 @@ extern "C" int sandy_hip_moe_matmul(const SandyTensor* x, const SandyTensor* exp
         // contraction is split over the waves (8 rows 18 -> 10; 40 rows 28 -> 31).
         // Short contractions have too few chunks to keep in flight: k 64 4.3 / 5.1 (3
         // sequences, 128 experts x 3703 x 192, 60 rows 49 / 68), k 512 13.7 / 7.2 for 4
-        // rows of 64 experts x 1577 and 18.5 / 20.3 for 60 of 200 x 1483
-        const bool few = rows * 2 <= experts && (K >= 640 || (K >= 512 && rows * 4 <= experts)) && M <= 65535 * 32;
+        // rows of 64 experts x 1577 and 18.5 / 20.3 for 60 of 200 x 1483; and for fewer
+        // routes than an eighth of the experts the launch of all of them counts: 3 rows of
+        // 108 x 2053 x 384 7.9 / 5.1, 1 of 2 x 11 x 3942 x 448 6.9 / 5.3, 5 of 2 x 80 x 2740 x
+        // 128 6.7 / 5.0, but 2 of 40 x 383 x 320 4.6 / 4.8, 2 of 4 x 64 x 78 x 128 3.4 / 4.0
+        const bool rare = rows * 8 <= experts && K >= 128 && batch * experts * M >= 65536;
+        const bool few = rows * 2 <= experts && (K >= 640 || (K >= 512 && rows * 4 <= experts) || rare) && M <= 65535 * 32;
         const int stream_form = env_int("SANDY_MOE_STREAM", !few ? 0 : rows <= 16 && K >= 1536 ? 2 : 1);
         if (stream_form) {
             const int64_t slots = std::min(rows, experts);  // at most `rows` experts have a row

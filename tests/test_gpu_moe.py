@@ -372,11 +372,13 @@ def test_moe_matmul_many_rows(ops, oracle, monkeypatch, counts, M, K):
 
 
 @pytest.mark.parametrize("B,E,rows,M,K", [(1, 1, 64, 40, 1024), (1, 1, 65, 40, 1024), (9, 1, 130, 200, 640), (1, 1, 2100, 400, 640),
-                                          (3, 11, 700, 1000, 1024), (2, 40, 4200, 400, 640)])
+                                          (3, 11, 700, 1000, 1024), (2, 40, 4200, 400, 640), (1, 16, 2, 4096, 128),
+                                          (1, 16, 2, 4095, 128), (2, 16, 3, 4096, 128), (2, 24, 3, 1500, 192)])
 def test_moe_matmul_tile_runs(ops, oracle, B, E, rows, M, K):
     """The many-rows tiles with fewer tiles than XCDs, in sequences that take
     turns, and in runs of every length up to 16; one expert up to 64 rows is
-    the other kernel's."""
+    the other kernel's.  And a short contraction's few routes on both sides of
+    the line to the weight stream."""
     r = rng(rows + M)
     offs = np.stack([np.array([0, *sorted(r.integers(0, rows + 1, E - 1)), rows]) for _ in range(B)]).astype(np.int64)
     x = from_f32(normal(r, (B, rows, K)), torch.bfloat16)
