@@ -1671,8 +1671,9 @@ extern "C" int sandy_hip_moe_gather(const SandyTensor* x, const SandyTensor* top
     // several sequences queue up while the ranking runs one workgroup a sequence (us, here
     // / ranking: 60000 routes of 1 a token, 938 workgroups a sequence, 3 sequences 172 /
     // 262, 6 325 / 294, 64 3274 / 1044; 64000 of 8, 1000 workgroups, 3 210 / 533, 16 1030 /
-    // 682; 16384 of 4, 256 workgroups, 8 94 / 100, 12 133 / 125)
-    const bool ranked = routes > kDispatchRoutes && batch * wgs > 3000;
+    // 682; 47968 of 8, 750 workgroups, 8 292 / 451; 16384 of 4, 256 workgroups, 8 94 / 100,
+    // 12 133 / 125)
+    const bool ranked = routes > kDispatchRoutes && batch * wgs > (top_k < 8 ? 3000 : 8000);
     if (routes <= kTokenRoutes && !ranked && batch <= 65535 && aligned && top_k <= 64 && 2 * num_experts + 64 <= 16384 &&
         env_int("SANDY_MOE_ROUTE_GENERAL", 0) == 0) {
         if (wgs > 0x7fffffff) return fail(e, SANDY_ERR_UNSUPPORTED, "moe_gather too many tokens");

@@ -181,12 +181,13 @@ def test_moe_gather_long(ops, oracle, T, E, K, idx):
     assert_equal(off, np.concatenate([[0], np.cumsum(counts)]).astype(np.int64), "expert_offsets")
 
 
-@pytest.mark.parametrize("B", [11, 12])
-def test_moe_gather_long_batched(ops, oracle, B):
+@pytest.mark.parametrize("B,K", [(11, 4), (12, 4), (15, 8), (16, 8)])
+def test_moe_gather_long_batched(ops, oracle, B, K):
     """Long route lists of several sequences: in one launch up to 3000 workgroups
-    together (11 x 257), ranked one workgroup a sequence past it."""
+    together (11 x 257; 8000 for 8 routes a token, 15 x 513), ranked one workgroup
+    a sequence past it."""
     r = rng(B)
-    T, E, K = 4100, 9, 4
+    T, E = 4100, 9
     ids = r.integers(0, E, (B, T, K)).astype(np.int64)
     x = from_f32(normal(r, (B, T, 8)), torch.bfloat16)
     w = from_f32(np.abs(normal(r, (B, T, K))), torch.bfloat16)
