@@ -534,17 +534,18 @@ __global__ __launch_bounds__((Geo<T, D, RW>::THREADS), (Geo<T, D, RW>::kF32 && D
         }
     }
     if (PAGED && !pages_ok) atomicOr(a.errw, static_cast<uint32_t>(SANDY_DEVERR_BLOCK));
-    // f32: divided in 64 bits, one rounding an output
-    using Inv = std::conditional_t<kF32, double, float>;
-    const Inv inv = Inv(1) / static_cast<Inv>(l);
+    // f32: the reciprocal as two floats, so that the output is rounded about once
+    const double inv64 = 1.0 / l;
+    const float inv = kF32 ? static_cast<float>(inv64) : 1.0f / static_cast<float>(l);
+    const float inv_lo = kF32 ? static_cast<float>(inv64 - static_cast<double>(inv)) : 0.0f;
     // a row that sees no key (or only NaN scores) is zero, as in the general kernel
     const bool none = m == -INFINITY;
     bool finite = true;
 #pragma unroll
-    for (int t = 0; t < DT; t++)
+    for (int t = 0; kw == 0 && t < DT; t++)
 #pragma unroll
         for (int i = 0; i < 16; i++) {
-            acc[t][i] = none ? 0.0f : static_cast<float>(static_cast<Inv>(acc[t][i]) * inv);
+            acc[t][i] = none ? 0.0f : kF32 ? fmaf(acc[t][i], inv, acc[t][i] * inv_lo) : acc[t][i] * inv;
             finite = finite && fabsf(acc[t][i]) < INFINITY;
         }
     // nothing is stored before it is known which rows are computed again: those read
