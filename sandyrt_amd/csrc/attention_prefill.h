@@ -26,6 +26,7 @@ struct PrefillArgs {
     int32_t tq, tk;
     int32_t row_blocks;  // row tiles per (b, kh)
     int32_t table_pages; // page addresses staged in LDS (0: read from memory)
+    int32_t in_place;    // out may share memory with q
     int64_t window;
     float scale, scale_log2;  // scale * log2(e)
     int32_t dtype;            // F32 or BF16

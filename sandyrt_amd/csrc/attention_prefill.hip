@@ -548,8 +548,23 @@ __global__ __launch_bounds__((Geo<T, D, RW>::THREADS), (Geo<T, D, RW>::kF32 && D
             acc[t][i] = none ? 0.0f : kF32 ? fmaf(acc[t][i], inv, acc[t][i] * inv_lo) : acc[t][i] * inv;
             finite = finite && fabsf(acc[t][i]) < INFINITY;
         }
-    // nothing is stored before it is known which rows are computed again: those read
-    // their q, and `out` may be `q`
+    auto put = [&] {
+        char* op = static_cast<char*>(a.out) + (b * a.os[0] + (kh * a.group + qg) * a.os[1] + qt * a.os[2] + 32 * DT * ds + 4 * half) * ES;
+#pragma unroll
+        for (int t = 0; t < DT; t++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                float o[4];
+#pragma unroll
+                for (int x = 0; x < 4; x++) o[x] = acc[t][4 * i + x];
+                char* to = op + (32 * t + 8 * i) * ES;
+                if constexpr (kF32) *reinterpret_cast<float4*>(to) = make_float4(o[0], o[1], o[2], o[3]);
+                else *reinterpret_cast<uint2*>(to) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+            }
+    };
+    // rows computed again read their q: where `out` may be `q`, nothing is stored before
+    // it is known which those are (elsewhere the stores need not wait for the others)
+    if (!a.in_place && kw == 0 && row < rows) put();
     const bool redo = __syncthreads_or(kw == 0 && row < rows && !finite);
     int* bad = reinterpret_cast<int*>(lds);           // [32 * RW] rows to compute again
     float* qf = reinterpret_cast<float*>(lds + 512);  // [32 * RW][D] their q
@@ -563,20 +578,7 @@ __global__ __launch_bounds__((Geo<T, D, RW>::THREADS), (Geo<T, D, RW>::kF32 && D
         if (kw == 0 && row < rows && !finite) bad[32 * rw + col] = 1;
         __syncthreads();
     }
-    if (kw == 0 && row < rows && !(redo && bad[32 * rw + col])) {
-        char* op = static_cast<char*>(a.out) + (b * a.os[0] + (kh * a.group + qg) * a.os[1] + qt * a.os[2] + 32 * DT * ds + 4 * half) * ES;
-#pragma unroll
-        for (int t = 0; t < DT; t++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                float o[4];
-#pragma unroll
-                for (int x = 0; x < 4; x++) o[x] = acc[t][4 * i + x];
-                char* to = op + (32 * t + 8 * i) * ES;
-                if constexpr (kF32) *reinterpret_cast<float4*>(to) = make_float4(o[0], o[1], o[2], o[3]);
-                else *reinterpret_cast<uint2*>(to) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
-            }
-    }
+    if (a.in_place && kw == 0 && row < rows && !(redo && bad[32 * rw + col])) put();
     if (!redo) return;
     constexpr int kMine = 32 * RW / (G_::THREADS / 64);  // rows of a wave
     constexpr int R = D == 64 ? 8 : 4;
@@ -588,10 +590,23 @@ __global__ __launch_bounds__((Geo<T, D, RW>::THREADS), (Geo<T, D, RW>::kF32 && D
     }
 }
 
+// First and last byte that [batch, hq, tq, dim] elements of `es` bytes at these strides touch.
+struct Span {
+    uintptr_t first, last;
+    Span(const void* p, const int64_t* s, const PrefillArgs& a, int64_t es) {
+        const int64_t n[3] = {a.batch - 1, a.hq - 1, a.tq - 1};
+        first = last = reinterpret_cast<uintptr_t>(p);
+        last += static_cast<uintptr_t>(a.dim * es - 1);
+        for (int i = 0; i < 3; i++) (s[i] < 0 ? first : last) += static_cast<uintptr_t>(n[i] * s[i] * es);
+    }
+};
+
 template <typename T, int D, int RW, bool PAGED>
 int launch_form(const PrefillArgs& a, hipStream_t stream, Err e) {
     static_assert(Geo<T, D, RW>::kBytes + kTablePages * 16 <= 160 * 1024 - 256, "LDS of a workgroup");
     PrefillArgs args = a;
+    const Span q(a.q, a.qs, a, Geo<T, D, RW>::ES), out(a.out, a.os, a, Geo<T, D, RW>::ES);
+    args.in_place = q.first <= out.last && out.first <= q.last;
     size_t bytes = Geo<T, D, RW>::kBytes;
     if (PAGED) {
         const int64_t span = prefill_page_span(a.tk, a.window, RW, a.group, a.log2_page);
