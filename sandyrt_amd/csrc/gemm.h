@@ -71,8 +71,9 @@ struct GemmArgs {
     const uint16_t* bias;  // [N] or null
     uint16_t* out;         // [batch, M, N]
     int64_t M, N, K;
-    int32_t col_tiles, row_tiles, splits, split_chunks;
-    int32_t fold;          // gemm_tile_kernel: products in one run of workgroups (else one a grid layer)
+    int32_t col_tiles, row_tiles;
+    int32_t splits;        // parts of K; gemm_tile_kernel: products in one run of workgroups (else one a grid layer)
+    int32_t split_chunks;
     float* part;           // [tiles, splits, 4 waves, RT * CT * 64 lanes * 4]
     uint32_t* counters;    // [tiles] arrivals (zero between launches)
     BatchMap bm;

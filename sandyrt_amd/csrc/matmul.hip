@@ -54,11 +54,11 @@ __global__ __launch_bounds__(256 * KS, 2) void gemm_tile_kernel(GemmArgs g) {
     // neighbouring tiles, rows fastest, so its L2 serves the weight tile to every row
     // tile.  The products of a batch follow one another in that run: each product's
     // tiles dealt out by themselves, those of one to eight tiles left XCDs idle
-    const int tiles = g.row_tiles * g.col_tiles, all = tiles * g.fold, per = (all + 7) / 8;
+    const int tiles = g.row_tiles * g.col_tiles, all = tiles * g.splits, per = (all + 7) / 8;
     int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if (static_cast<int>(blockIdx.x >> 3) >= per || tile >= all) return;
     int64_t product = blockIdx.z;
-    if (g.fold > 1) {
+    if (g.splits > 1) {
         product = tile / tiles;
         tile -= static_cast<int>(product) * tiles;
     }
@@ -626,11 +626,11 @@ int launch(const Plan& p, const SandyTensor& l, const SandyTensor& r, const Sand
             g.row_tiles = static_cast<int32_t>(rt);
             g.col_tiles = static_cast<int32_t>(ct);
             const bool fold = rt * ct * p.batches <= 0x7ffffff0;
-            g.fold = fold ? static_cast<int32_t>(p.batches) : 1;
+            g.splits = fold ? static_cast<int32_t>(p.batches) : 1;
             if (G_::kBytes > 64 * 1024)
                 SANDY_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, G_::kBytes), e, what);
-            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((rt * ct * g.fold + 7) / 8 * 8), 1,
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((rt * ct * g.splits + 7) / 8 * 8), 1,
                                             static_cast<unsigned>(fold ? 1 : p.batches)),
                                dim3(G_::THREADS), G_::kBytes, stream, g);
             return SANDY_OK;
