@@ -15,7 +15,7 @@
 //   - P^T leaves the product in the B-operand layout of O^T += V^T P^T, with
 //     V^T read by ds_read_b64_tr_b16 in the same key order;
 //   - P enters as three bf16 operands that together are p exactly (two of them
-//     kept about 17 bits and were 17% faster at 2048 queries); the row sums are
+//     kept about 17 bits and were 15% faster at 2048 queries); the row sums are
 //     kept in float64.
 // f32 takes v_mfma_f32_32x32x2_f32 for both products (f32 operands throughout,
 // P straight from its registers) and expf; bound by that instruction's rate, a
@@ -27,7 +27,7 @@
 // fit, one barrier each.
 // Bound: softmax VALU work, the cutting of P included (52% of the cycles at D 64,
 // MFMA 26%).  Measured, us a call (general kernel -> here): 2048 queries, 32 / 4
-// heads, D 64 14357 -> 50; 777 queries after 1500 keys, window 1024, 8 / 2 heads,
+// heads, D 64 14357 -> 48; 777 queries after 1500 keys, window 1024, 8 / 2 heads,
 // D 256, pages of 16: 4896 -> 42; 1500 after 300, 16 / 2 heads, D 128: 48; f32, 12
 // heads, D 64: 1000 queries 1434 -> 43, 64 queries 23.5 -> 10.
 // Against 64 bits (2 to 130 queries after 0 to 2000 keys, scores of three spreads)
